@@ -427,9 +427,7 @@ int32_t zb_profile_select(const char* names);
  * returns the previous value (ZB_EINVAL for an unknown name or a value out of range),
  * zb_knob_get the current one.
  *   "refine_queue" 0..2 (0): zb_refine_phases as one block per work item (0) or as a persistent
- *                            grid draining device-side queues (1; 2: with the NMI's second pass
- *                            looking the master up again rather than keeping its values, fewer
- *                            registers)
+ *                            grid draining device-side queues (1; 2: the same)
  *   "rings_group"  0..64 (0): ring pairs per block of the sphere stage's ring transforms, a power
  *                            of two (0: 16 KB of LDS worth; at most n / 2 and 64 KB)
  *   "prep_global"  0..1 (0): zb_prep_work's filters through global memory even where LDS holds

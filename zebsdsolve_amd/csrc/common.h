@@ -84,6 +84,22 @@ __device__ __forceinline__ float4 qexp(float3 p) {
     return make_float4(cosf(0.5f * th), k * p.x, k * p.y, k * p.z);
 }
 
+// The rotation of a quaternion held ready for many vectors: w, u and 2 u of q = (w, u). turn() is
+// qrot bit for bit (2 (u x v) as (2 u) x v: doubling commutes with rounding), three additions
+// fewer.
+struct Turn {
+    float w;
+    float3 u, u2;
+};
+__device__ __forceinline__ Turn turn_of(float4 q) {
+    return Turn{q.x, make_float3(q.y, q.z, q.w), make_float3(2.f * q.y, 2.f * q.z, 2.f * q.w)};
+}
+__device__ __forceinline__ float3 turn(const Turn& r, float3 v) {
+    const float3 t = cross3(r.u2, v);
+    const float3 c = cross3(r.u, t);
+    return make_float3(v.x + r.w * t.x + c.x, v.y + r.w * t.y + c.y, v.z + r.w * t.z + c.z);
+}
+
 // (the hardware reciprocal square root, 1 ulp)
 __device__ __forceinline__ float3 normalize3(float3 v) {
     float r = __builtin_amdgcn_rsqf(dot3(v, v));
@@ -119,7 +135,8 @@ __device__ __forceinline__ float2 sphere_to_square(float3 v) {
         (xbig ? ay : ax) * __builtin_amdgcn_rcpf(fmaxf(xbig ? ax : ay, 1e-30f)));
     const float u = xbig ? xn : t, w = xbig ? t : xn;
     const float sc = 0.79788456080286536f;  // 1 / sqrt(pi / 2)
-    return make_float2(u * sc * (v.x < 0.f ? -1.f : 1.f), w * sc * (v.y < 0.f ? -1.f : 1.f));
+    // (u, w >= 0, and 0 where v.x, v.y are: the sign bit is the sign)
+    return make_float2(copysignf(u * sc, v.x), copysignf(w * sc, v.y));
 }
 
 // Square coordinates -> unit vector on the northern or southern hemisphere (f32).
@@ -172,14 +189,16 @@ struct Taps {
 
 // The texel (offset of its top-left corner over both sheets) and the fractions for direction v.
 __device__ __forceinline__ int sheet_texel(int side, float3 v, float& tj, float& ti) {
-    float2 uv = sphere_to_square(v);
-    float last = (float)(side - 1);
-    float fj = fminf(fmaxf((uv.x + 1.f) * 0.5f * last, 0.f), last);
-    float fi = fminf(fmaxf((uv.y + 1.f) * 0.5f * last, 0.f), last);
-    int c0 = min((int)fj, side - 2), r0 = min((int)fi, side - 2);
+    // (halving commutes with rounding: (uv + 1) / 2 last; the median clamps to [0, last] in one
+    // instruction; rows and sides are far below 2^24, where the 24-bit product runs at full rate)
+    const float2 uv = sphere_to_square(v);
+    const float last = (float)(side - 1), half = 0.5f * last;
+    const float fj = __builtin_amdgcn_fmed3f((uv.x + 1.f) * half, 0.f, last);
+    const float fi = __builtin_amdgcn_fmed3f((uv.y + 1.f) * half, 0.f, last);
+    const int c0 = min((int)fj, side - 2), r0 = min((int)fi, side - 2);
     tj = fj - (float)c0;
     ti = fi - (float)r0;
-    return r0 * side + c0 + (v.z < 0.f ? side * side : 0);
+    return __mul24(r0, side) + c0 + (v.z < 0.f ? side * side : 0);
 }
 
 template <typename T>
@@ -279,6 +298,27 @@ __device__ __forceinline__ float4 sheet_bilinear<float4>(const float4* __restric
     Taps<float4> t;
     sheet_taps<float4>(s, side, v, t);
     return taps_blend(t);
+}
+
+// ── sums over a wave ──
+// v plus the value of the lane that DPP control CTRL reads (within rows of 16 lanes).
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float v) {
+    return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+
+// The sum over the wave in every lane, as a xor butterfly from distance 1 to 32 gives it bit for
+// bit (a + b == b + a; once the lanes of a group agree, the mirrored lane stands for the xor one):
+// DPP moves within rows of 16, row and half exchanges above, and no trip through LDS.
+__device__ __forceinline__ float wave_sum(float v) {
+    v = dpp_add<0xB1>(v);   // quad_perm 1 0 3 2
+    v = dpp_add<0x4E>(v);   // quad_perm 2 3 0 1
+    v = dpp_add<0x141>(v);  // row_half_mirror
+    v = dpp_add<0x140>(v);  // row_mirror
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(h[0]) + __uint_as_float(h[1]);
 }
 
 // ── complex helpers ──

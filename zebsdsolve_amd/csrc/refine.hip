@@ -1,13 +1,17 @@
-// Orientation refinement on the detector, fused: one wave (64 lanes) per item runs the seed, every
-// Gauss-Newton iteration, the normalized mutual information and the record, in one launch
-// (the reference's detector.wgsl seed, refine_init, sums_rot + refine_rot_step per iteration,
-// nmi and collect; src/detector.zig:178-212).
+// Orientation refinement on the detector, fused: one block of 2 to 16 waves (64 lanes each) per
+// item runs the seed, every Gauss-Newton iteration, the normalized mutual information and the
+// record, in one launch (the reference's detector.wgsl seed, refine_init, sums_rot +
+// refine_rot_step per iteration, nmi and collect; src/detector.zig:178-212).
 //
 // Per iteration each lane adds up its pixels' share of the 19 sums the step needs (1, M, M^2,
-// M e, d, M d, e d and the upper triangle of d d', with d = c x grad M(c) for c = q . ray); an
-// xor-butterfly over the wave leaves every lane with the same totals (a + b == b + a bit for
-// bit), so every lane takes the same step with no broadcast and no barrier. The master's
-// gradient field holds (grad M, M) per texel: one bilinear lookup reads both.
+// M e, d, M d, e d and the upper triangle of d d', with d = c x grad M(c) for c = q . ray); the
+// wave that adds the last pixels sums over the lanes and takes the step for the block. The
+// master's gradient field holds (grad M, M) per texel: one bilinear lookup reads both.
+// What bounds it: the gathers' cache lines (a step of 64 pixels touches 70 to 100 lines of 128
+// bytes, at 64 bytes a clock into the CU's cache) beside 110 vector instructions a step. One wave an
+// item, its list and pattern read again in each pass, left most of the chip idle for few or large
+// items: 8 items of 120 x 120 took 723 us and take 235, 40 of 240 x 240 3 673 and 569, 4 500 of
+// 60 x 60 634 and 513, 16 000 1 944 and 1 716 (5 iterations at 60 x 60, 8 else).
 #include <algorithm>
 #include <map>
 #include <mutex>
@@ -24,29 +28,24 @@ struct RefArg {
     int iters, nmi_bins, seed_stride, out0;
     float max_step, scale0, scale_min, scale_max;
     float stamp;
-    // 1: the masked pixels as a list of 16-bit indices in LDS (frames up to 65 536 pixels whose
-    // list fits); 0: the whole frame walked, each pixel tested against the mask (larger frames)
-    int use_list;
+    int tiles;  // 8 x 8 tiles of the frame the tile walk lists (0: every tile is walked)
 };
-
-struct Sums {
-    float n, m, mm, me;
-    float3 sd, sv, se, hd, ho;
-};
-
-__device__ __forceinline__ float3 f3add(float3 a, float3 b) { return make_float3(a.x + b.x, a.y + b.y, a.z + b.z); }
-__device__ __forceinline__ float3 f3s(float3 a, float s) { return make_float3(a.x * s, a.y * s, a.z * s); }
-
-__device__ __forceinline__ float wsum(float v) {
-    for (int o = 1; o < 64; o <<= 1) v += __shfl_xor(v, o, 64);
-    return v;
-}
-
-__device__ __forceinline__ float3 wsum3(float3 v) { return make_float3(wsum(v.x), wsum(v.y), wsum(v.z)); }
 
 // A value every lane holds alike, read from the first lane into a scalar register.
 __device__ __forceinline__ float ufloat(float v) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v))); }
 __device__ __forceinline__ float4 uniform4(float4 v) { return make_float4(ufloat(v.x), ufloat(v.y), ufloat(v.z), ufloat(v.w)); }
+// (a number known to the compiler, as an argument)
+template <int N>
+struct Const {
+    static constexpr int value = N;
+};
+__device__ __forceinline__ float lane_of(float v, int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); }
+__device__ __forceinline__ float3 f3s(float3 a, float s) { return make_float3(a.x * s, a.y * s, a.z * s); }
+
+__device__ __forceinline__ bool under_mask(const RefArg& a, int r, int c) {
+    const float dr = (float)r - a.mask[0], dc = (float)c - a.mask[1];
+    return r < a.h && c < a.w && (a.mask[2] <= 0.f || dr * dr + dc * dc <= a.mask[2]);
+}
 
 // The masked pixels of the frame as pixel indices, built by each block into LDS (the same list
 // for every item): the passes then walk only the pixels under the mask, 64 at a time, instead of
@@ -54,133 +53,218 @@ __device__ __forceinline__ float4 uniform4(float4 v) { return make_float4(ufloat
 // row-major tile order, each tile's pixels row-major), so that the 64 lanes of a pass look up a
 // compact patch of the detector, whose rays land on nearby texels of the master, rather than a
 // row segment, whose rays trace a long curve across it: fewer cache lines per gather (the
-// refinement 6.8 % faster than with row-major order).
-__device__ int build_list(const RefArg& a, unsigned short* list, int lane) {
-    const int tw = (a.w + 7) >> 3, th = (a.h + 7) >> 3, nt = tw * th;
-    auto inside = [&](int r, int c) {
-        const float dr = (float)r - a.mask[0], dc = (float)c - a.mask[1];
-        return a.mask[2] <= 0.f || dr * dr + dc * dc <= a.mask[2];
-    };
-    int total = 0;
-    for (int t0 = 0; t0 < nt; t0 += 64) {
-        // lane t counts its tile's masked pixels; an exclusive prefix over the 64 tiles places them
-        const int t = t0 + lane;
-        const int r0 = (t / tw) * 8, c0 = (t % tw) * 8;
-        int cnt = 0;
-        if (t < nt)
-            for (int r = r0; r < min(r0 + 8, a.h); ++r)
-                for (int c = c0; c < min(c0 + 8, a.w); ++c) cnt += inside(r, c) ? 1 : 0;
-        int inc = cnt;
-        for (int o = 1; o < 64; o <<= 1) {
-            const int y = __shfl_up(inc, o, 64);
-            if (lane >= o) inc += y;
+// refinement 6.8 % faster than with row-major order). One lane a pixel of the tile, the place in
+// the list from the tile's ballot; with several waves each takes a run of the tiles, counted
+// first (cnt: an int a wave). TILES: the tiles that hold a masked pixel instead, as tile numbers.
+template <int W, bool TILES>
+__device__ int build_list(const RefArg& a, unsigned short* list, int* cnt, int wave, int lane) {
+    const int tw = (a.w + 7) >> 3, nt = tw * ((a.h + 7) >> 3);
+    const int per = (nt + W - 1) / W;
+    const int t_lo = min(wave * per, nt), t_hi = min(t_lo + per, nt);
+    const int y = lane >> 3, x = lane & 7;
+    int at = 0, total = 0;
+    auto walk = [&](auto put) {
+        int tr = t_lo / tw, tc = t_lo - (t_lo / tw) * tw;
+        for (int t = t_lo; t < t_hi; ++t) {
+            const int r = tr * 8 + y, c = tc * 8 + x;
+            const bool in = under_mask(a, r, c);
+            const unsigned long long m = __ballot(in);
+            put(t, r, c, in, m);
+            at += TILES ? (m ? 1 : 0) : __popcll(m);
+            if (++tc == tw) tc = 0, ++tr;
         }
-        int at = total + inc - cnt;
-        if (t < nt)
-            for (int r = r0; r < min(r0 + 8, a.h); ++r)
-                for (int c = c0; c < min(c0 + 8, a.w); ++c)
-                    if (inside(r, c)) list[at++] = (unsigned short)(r * a.w + c);
-        total += __shfl(inc, 63, 64);
+    };
+    if constexpr (W > 1) {
+        // (counted)
+        walk([](int, int, int, bool, unsigned long long) {});
+        if (lane == 0) cnt[wave] = at;
+        __syncthreads();
+        at = 0;
+        for (int v = 0; v < W; ++v) {
+            const int k = cnt[v];
+            if (v < wave) at += k;
+            total += k;
+        }
     }
+    walk([&](int t, int r, int c, bool in, unsigned long long m) {
+        if constexpr (TILES) {
+            if (m && lane == 0) list[at] = (unsigned short)t;
+        } else {
+            if (in) list[at + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u))] = (unsigned short)(r * a.w + c);
+        }
+    });
+    if constexpr (W == 1) total = at;
     __syncthreads();
     return total;
 }
 
-// Pixel k of a pass: the list's k-th (the masked pixels, in LDS) or, without a list, the
-// frame's k-th; `ok` says whether it counts (k inside the pass, the pixel under the mask). Past
-// the end the last pixel is looked up again and counts for nothing.
-template <bool LIST>
-__device__ __forceinline__ int pass_pixel(const RefArg& a, const unsigned short* list, int n_px, int k, bool& ok) {
-    const int kk = min(k, n_px - 1);
-    if constexpr (LIST) {
-        ok = k < n_px;
-        return list[kk];
-    }
-    const int row = kk / a.w;
-    const float dr = (float)row - a.mask[0], dc = (float)(kk - row * a.w) - a.mask[1];
-    ok = k < n_px && (a.mask[2] <= 0.f || dr * dr + dc * dc <= a.mask[2]);
-    return kk;
-}
-
-// The ray of pixel `pix` (row-major index) from the item's origin t, in the sample frame; the
-// row by a float product below 65 536 pixels (exact there), by division above.
-template <bool LIST>
-__device__ __forceinline__ float3 pixel_ray(const RefArg& a, int pix, float inv_w, float3 t) {
-    const int row = LIST ? (int)(((float)pix + 0.5f) * inv_w) : pix / a.w;
-    const float fr = (float)row, fc = (float)(pix - row * a.w);
-    return make_float3(a.c0[0] * fr + a.c1[0] * fc + t.x, a.c0[1] * fr + a.c1[1] * fc + t.y, a.c0[2] * fr + a.c1[2] * fc + t.z);
-}
-
+// An item's masked pixels are taken 64 a step, one a lane. A list form's steps are the list's
+// entries in order, cut into chunks of consecutive steps dealt to the block's W waves in turn.
+// Each wave looks its chunk's pixels up by itself and keeps what the sums need in registers; the
+// sums then run through the chunks in order, handed from wave to wave through LDS, so that each
+// lane adds its pixels up in the list's order whatever W is: a record's bits depend neither on the
+// launch nor on the batch. (With partial sums a wave the last steps' acceptance, decided in the
+// sums' last bits, came out otherwise for some items.) The look-ups are eight parts in nine of a
+// pass's instructions and run side by side; the chain of additions is the rest.
+//  REF_HELD: at most kHeld steps a wave: each lane holds its pixels' rays and pattern values in
+//            registers over all passes;
+//  REF_LIST: any number, the list and the pattern read again in each pass;
+//  REF_TILES: frames whose pixels pass 16-bit indices or whose list passes LDS: a step is one
+//            8 x 8 tile of the frame with the mask tested a pixel, from the list of tiles that hold
+//            a masked pixel (every tile where that list passes LDS: tiles = 0), step s to wave s
+//            mod W, and each wave's sums are added up on their own.
+enum { REF_HELD, REF_LIST, REF_TILES };
+constexpr int kHeld = 12;   // steps a lane holds (REF_HELD)
+constexpr int kChunk = 6;   // steps of a chunk
 // Pixels per lane whose gathers are in flight together: a lane issues the loads of kBatch pixels
-// (3 each) before it blends any.
-constexpr int kBatch = 4;
+// (2 each) before it blends any.
+constexpr int kBatch = 3;
+constexpr int kPart = 20;  // floats handed over: the 19 sums of a pass and a pad
 
-template <bool LIST>
-__device__ Sums rot_sums(const RefArg& a, __amdgpu_buffer_rsrc_t mgh, const float* __restrict__ pat, const unsigned short* list, int n_px,
-                         float inv_w, float4 q, float3 t, int lane) {
-    Sums s;
-    s.n = s.m = s.mm = s.me = 0.f;
-    s.sd = s.sv = s.se = s.hd = s.ho = make_float3(0.f, 0.f, 0.f);
-    for (int k0 = lane; k0 < n_px; k0 += 64 * kBatch) {
-        TapsH tp[kBatch];
-        float3 c[kBatch];
-        float e[kBatch];
+// The refinement's state (detector.wgsl refine_init), kept in LDS between the passes (its
+// registers would be every wave's).
+struct Gn {
+    float4 cur, qbest;
+    float best, mu;
+    float3 gbest;
+    float hbest[6];
+    float last_step, promised, step_size, accepted;
+};
+
+template <int W>
+struct alignas(16) Shared {
+    float4 acc[kPart / 4][64];  // the chain's sums, a lane's own (list forms)
+    float part[W][kPart];       // each wave's sums (REF_TILES); each wave's extremes
+    Gn gn;
+    int cnt[W];
+    int turn;  // the chunk whose sums are to be added next, counted over the item's passes
+};
+
+struct Held {
+    float3 u[kHeld];
+    float e[kHeld];
+};
+
+// The chunks of n_steps for W waves: as even as whole steps allow, at most kChunk steps each.
+struct Chunks {
+    int steps, size, count, rounds;
+};
+template <int W>
+__device__ __forceinline__ Chunks chunks_of(int n_px) {
+    Chunks c;
+    c.steps = (n_px + 63) >> 6;
+    c.rounds = max((c.steps + W * kChunk - 1) / (W * kChunk), 1);
+    c.size = max((c.steps + W * c.rounds - 1) / (W * c.rounds), 1);
+    c.count = max((c.steps + c.size - 1) / c.size, 1);
+    return c;
+}
+
+// Waits until the chain reaches chunk `id` (its turn comes after finitely many chunks of other
+// waves of the block, all resident; the bound only keeps a wave from waiting for ever).
+__device__ __forceinline__ void wait_turn(int* turn, int id) {
+    for (int k = 0; k < (1 << 22); ++k) {
+        if (__builtin_amdgcn_readfirstlane(__hip_atomic_load(turn, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP)) == id) break;
+        __builtin_amdgcn_s_sleep(1);
+    }
+}
+__device__ __forceinline__ void pass_turn(int* turn, int id, int lane) {
+    if (lane == 0) __hip_atomic_store(turn, id + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// Steps wave `wave` takes of n_steps dealt one by one.
+template <int W>
+__device__ __forceinline__ int own_steps(int n_steps, int wave) {
+    return (n_steps - wave + W - 1) / W;
+}
+
+// The ray of pixel (row, col) from the item's origin t, in the sample frame, of unit length.
+__device__ __forceinline__ float3 pixel_ray(const RefArg& a, int row, int col, float3 t) {
+    const float fr = (float)row, fc = (float)col;
+    return normalize3(make_float3(a.c0[0] * fr + a.c1[0] * fc + t.x, a.c0[1] * fr + a.c1[1] * fc + t.y, a.c0[2] * fr + a.c1[2] * fc + t.z));
+}
+
+// A list form's pixel k: its ray and pattern value. The row by a float product (exact below
+// 65 536 pixels).
+__device__ __forceinline__ float3 list_pixel(const RefArg& a, const unsigned short* list, int k, int n_px, float inv_w, float3 t,
+                                             const float* __restrict__ pat, float& e) {
+    const int pix = list[min(k, n_px - 1)];
+    const int row = (int)(((float)pix + 0.5f) * inv_w);
+    e = pat[pix];
+    return pixel_ray(a, row, pix - __mul24(row, a.w), t);
+}
+
+// The look-ups of one chunk of a list form, kBatch steps in flight: tap(p, ray) issues the loads
+// of step p of the batch, keep(i, p, ray, pattern value) takes step i's in.
+template <int MODE, int ROUND, typename Tap, typename Keep>
+__device__ __forceinline__ void look_up(const RefArg& a, const unsigned short* list, int n_px, float inv_w, float3 t, const float* __restrict__ pat,
+                                        const Held& held, int step0, int cnt, int lane, Tap tap, Keep keep) {
+#pragma unroll
+    for (int i0 = 0; i0 < kChunk; i0 += kBatch) {
+        if (i0 < cnt) {
+            float3 u[kBatch];
+            float e[kBatch];
+#pragma unroll
+            for (int p = 0; p < kBatch; ++p) {
+                if constexpr (MODE == REF_HELD) {
+                    u[p] = held.u[ROUND * kChunk + i0 + p];
+                    e[p] = held.e[ROUND * kChunk + i0 + p];
+                } else {
+                    u[p] = list_pixel(a, list, 64 * (step0 + i0 + p) + lane, n_px, inv_w, t, pat, e[p]);
+                }
+                u[p] = tap(p, u[p]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int p = 0; p < kBatch; ++p) keep(i0 + p, p, u[p], e[p]);
+        }
+    }
+}
+
+// One wave's tiles, kBatch in flight: tap(p, ray, pixel) issues the loads of step p of the batch,
+// keep(p) takes them in on the lanes whose pixel counts.
+template <int W, typename Tap, typename Keep>
+__device__ __forceinline__ void walk_tiles(const RefArg& a, const unsigned short* list, int n_tiles, float3 t, int wave, int lane, Tap tap, Keep keep) {
+    const int tw = (a.w + 7) >> 3;
+    const int own = own_steps<W>(n_tiles, wave);
+    for (int i0 = 0; i0 < own; i0 += kBatch) {
         bool ok[kBatch];
 #pragma unroll
         for (int p = 0; p < kBatch; ++p) {
-            // lanes past the end (or off the mask) look up a pixel and add nothing
-            const int pix = pass_pixel<LIST>(a, list, n_px, k0 + 64 * p, ok[p]);
-            c[p] = qrot(q, normalize3(pixel_ray<LIST>(a, pix, inv_w, t)));
-            sheet_taps_h(mgh, a.side, c[p], tp[p]);
-            e[p] = pat[pix];
+            // steps past the end look up the wave's last tile again and add nothing
+            const int k = wave + W * min(i0 + p, own - 1);
+            const int tile = __builtin_amdgcn_readfirstlane(a.tiles ? (int)list[k] : k);
+            const int tr = tile / tw;
+            const int r = tr * 8 + (lane >> 3), c = (tile - tr * tw) * 8 + (lane & 7);
+            ok[p] = i0 + p < own && under_mask(a, r, c);
+            const int rr = min(r, a.h - 1), cc = min(c, a.w - 1);
+            tap(p, pixel_ray(a, rr, cc, t), rr * a.w + cc);
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int p = 0; p < kBatch; ++p) {
-            if (ok[p]) {
-                const float4 m = taps_blend(tp[p]);
-                const float3 d = cross3(c[p], make_float3(m.x, m.y, m.z));
-                s.n += 1.f;
-                s.m += m.w;
-                s.mm += m.w * m.w;
-                s.me += m.w * e[p];
-                s.sd = f3add(s.sd, d);
-                s.sv = f3add(s.sv, f3s(d, m.w));
-                s.se = f3add(s.se, f3s(d, e[p]));
-                s.hd = f3add(s.hd, make_float3(d.x * d.x, d.y * d.y, d.z * d.z));
-                s.ho = f3add(s.ho, make_float3(d.x * d.y, d.x * d.z, d.y * d.z));
-            }
-        }
+        for (int p = 0; p < kBatch; ++p)
+            if (ok[p]) keep(p);
     }
-    s.n = wsum(s.n);
-    s.m = wsum(s.m);
-    s.mm = wsum(s.mm);
-    s.me = wsum(s.me);
-    s.sd = wsum3(s.sd);
-    s.sv = wsum3(s.sv);
-    s.se = wsum3(s.se);
-    s.hd = wsum3(s.hd);
-    s.ho = wsum3(s.ho);
-    return s;
 }
 
-// The master's values at orientation q for the list pixels k0 + 64 p, p < kBatch (lanes past the
-// end get the last pixel's), with the pattern's values there: all gathers issued before any
-// blend. msh: a buffer resource over the float32 sheets.
-template <bool LIST>
-__device__ __forceinline__ void sims_batch(const RefArg& a, __amdgpu_buffer_rsrc_t msh, const float* __restrict__ pat,
-                                           const unsigned short* list, int n_px, float inv_w, float4 q, float3 t, int k0,
-                                           float* sim, float* e, bool* ok) {
-    TapsM tp[kBatch];
+// 20 values summed over the wave's lanes: lane 16 r ends with the sums of v[4 j + {0, 2, 1, 3}[r]],
+// j < 5. Two values share a register after each of the first two exchanges (halves, then rows of
+// 16), so that the sums take 50 instructions, not the 120 of a butterfly for each.
+__device__ __forceinline__ void wave_sums20(const float* v, float* out) {
+    float x[10];
 #pragma unroll
-    for (int p = 0; p < kBatch; ++p) {
-        const int pix = pass_pixel<LIST>(a, list, n_px, k0 + 64 * p, ok[p]);
-        sheet_taps_m(msh, a.side, qrot(q, normalize3(pixel_ray<LIST>(a, pix, inv_w, t))), tp[p]);
-        e[p] = pat[pix];
+    for (int i = 0; i < 10; ++i) {
+        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[2 * i]), __float_as_uint(v[2 * i + 1]), false, false);
+        x[i] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
     }
-    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int p = 0; p < kBatch; ++p) sim[p] = taps_blend(tp[p]);
+    for (int j = 0; j < 5; ++j) {
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x[2 * j]), __float_as_uint(x[2 * j + 1]), false, false);
+        float s = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+        s = dpp_add<0x128>(s);  // row_ror:8, 4, 2, 1
+        s = dpp_add<0x124>(s);
+        s = dpp_add<0x122>(s);
+        out[j] = dpp_add<0x121>(s);
+    }
 }
 
 __device__ __forceinline__ float det3(float3 c0, float3 c1, float3 c2) {
@@ -197,134 +281,300 @@ __device__ __forceinline__ float3 solve3(const float* h, float3 g) {
     return make_float3(det3(g, m1, m2) / det, det3(m0, g, m2) / det, det3(m0, m1, g) / det);
 }
 
-// One item's refinement, NMI and record (at records[out0 + b]), with the masked-pixel list (LIST)
-// already built and the histogram cleared.
+// One pass's sums s (count, M, M^2, M e, M d, d, e d, d d' diagonal and off it, as rot_sums lays
+// them out) taken in: the NCC, its gradient and Gauss-Newton matrix over the rotation
+// (detector.wgsl:561-583), acceptance against the best so far, and unless `last` the next step.
+__device__ __forceinline__ void gn_step(const RefArg& a, const float* s, bool last, Gn& g) {
+    const float n = fmaxf(s[0], 1.f);
+    const float mean = s[1] / n;
+    const float var_n = s[2] - n * mean * mean;
+    float ncc = -2.f;
+    float3 grad = make_float3(0.f, 0.f, 0.f);
+    float hess[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    const float3 sd = make_float3(s[4], s[5], s[6]), sv = make_float3(s[7], s[8], s[9]), se = make_float3(s[10], s[11], s[12]);
+    if (var_n > 1e-12f) {
+        const float inv = 1.f / sqrtf(var_n);
+        ncc = s[3] * inv;
+        const float3 au = f3s(make_float3(sv.x - mean * sd.x, sv.y - mean * sd.y, sv.z - mean * sd.z), inv);
+        grad = f3s(make_float3(se.x - ncc * au.x, se.y - ncc * au.y, se.z - ncc * au.z), inv);
+        const float iv = inv * inv;
+        hess[0] = (s[13] - sd.x * sd.x / n - au.x * au.x) * iv;
+        hess[1] = (s[16] - sd.x * sd.y / n - au.x * au.y) * iv;
+        hess[2] = (s[17] - sd.x * sd.z / n - au.x * au.z) * iv;
+        hess[3] = (s[14] - sd.y * sd.y / n - au.y * au.y) * iv;
+        hess[4] = (s[18] - sd.y * sd.z / n - au.y * au.z) * iv;
+        hess[5] = (s[15] - sd.z * sd.z / n - au.z * au.z) * iv;
+    }
+    // accept against the best so far, rescaling the curvature by gain / promise
+    if (ncc > g.best) {
+        if (g.accepted > 0.5f && g.promised > 1e-6f) {
+            const float rho = (ncc - g.best) / g.promised;
+            g.mu = fminf(fmaxf(g.mu * (2.f - rho), g.mu / 3.f), g.mu * 3.f);
+        }
+        g.qbest = g.cur;
+        g.best = ncc;
+        g.gbest = grad;
+#pragma unroll
+        for (int i = 0; i < 6; ++i) g.hbest[i] = hess[i];
+        g.last_step = g.step_size;
+        g.accepted += 1.f;
+    } else {
+        g.mu = g.mu * 3.f;
+    }
+    g.mu = fminf(fmaxf(g.mu, a.scale_min), a.scale_max);
+    if (last) return;
+    float hh[6];
+#pragma unroll
+    for (int i = 0; i < 6; ++i) hh[i] = g.hbest[i] * g.mu;
+    const float tr = fmaxf(hh[0] + hh[3] + hh[5], 1e-20f);
+    hh[0] += 1e-6f * tr;
+    hh[3] += 1e-6f * tr;
+    hh[5] += 1e-6f * tr;
+    float3 st = solve3(hh, g.gbest);
+    const float len = sqrtf(dot3(st, st));
+    if (len > a.max_step) st = f3s(st, a.max_step / len);
+    const float quad = hh[0] * st.x * st.x + hh[3] * st.y * st.y + hh[5] * st.z * st.z +
+                       2.f * (hh[1] * st.x * st.y + hh[2] * st.x * st.z + hh[4] * st.y * st.z);
+    g.promised = dot3(g.gbest, st) - 0.5f * quad;
+    g.step_size = sqrtf(dot3(st, st));
+    g.cur = qnormalize(qmul(qexp(st), g.qbest));
+}
+
+// What one pixel adds to a pass's sums: 0 count, 1 M, 2 M^2, 3 M e, 4 d, 7 M d, 10 e d, 13 d d'
+// diagonal, 16 off it (d = c x grad M in the direction c, e the pattern's value).
+__device__ __forceinline__ void add_pixel(float* s, float m, float3 d, float e) {
+    s[0] += 1.f;
+    s[1] += m;
+    s[2] += m * m;
+    s[3] += m * e;
+    s[4] += d.x, s[5] += d.y, s[6] += d.z;
+    s[7] += d.x * m, s[8] += d.y * m, s[9] += d.z * m;
+    s[10] += d.x * e, s[11] += d.y * e, s[12] += d.z * e;
+    s[13] += d.x * d.x, s[14] += d.y * d.y, s[15] += d.z * d.z;
+    s[16] += d.x * d.y, s[17] += d.x * d.z, s[18] += d.y * d.z;
+}
+
+// One item's refinement, NMI and record (at records[out0 + b]) by the block's W waves, with the
+// list of masked pixels or tiles already built and the histogram cleared.
 // The Gauss-Newton passes read the half-precision gradient field (mgh: two adjacent 16-byte loads
 // a lookup, each a texel and the one below it; half the vector-memory instructions of float32
-// texels); the recorded NCC and
-// the NMI are those of the float32 master (ms, the values the field holds in .w) at the best
-// orientation, from the NMI's first pass (one 8-byte load per texel row pair).
-// MAXP > 0: each lane keeps the master values of its (at most MAXP) pixels at the best
-// orientation from the first NMI pass for the second; MAXP = 0: the second pass looks them up
-// again.
-template <int MAXP, bool LIST>
+// texels); the recorded NCC and the NMI are those of the float32 master (ms, the values the field
+// holds in .w) at the best orientation, from the NMI's first pass (one 8-byte load per texel row
+// pair). REF_HELD keeps its pixels' master values from that pass for the second, the others look
+// them up again.
+template <int W, int MODE>
 __device__ __forceinline__ void refine_item(const RefArg& a, const float* __restrict__ ms, const uint2* __restrict__ mgh, const float* __restrict__ pats,
                                             const float4* __restrict__ items, const float* __restrict__ seeds, int seed_stride,
-                                            float* __restrict__ records, int out0, unsigned* hist, const unsigned short* list, int n_px, int b,
-                                            int lane) {
-    static_assert(MAXP % kBatch == 0, "MAXP: whole batches");
+                                            float* __restrict__ records, int out0, unsigned* hist, const unsigned short* list, int n_px,
+                                            Shared<W>& sh, int b, int wave, int lane) {
     const float inv_w = 1.f / (float)a.w;
     // the item's values are the same in every lane: held in scalar registers
     const float4 it = uniform4(items[b]);
     const float3 t = make_float3(it.x, it.y, it.z);
     const float* pat = pats + (size_t)(int)it.w * a.h * a.w;
-    const float* sd = seeds + (size_t)b * seed_stride;
-    float4 cur = uniform4(make_float4(sd[0], sd[1], sd[2], sd[3]));
-
-    // refinement state (detector.wgsl refine_init)
-    float4 qbest = cur;
-    float best = -2.f;
-    float mu = a.scale0;
-    float3 gbest = make_float3(0.f, 0.f, 0.f);
-    float hbest[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    float last_step = 0.f, promised = 0.f, step_size = 0.f, accepted = 0.f;
+    const Chunks ch = chunks_of<W>(MODE == REF_TILES ? 0 : n_px);
+    // the wave's chunk of round `round`: its first step and its steps (0: none)
+    auto chunk = [&](int round, int& id, int& step0) {
+        id = round * W + wave;
+        step0 = id * ch.size;
+        return min(max(ch.steps - step0, 0), ch.size);
+    };
+    Held held;
+    if constexpr (MODE == REF_HELD) {
+#pragma unroll
+        for (int r = 0; r < kHeld / kChunk; ++r) {
+            int id, step0;
+            const int cnt = r < ch.rounds ? chunk(r, id, step0) : 0;
+#pragma unroll
+            for (int i = 0; i < kChunk; ++i) {
+                held.u[r * kChunk + i] = make_float3(0.f, 0.f, 1.f);
+                held.e[r * kChunk + i] = 0.f;
+                if (i < cnt)
+                    held.u[r * kChunk + i] = list_pixel(a, list, 64 * (step0 + i) + lane, n_px, inv_w, t, pat, held.e[r * kChunk + i]);
+            }
+        }
+    }
+    if (wave == 0) {
+        Gn g;
+        const float* sd = seeds + (size_t)b * seed_stride;
+        g.cur = make_float4(ufloat(sd[0]), ufloat(sd[1]), ufloat(sd[2]), ufloat(sd[3]));
+        g.qbest = g.cur;
+        g.best = -2.f;
+        g.mu = a.scale0;
+        g.gbest = make_float3(0.f, 0.f, 0.f);
+#pragma unroll
+        for (int i = 0; i < 6; ++i) g.hbest[i] = 0.f;
+        g.last_step = g.promised = g.step_size = g.accepted = 0.f;
+        if (lane == 0) {
+            sh.gn = g;
+            sh.turn = 0;
+        }
+    }
+    __syncthreads();
     const __amdgpu_buffer_rsrc_t fh = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint2*>(mgh), (short)0, 2 * a.side * a.side * 16, 0x00020000);
     const __amdgpu_buffer_rsrc_t fm = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(ms), (short)0, 2 * a.side * a.side * 4, 0x00020000);
 
+    int base = 0;  // chunks of the passes before
     for (int itn = 0; itn <= a.iters; ++itn) {
-        const Sums s = rot_sums<LIST>(a, fh, pat, list, n_px, inv_w, cur, t, lane);
-        // NCC, its gradient and Gauss-Newton matrix over the rotation (detector.wgsl:561-583)
-        const float n = fmaxf(s.n, 1.f);
-        const float mean = s.m / n;
-        const float var_n = s.mm - n * mean * mean;
-        float ncc = -2.f;
-        float3 grad = make_float3(0.f, 0.f, 0.f);
-        float hess[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        if (var_n > 1e-12f) {
-            const float inv = 1.f / sqrtf(var_n);
-            ncc = s.me * inv;
-            const float3 au = f3s(make_float3(s.sv.x - mean * s.sd.x, s.sv.y - mean * s.sd.y, s.sv.z - mean * s.sd.z), inv);
-            grad = f3s(make_float3(s.se.x - ncc * au.x, s.se.y - ncc * au.y, s.se.z - ncc * au.z), inv);
-            const float iv = inv * inv;
-            hess[0] = (s.hd.x - s.sd.x * s.sd.x / n - au.x * au.x) * iv;
-            hess[1] = (s.ho.x - s.sd.x * s.sd.y / n - au.x * au.y) * iv;
-            hess[2] = (s.ho.y - s.sd.x * s.sd.z / n - au.x * au.z) * iv;
-            hess[3] = (s.hd.y - s.sd.y * s.sd.y / n - au.y * au.y) * iv;
-            hess[4] = (s.ho.z - s.sd.y * s.sd.z / n - au.y * au.z) * iv;
-            hess[5] = (s.hd.z - s.sd.z * s.sd.z / n - au.z * au.z) * iv;
-        }
-        // accept against the best so far, rescaling the curvature by gain / promise
-        if (ncc > best) {
-            if (accepted > 0.5f && promised > 1e-6f) {
-                const float rho = (ncc - best) / promised;
-                mu = fminf(fmaxf(mu * (2.f - rho), mu / 3.f), mu * 3.f);
+        const Turn q = turn_of(uniform4(sh.gn.cur));
+        float s[kPart];
+#pragma unroll
+        for (int i = 0; i < kPart; ++i) s[i] = 0.f;
+        TapsH tp[kBatch];
+        auto take_step = [&]() {
+            Gn g = sh.gn;
+            gn_step(a, s, itn == a.iters, g);
+            if (lane == 0) sh.gn = g;
+        };
+        if constexpr (MODE != REF_TILES) {
+            auto round = [&](int r, auto rc) {
+                int id, step0;
+                const int cnt = chunk(r, id, step0);
+                if (id >= ch.count) return;
+                float m[kChunk], e[kChunk];
+                float3 d[kChunk];
+                look_up<MODE, decltype(rc)::value>(
+                    a, list, n_px, inv_w, t, pat, held, step0, cnt, lane,
+                    [&](int p, float3 u) {
+                        const float3 c = turn(q, u);
+                        sheet_taps_h(fh, a.side, c, tp[p]);
+                        return c;
+                    },
+                    [&](int i, int p, float3 c, float ev) {
+                        const float4 v = taps_blend(tp[p]);
+                        d[i] = cross3(c, make_float3(v.x, v.y, v.z));
+                        m[i] = v.w;
+                        e[i] = ev;
+                    });
+                wait_turn(&sh.turn, base + id);
+                if (id > 0) {
+#pragma unroll
+                    for (int j = 0; j < kPart / 4; ++j) {
+                        const float4 x = sh.acc[j][lane];
+                        s[4 * j] = x.x, s[4 * j + 1] = x.y, s[4 * j + 2] = x.z, s[4 * j + 3] = x.w;
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < kChunk; ++i)
+                    if (i < cnt && 64 * (step0 + i) + lane < n_px) add_pixel(s, m[i], d[i], e[i]);
+                if (id + 1 < ch.count) {
+#pragma unroll
+                    for (int j = 0; j < kPart / 4; ++j) sh.acc[j][lane] = make_float4(s[4 * j], s[4 * j + 1], s[4 * j + 2], s[4 * j + 3]);
+                    pass_turn(&sh.turn, base + id, lane);
+                } else {
+                    // the pass's last chunk: the totals and the step
+#pragma unroll
+                    for (int i = 0; i < kPart - 1; ++i) s[i] = wave_sum(s[i]);
+                    take_step();
+                    pass_turn(&sh.turn, base + id, lane);
+                }
+            };
+            if constexpr (MODE == REF_HELD) {
+                round(0, Const<0>{});
+                if (ch.rounds > 1) round(1, Const<1>{});
+            } else {
+                for (int r = 0; r < ch.rounds; ++r) round(r, Const<0>{});
             }
-            qbest = cur;
-            best = ncc;
-            gbest = grad;
-#pragma unroll
-            for (int i = 0; i < 6; ++i) hbest[i] = hess[i];
-            last_step = step_size;
-            accepted += 1.f;
+            base += ch.count;
         } else {
-            mu = mu * 3.f;
-        }
-        mu = fminf(fmaxf(mu, a.scale_min), a.scale_max);
-        if (itn == a.iters) break;
-        float hh[6];
+            float3 c[kBatch];
+            float e[kBatch];
+            walk_tiles<W>(
+                a, list, n_px, t, wave, lane,
+                [&](int p, float3 u, int pix) {
+                    c[p] = turn(q, u);
+                    sheet_taps_h(fh, a.side, c[p], tp[p]);
+                    e[p] = pat[pix];
+                },
+                [&](int p) {
+                    const float4 v = taps_blend(tp[p]);
+                    add_pixel(s, v.w, cross3(c[p], make_float3(v.x, v.y, v.z)), e[p]);
+                });
+            float part[5];
+            wave_sums20(s, part);
+            if ((lane & 15) == 0) {
+                const int r = lane >> 4, at = r == 1 ? 2 : r == 2 ? 1 : r;
 #pragma unroll
-        for (int i = 0; i < 6; ++i) hh[i] = hbest[i] * mu;
-        const float tr = fmaxf(hh[0] + hh[3] + hh[5], 1e-20f);
-        hh[0] += 1e-6f * tr;
-        hh[3] += 1e-6f * tr;
-        hh[5] += 1e-6f * tr;
-        float3 st = solve3(hh, gbest);
-        const float len = sqrtf(dot3(st, st));
-        if (len > a.max_step) st = f3s(st, a.max_step / len);
-        const float quad = hh[0] * st.x * st.x + hh[3] * st.y * st.y + hh[5] * st.z * st.z +
-                           2.f * (hh[1] * st.x * st.y + hh[2] * st.x * st.z + hh[4] * st.y * st.z);
-        promised = dot3(gbest, st) - 0.5f * quad;
-        step_size = sqrtf(dot3(st, st));
-        cur = qnormalize(qmul(qexp(st), qbest));
+                for (int j = 0; j < 5; ++j) sh.part[wave][4 * j + at] = part[j];
+            }
+            __syncthreads();
+            if (wave == 0) {
+                float v = 0.f;
+                if (lane < kPart)
+                    for (int w = 0; w < W; ++w) v += sh.part[w][lane];
+#pragma unroll
+                for (int i = 0; i < kPart; ++i) s[i] = lane_of(v, i);
+                take_step();
+            }
+        }
+        __syncthreads();
     }
 
     // normalized mutual information of the pattern and the master at the best orientation,
     // each binned between its own extremes under the mask (detector.wgsl:739-832)
+    const Turn q = turn_of(uniform4(sh.gn.qbest));
     const int nb = a.nmi_bins;
     float emin = 3.4e38f, emax = -3.4e38f, smin = 3.4e38f, smax = -3.4e38f;
-    float f_n = 0.f, f_m = 0.f, f_mm = 0.f, f_me = 0.f;  // the NCC's sums there (float32 master)
-    auto extremes = [&](float e, float sim) {
-        emin = fminf(emin, e);
-        emax = fmaxf(emax, e);
+    float4 f = make_float4(0.f, 0.f, 0.f, 0.f);  // the NCC's sums there (float32 master): count, M, M^2, M e
+    float simv[MODE == REF_HELD ? kHeld : 1];
+    TapsM tp[kBatch];
+    float e[kBatch];
+    auto extremes = [&](float ev, float sim) {
+        emin = fminf(emin, ev);
+        emax = fmaxf(emax, ev);
         smin = fminf(smin, sim);
         smax = fmaxf(smax, sim);
-        f_n += 1.f;
-        f_m += sim;
-        f_mm += sim * sim;
-        f_me += sim * e;
     };
-    float simv[MAXP > 0 ? MAXP : 1];
-    if constexpr (MAXP > 0) {
+    auto ncc_sums = [&](float ev, float sim) {
+        f.x += 1.f;
+        f.y += sim;
+        f.z += sim * sim;
+        f.w += sim * ev;
+    };
+    auto tap_m = [&](int p, float3 u) {
+        const float3 c = turn(q, u);
+        sheet_taps_m(fm, a.side, c, tp[p]);
+        return c;
+    };
+    auto tile_tap = [&](int p, float3 u, int pix) {
+        tap_m(p, u);
+        e[p] = pat[pix];
+    };
+    if constexpr (MODE != REF_TILES) {
+        auto round = [&](int r, auto rc) {
+            int id, step0;
+            const int cnt = chunk(r, id, step0);
+            if (id >= ch.count) return;
+            float sv[kChunk], ev[kChunk];
+            look_up<MODE, decltype(rc)::value>(a, list, n_px, inv_w, t, pat, held, step0, cnt, lane, tap_m, [&](int i, int p, float3, float x) {
+                sv[i] = taps_blend(tp[p]);
+                ev[i] = x;
+            });
 #pragma unroll
-        for (int i0 = 0; i0 < MAXP; i0 += kBatch) {
-            float sim[kBatch] = {}, e[kBatch] = {};
-            bool ok[kBatch] = {};
-            if (64 * i0 < n_px) sims_batch<LIST>(a, fm, pat, list, n_px, inv_w, qbest, t, lane + 64 * i0, sim, e, ok);
-#pragma unroll
-            for (int p = 0; p < kBatch; ++p) {
-                simv[i0 + p] = sim[p];
-                if (ok[p]) extremes(e[p], sim[p]);
+            for (int i = 0; i < kChunk; ++i) {
+                if constexpr (MODE == REF_HELD) simv[decltype(rc)::value * kChunk + i] = sv[i];
+                if (i < cnt && 64 * (step0 + i) + lane < n_px) extremes(ev[i], sv[i]);
             }
+            wait_turn(&sh.turn, base + id);
+            if (id > 0) f = sh.acc[0][lane];
+#pragma unroll
+            for (int i = 0; i < kChunk; ++i)
+                if (i < cnt && 64 * (step0 + i) + lane < n_px) ncc_sums(ev[i], sv[i]);
+            sh.acc[0][lane] = f;
+            pass_turn(&sh.turn, base + id, lane);
+        };
+        if constexpr (MODE == REF_HELD) {
+            round(0, Const<0>{});
+            if (ch.rounds > 1) round(1, Const<1>{});
+        } else {
+            for (int r = 0; r < ch.rounds; ++r) round(r, Const<0>{});
         }
     } else {
-        for (int k0 = lane; k0 < n_px; k0 += 64 * kBatch) {
-            float sim[kBatch], e[kBatch];
-            bool ok[kBatch];
-            sims_batch<LIST>(a, fm, pat, list, n_px, inv_w, qbest, t, k0, sim, e, ok);
-#pragma unroll
-            for (int p = 0; p < kBatch; ++p)
-                if (ok[p]) extremes(e[p], sim[p]);
-        }
+        walk_tiles<W>(a, list, n_px, t, wave, lane, tile_tap, [&](int p) {
+            const float sim = taps_blend(tp[p]);
+            extremes(e[p], sim);
+            ncc_sums(e[p], sim);
+        });
     }
     for (int o = 1; o < 64; o <<= 1) {
         emin = fminf(emin, __shfl_xor(emin, o, 64));
@@ -332,47 +582,46 @@ __device__ __forceinline__ void refine_item(const RefArg& a, const float* __rest
         smin = fminf(smin, __shfl_xor(smin, o, 64));
         smax = fmaxf(smax, __shfl_xor(smax, o, 64));
     }
-    // the recorded NCC: that of the float32 master at the best orientation (the rule of the
-    // Gauss-Newton passes)
-    float ncc_best = -2.f;
-    {
-        const float n = fmaxf(wsum(f_n), 1.f);
-        const float mean = wsum(f_m) / n;
-        const float var_n = wsum(f_mm) - n * mean * mean;
-        const float me = wsum(f_me);
-        if (var_n > 1e-12f) ncc_best = me * (1.f / sqrtf(var_n));
+    if constexpr (MODE == REF_TILES) f = make_float4(wave_sum(f.x), wave_sum(f.y), wave_sum(f.z), wave_sum(f.w));
+    if (lane == 0) {
+        float4* p = (float4*)sh.part[wave];
+        p[0] = make_float4(emin, emax, smin, smax);
+        p[1] = f;
+    }
+    __syncthreads();
+    for (int w = 0; w < W; ++w) {
+        const float4 x = ((const float4*)sh.part[w])[0];
+        emin = fminf(emin, x.x), emax = fmaxf(emax, x.y), smin = fminf(smin, x.z), smax = fmaxf(smax, x.w);
     }
     const float ke = (float)nb / fmaxf(emax - emin, 1e-20f);
     const float ks = (float)nb / fmaxf(smax - smin, 1e-20f);
-    auto bin = [&](float e, float sim) {
-        const int be = min((int)((e - emin) * ke), nb - 1);
+    auto bin = [&](float ev, float sim) {
+        const int be = min((int)((ev - emin) * ke), nb - 1);
         const int bs = min((int)((sim - smin) * ks), nb - 1);
         atomicAdd(&hist[be * nb + bs], 1u);
     };
-    if constexpr (MAXP > 0) {
+    if constexpr (MODE == REF_HELD) {
 #pragma unroll
-        for (int i0 = 0; i0 < MAXP; i0 += kBatch) {
-            if (64 * i0 < n_px) {
-                float e[kBatch];
-                bool ok[kBatch];
+        for (int r = 0; r < kHeld / kChunk; ++r) {
+            int id, step0;
+            const int cnt = r < ch.rounds ? chunk(r, id, step0) : 0;
 #pragma unroll
-                for (int p = 0; p < kBatch; ++p) e[p] = pat[pass_pixel<LIST>(a, list, n_px, lane + 64 * (i0 + p), ok[p])];
-#pragma unroll
-                for (int p = 0; p < kBatch; ++p)
-                    if (ok[p]) bin(e[p], simv[i0 + p]);
-            }
+            for (int i = 0; i < kChunk; ++i)
+                if (i < cnt && 64 * (step0 + i) + lane < n_px) bin(held.e[r * kChunk + i], simv[r * kChunk + i]);
+        }
+    } else if constexpr (MODE == REF_LIST) {
+        for (int r = 0; r < ch.rounds; ++r) {
+            int id, step0;
+            const int cnt = chunk(r, id, step0);
+            look_up<MODE, 0>(a, list, n_px, inv_w, t, pat, held, step0, cnt, lane, tap_m, [&](int i, int p, float3, float x) {
+                if (i < cnt && 64 * (step0 + i) + lane < n_px) bin(x, taps_blend(tp[p]));
+            });
         }
     } else {
-        for (int k0 = lane; k0 < n_px; k0 += 64 * kBatch) {
-            float sim[kBatch], e[kBatch];
-            bool ok[kBatch];
-            sims_batch<LIST>(a, fm, pat, list, n_px, inv_w, qbest, t, k0, sim, e, ok);
-#pragma unroll
-            for (int p = 0; p < kBatch; ++p)
-                if (ok[p]) bin(e[p], sim[p]);
-        }
+        walk_tiles<W>(a, list, n_px, t, wave, lane, tile_tap, [&](int p) { bin(e[p], taps_blend(tp[p])); });
     }
     __syncthreads();
+    if (wave != 0) return;
     float hj = 0.f, tot = 0.f, hm = 0.f;
     for (int i = lane; i < nb * nb; i += 64) {
         const float c = (float)hist[i];
@@ -388,60 +637,60 @@ __device__ __forceinline__ void refine_item(const RefArg& a, const float* __rest
         if (rs > 0.f) hm -= rs * logf(rs);
         if (cs > 0.f) hm -= cs * logf(cs);
     }
-    hj = wsum(hj);
-    tot = wsum(tot);
-    hm = wsum(hm);
+    hj = wave_sum(hj);
+    tot = wave_sum(tot);
+    hm = wave_sum(hm);
+    // the recorded NCC: that of the float32 master at the best orientation (the rule of the
+    // Gauss-Newton passes)
+    if constexpr (MODE == REF_TILES) {
+        f = make_float4(0.f, 0.f, 0.f, 0.f);
+        for (int w = 0; w < W; ++w) {
+            const float4 x = ((const float4*)sh.part[w])[1];
+            f = make_float4(f.x + x.x, f.y + x.y, f.z + x.z, f.w + x.w);
+        }
+    } else {
+        f = sh.acc[0][lane];
+        f = make_float4(wave_sum(f.x), wave_sum(f.y), wave_sum(f.z), wave_sum(f.w));
+    }
+    float ncc_best = -2.f;
+    {
+        const float n = fmaxf(f.x, 1.f);
+        const float mean = f.y / n;
+        const float var_n = f.z - n * mean * mean;
+        if (var_n > 1e-12f) ncc_best = f.w * (1.f / sqrtf(var_n));
+    }
     if (lane == 0) {
         const float nn = fmaxf(tot, 1.f);
         const float h_joint = logf(nn) + hj / nn;
         const float h_marg = 2.f * logf(nn) + hm / nn;
         const float nmi = h_marg > 1e-12f ? 2.f * (h_marg - h_joint) / h_marg : 0.f;
         float* r = records + (size_t)(out0 + b) * 8;
-        r[0] = qbest.x;
-        r[1] = qbest.y;
-        r[2] = qbest.z;
-        r[3] = qbest.w;
+        r[0] = sh.gn.qbest.x;
+        r[1] = sh.gn.qbest.y;
+        r[2] = sh.gn.qbest.z;
+        r[3] = sh.gn.qbest.w;
         r[4] = ncc_best;
         r[5] = nmi;
-        r[6] = last_step;
+        r[6] = sh.gn.last_step;
         r[7] = a.stamp;
     }
 }
 
-// One block per item. With `order` (zb_refine_order's permutation), block i refines item
-// order[xcd_block(i)]: the blocks of one XCD take a contiguous run of items sorted by the master
-// region they look up, so that their gathers share that XCD's L2. Without it, block i refines
-// item i.
-template <int MAXP, bool LIST>
-__global__ void __launch_bounds__(64) k_refine(RefArg a, const float* __restrict__ ms, const uint2* __restrict__ mgh, const float* __restrict__ pats,
-                                               const float4* __restrict__ items, const float* __restrict__ seeds, int n_items,
-                                               const int* __restrict__ order, float* __restrict__ records) {
-    extern __shared__ unsigned lds[];
-    unsigned* hist = lds;                                               // [nmi_bins][nmi_bins]
-    unsigned short* list = LIST ? (unsigned short*)(lds + a.nmi_bins * a.nmi_bins) : nullptr;  // the masked pixels
-    const int b = order ? order[xcd_block(blockIdx.x, gridDim.x)] : (int)blockIdx.x;
-    const int lane = threadIdx.x;
-    for (int i = lane; i < a.nmi_bins * a.nmi_bins; i += 64) hist[i] = 0u;
-    int n_px = a.h * a.w;
-    if constexpr (LIST) n_px = build_list(a, list, lane);
-    else __syncthreads();
-    refine_item<MAXP, LIST>(a, ms, mgh, pats, items, seeds, a.seed_stride, records, a.out0, hist, list, n_px, b, lane);
-}
-
 // Several phases' refinements of one batch in one launch. The n_phases x n_items work items are
-// taken phase-major (item k of phase p is p * n_items + k, in that phase's order).
+// taken phase-major (item k of phase p is p * n_items + k, in that phase's order; zb_refine_order's
+// permutation sorts the items by the master region they look up).
 // k_refine_grid: one block per work item, block i taking work item xcd_block(i), so that each XCD
-// takes a contiguous run of the sequence; the hardware deals blocks to CUs as others finish.
+// takes a contiguous run of the sequence (its items' gathers share that XCD's L2); the hardware
+// deals blocks to CUs as others finish.
 // k_refine_queue: a persistent grid (as many blocks as stay resident) pulling work items from
 // device-side queues: the sequence cut into kQueues contiguous runs, one per XCD, each with its
 // own counter; a block first drains its own XCD's run (block id mod 8, the round-robin dealing
 // xcd_block assumes), then the other runs in turn, and leaves when all are empty, so that every
-// block reaches that exit. Each block builds the masked-pixel list once for all its items.
-// The phases' array pointers are separate restrict kernel arguments (so that the compiler keeps
-// k_refine's register budget: without the no-alias guarantee it holds more values live); their
-// sides, seed strides and orders come as one more argument to the grid form, and for the queue
-// form sit in a table in the work buffer after the queue counters, written with them by
-// k_queue_setup on the same stream before the launch.
+// block reaches that exit. Each block builds the list of masked pixels once for all its items.
+// The phases' array pointers are separate restrict kernel arguments (so that the compiler knows
+// them not to alias the records); their sides, seed strides and orders come as one more argument
+// to the grid form, and for the queue form sit in a table in the work buffer after the queue
+// counters, written with them by k_queue_setup on the same stream before the launch.
 constexpr int kMaxRefinePhases = 4;
 constexpr int kQueues = 8;
 constexpr int kQueueStride = 16;
@@ -464,16 +713,16 @@ __device__ __forceinline__ T pick(int p, T x0, T x1, T x2, T x3) {
 }
 
 // Work item w of the sequence: phase p, item b (in that phase's order); then the item refined.
-template <int MAXP, bool LIST>
+template <int W, int MODE>
 __device__ __forceinline__ void refine_work(const RefArg& a, RefPhase e, int p, int i, ZB_PHASE_ARGS(0), ZB_PHASE_ARGS(1), ZB_PHASE_ARGS(2),
                                             ZB_PHASE_ARGS(3), const float* __restrict__ pats, const float4* __restrict__ items, unsigned* hist,
-                                            const unsigned short* list, int n_px, int lane) {
+                                            const unsigned short* list, int n_px, Shared<W>& sh, int wave, int lane) {
     const int* order = e.order;
     const int b = order ? __builtin_amdgcn_readfirstlane(order[i]) : i;
     RefArg ap = a;
     ap.side = __builtin_amdgcn_readfirstlane(e.side);
-    refine_item<MAXP, LIST>(ap, pick(p, ms0, ms1, ms2, ms3), pick(p, mgh0, mgh1, mgh2, mgh3), pats, items, pick(p, sd0, sd1, sd2, sd3),
-                            __builtin_amdgcn_readfirstlane(e.seed_stride), pick(p, rec0, rec1, rec2, rec3), a.out0, hist, list, n_px, b, lane);
+    refine_item<W, MODE>(ap, pick(p, ms0, ms1, ms2, ms3), pick(p, mgh0, mgh1, mgh2, mgh3), pats, items, pick(p, sd0, sd1, sd2, sd3),
+                         __builtin_amdgcn_readfirstlane(e.seed_stride), pick(p, rec0, rec1, rec2, rec3), a.out0, hist, list, n_px, sh, b, wave, lane);
 }
 
 // Work item w of the sequence: phase p and item i (in that phase's order).
@@ -482,54 +731,60 @@ __device__ __forceinline__ void work_item(unsigned w, int n_items, int& p, int& 
     i = __builtin_amdgcn_readfirstlane((int)(w - (unsigned)p * (unsigned)n_items));
 }
 
-template <int MAXP, bool LIST>
-__global__ void __launch_bounds__(64) k_refine_grid(RefArg a, ZB_PHASE_ARGS(0), ZB_PHASE_ARGS(1), ZB_PHASE_ARGS(2), ZB_PHASE_ARGS(3),
-                                                    const float* __restrict__ pats, const float4* __restrict__ items, int n_items,
-                                                    RefPhases ph) {
+// The list of masked pixels or of tiles; how many (the tiles walked without a list).
+template <int W, int MODE>
+__device__ __forceinline__ int block_list(const RefArg& a, unsigned short* list, Shared<W>& sh, int wave, int lane) {
+    if constexpr (MODE != REF_TILES) return build_list<W, false>(a, list, sh.cnt, wave, lane);
+    if (a.tiles) return build_list<W, true>(a, list, sh.cnt, wave, lane);
+    return ((a.w + 7) >> 3) * ((a.h + 7) >> 3);
+}
+
+template <int W, int MODE>
+__global__ void __launch_bounds__(64 * W) k_refine_grid(RefArg a, ZB_PHASE_ARGS(0), ZB_PHASE_ARGS(1), ZB_PHASE_ARGS(2), ZB_PHASE_ARGS(3),
+                                                        const float* __restrict__ pats, const float4* __restrict__ items, int n_items,
+                                                        RefPhases ph) {
     extern __shared__ unsigned lds[];
+    __shared__ Shared<W> sh;
     unsigned* hist = lds;
-    unsigned short* list = LIST ? (unsigned short*)(lds + a.nmi_bins * a.nmi_bins) : nullptr;
-    const int lane = threadIdx.x;
-    for (int j = lane; j < a.nmi_bins * a.nmi_bins; j += 64) hist[j] = 0u;
-    int n_px = a.h * a.w;
-    if constexpr (LIST) n_px = build_list(a, list, lane);
-    else __syncthreads();
+    unsigned short* list = (unsigned short*)(lds + a.nmi_bins * a.nmi_bins);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    for (int j = threadIdx.x; j < a.nmi_bins * a.nmi_bins; j += 64 * W) hist[j] = 0u;
+    const int n_px = block_list<W, MODE>(a, list, sh, wave, lane);
     int p, i;
     work_item((unsigned)xcd_block(blockIdx.x, gridDim.x), n_items, p, i);
     // the phase's entry picked from the argument (an index into it would place it in memory)
     const RefPhase e = pick(p, ph.p[0], ph.p[1], ph.p[2], ph.p[3]);
-    refine_work<MAXP, LIST>(a, e, p, i, ms0, mgh0, sd0, rec0, ms1, mgh1, sd1, rec1, ms2, mgh2, sd2, rec2, ms3, mgh3, sd3, rec3, pats, items, hist,
-                            list, n_px, lane);
+    refine_work<W, MODE>(a, e, p, i, ms0, mgh0, sd0, rec0, ms1, mgh1, sd1, rec1, ms2, mgh2, sd2, rec2, ms3, mgh3, sd3, rec3, pats, items, hist,
+                         list, n_px, sh, wave, lane);
 }
 
-template <int MAXP, bool LIST>
-__global__ void __launch_bounds__(64) k_refine_queue(RefArg a, ZB_PHASE_ARGS(0), ZB_PHASE_ARGS(1), ZB_PHASE_ARGS(2), ZB_PHASE_ARGS(3),
-                                                     int n_phases, const float* __restrict__ pats, const float4* __restrict__ items, int n_items,
-                                                     unsigned* __restrict__ work) {
+template <int W, int MODE>
+__global__ void __launch_bounds__(64 * W) k_refine_queue(RefArg a, ZB_PHASE_ARGS(0), ZB_PHASE_ARGS(1), ZB_PHASE_ARGS(2), ZB_PHASE_ARGS(3),
+                                                         int n_phases, const float* __restrict__ pats, const float4* __restrict__ items, int n_items,
+                                                         unsigned* __restrict__ work) {
     extern __shared__ unsigned lds[];
+    __shared__ Shared<W> sh;
     unsigned* hist = lds;
-    unsigned short* list = LIST ? (unsigned short*)(lds + a.nmi_bins * a.nmi_bins) : nullptr;
+    unsigned short* list = (unsigned short*)(lds + a.nmi_bins * a.nmi_bins);
     const RefPhase* table = (const RefPhase*)((const char*)work + kTableOffset);
-    const int lane = threadIdx.x;
-    int n_px = a.h * a.w;
-    if constexpr (LIST) n_px = build_list(a, list, lane);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int n_px = block_list<W, MODE>(a, list, sh, wave, lane);
     const unsigned total = (unsigned)n_items * (unsigned)n_phases;  // below 2^31 (the entry point's check)
     for (int r = 0; r < kQueues; ++r) {
         const unsigned x = (blockIdx.x + r) & (kQueues - 1);
         const unsigned lo = (unsigned)((unsigned long long)total * x / kQueues);
         const unsigned len = (unsigned)((unsigned long long)total * (x + 1) / kQueues) - lo;
         for (;;) {
-            unsigned k = 0;
-            if (lane == 0) k = atomicAdd(work + x * kQueueStride, 1u);
-            k = __builtin_amdgcn_readfirstlane(k);
-            if (k >= len) break;
-            for (int j = lane; j < a.nmi_bins * a.nmi_bins; j += 64) hist[j] = 0u;
+            __syncthreads();  // every wave done with the last item's histogram and count
+            if (threadIdx.x == 0) sh.cnt[0] = (int)atomicAdd(work + x * kQueueStride, 1u);
+            for (int j = threadIdx.x; j < a.nmi_bins * a.nmi_bins; j += 64 * W) hist[j] = 0u;
             __syncthreads();
+            const unsigned k = (unsigned)__builtin_amdgcn_readfirstlane(sh.cnt[0]);
+            if (k >= len) break;
             int p, i;
             work_item(lo + k, n_items, p, i);
-            refine_work<MAXP, LIST>(a, table[p], p, i, ms0, mgh0, sd0, rec0, ms1, mgh1, sd1, rec1, ms2, mgh2, sd2, rec2, ms3, mgh3, sd3, rec3, pats,
-                                    items, hist, list, n_px, lane);
-            __syncthreads();  // every lane done with the histogram before the next item clears it
+            refine_work<W, MODE>(a, table[p], p, i, ms0, mgh0, sd0, rec0, ms1, mgh1, sd1, rec1, ms2, mgh2, sd2, rec2, ms3, mgh3, sd3, rec3, pats,
+                                 items, hist, list, n_px, sh, wave, lane);
         }
     }
 }
@@ -612,7 +867,8 @@ __global__ void __launch_bounds__(1024) k_order(RefArg a, const float4* __restri
 // rotation_only zeroes the shift's sums, as sums_reduce does for orientation refinement.
 constexpr int kSums = 43;
 
-// skip (or NULL): items whose entry is not 0 are left out (their sums untouched).
+// skip (or NULL): items whose entry is not 0 are left out (their sums untouched). LIST: the masked
+// pixels as a list in LDS; else the whole frame walked with the mask tested a pixel.
 template <bool LIST>
 __global__ void __launch_bounds__(64) k_sums6(RefArg a, const float4* __restrict__ mg, const float* __restrict__ pats, const float* __restrict__ poses,
                                               int rotation_only, const int* __restrict__ skip, float* __restrict__ out) {
@@ -622,8 +878,7 @@ __global__ void __launch_bounds__(64) k_sums6(RefArg a, const float4* __restrict
     if (skip && skip[b] != 0) return;
     const int lane = threadIdx.x;
     int n_px = a.h * a.w;
-    if constexpr (LIST) n_px = build_list(a, list, lane);
-    const unsigned short* lst = LIST ? list : nullptr;
+    if constexpr (LIST) n_px = build_list<1, false>(a, list, nullptr, 0, lane);
     const float inv_w = 1.f / (float)a.w;
     const float* ps = poses + (size_t)b * 8;
     const float3 t = make_float3(ps[0], ps[1], ps[2]);
@@ -634,10 +889,9 @@ __global__ void __launch_bounds__(64) k_sums6(RefArg a, const float4* __restrict
 #pragma unroll
     for (int i = 0; i < kSums; ++i) s[i] = 0.f;
     for (int k = lane; k < n_px; k += 64) {
-        bool ok;
-        const int pix = pass_pixel<LIST>(a, lst, n_px, k, ok);
-        if (!ok) continue;
+        const int pix = LIST ? (int)list[k] : k;
         const int row = LIST ? (int)(((float)pix + 0.5f) * inv_w) : pix / a.w;
+        if (!LIST && !under_mask(a, row, pix - row * a.w)) continue;
         const float fr = (float)row, fc = (float)(pix - row * a.w);
         const float3 u = make_float3(a.c0[0] * fr + a.c1[0] * fc + t.x, a.c0[1] * fr + a.c1[1] * fc + t.y, a.c0[2] * fr + a.c1[2] * fc + t.z);
         const float dist = sqrtf(dot3(u, u));
@@ -665,7 +919,7 @@ __global__ void __launch_bounds__(64) k_sums6(RefArg a, const float4* __restrict
         }
     }
 #pragma unroll
-    for (int i = 0; i < kSums; ++i) s[i] = wsum(s[i]);
+    for (int i = 0; i < kSums; ++i) s[i] = wave_sum(s[i]);
     // lane i writes sum i (the shift's sums zero for orientation refinement)
 #pragma unroll
     for (int i = 0; i < kSums; ++i) {
@@ -680,7 +934,8 @@ __global__ void __launch_bounds__(64) k_sums6(RefArg a, const float4* __restrict
 
 using namespace zb;
 
-static int ref_frame(const zb_frame* frame, int side, RefArg& a, size_t& lds, const char* who) {
+// The frame's geometry into `a`; returns its masked pixels, or an error (negative).
+static int ref_frame(const zb_frame* frame, int side, RefArg& a, const char* who) {
     for (int i = 0; i < 3; ++i) {
         a.c0[i] = frame->c0[i];
         a.c1[i] = frame->c1[i];
@@ -700,14 +955,11 @@ static int ref_frame(const zb_frame* frame, int side, RefArg& a, size_t& lds, co
             const float dr = (float)r - a.mask[0], dc = (float)c - a.mask[1];
             n_px += (a.mask[2] <= 0.f || dr * dr + dc * dc <= a.mask[2]) ? 1 : 0;
         }
-    // the masked pixels as a 16-bit list in LDS while their indices fit 16 bits and the list
-    // (with the NMI's histogram, at most 32 x 32 words) stays within 60 KB; else the whole frame
-    // is walked with the mask tested per pixel
-    const size_t list_bytes = ((size_t)n_px * 2 + 15) / 16 * 16;
-    a.use_list = ((long)a.h * a.w <= 65536 && list_bytes <= 60 * 1024) ? 1 : 0;
-    lds = a.use_list ? list_bytes : 0;
     return (int)n_px;
 }
+
+// Bytes of a list of n 16-bit entries in LDS.
+static size_t list_bytes(long n) { return ((size_t)n * 2 + 15) / 16 * 16; }
 
 static int32_t sums_run(const float* mgrad, int32_t side, const zb_frame* frame, const float* pats, const float* poses, int32_t n_items,
                         int32_t flags, const int32_t* skip, float* sums, void* stream);
@@ -738,14 +990,16 @@ static int32_t sums_run(const float* mgrad, int32_t side, const zb_frame* frame,
         return ZB_EINVAL;
     }
     RefArg a = {};
-    size_t lds = 0;
-    const int n_px = ref_frame(frame, side, a, lds, "zb_sums");
+    const int n_px = ref_frame(frame, side, a, "zb_sums");
     if (n_px < 0) return n_px;
-    if (a.use_list)
+    // the masked pixels as a 16-bit list in LDS while their indices fit 16 bits and the list stays
+    // within 60 KB; else the whole frame is walked with the mask tested per pixel
+    const size_t lds = list_bytes(n_px);
+    if ((long)a.h * a.w <= 65536 && lds <= 60 * 1024)
         ZB_LAUNCH("k_sums6", k_sums6<true>, dim3(n_items), dim3(64), lds, (hipStream_t)stream, a, (const float4*)mgrad, pats, poses,
                   (flags & ZB_SUMS_ROTATION_ONLY) ? 1 : 0, (const int*)skip, sums);
     else
-        ZB_LAUNCH("k_sums6", k_sums6<false>, dim3(n_items), dim3(64), lds, (hipStream_t)stream, a, (const float4*)mgrad, pats, poses,
+        ZB_LAUNCH("k_sums6", k_sums6<false>, dim3(n_items), dim3(64), 0, (hipStream_t)stream, a, (const float4*)mgrad, pats, poses,
                   (flags & ZB_SUMS_ROTATION_ONLY) ? 1 : 0, (const int*)skip, sums);
     return check_launch("zb_sums");
 }
@@ -761,6 +1015,136 @@ static void ref_opts(RefArg& a, const zb_refine_opts* o, int out0) {
     a.stamp = (float)o->stamp;
 }
 
+// The launch of a refinement: W waves a block, how its pixels are walked, and the LDS for the
+// joint histogram and the list. The list forms' records do not depend on W, so it follows the
+// speed (measured over frames of 40 x 40 to 180 x 180 and 3 to 16 000 items, 5 and 8 iterations):
+//  - while a block's lanes hold all their pixels, as few waves as hold them (2, 3 or 4): every
+//    wave adds hand-overs and barriers (40 x 40, 8 000 items: 582 us with 2 waves, 788 with 4;
+//    one wave an item, the list and the pattern read in each pass: 659), and holding beats reading
+//    the list again (60 x 60, 4 500 items: 514 us against 613);
+//  - above that, more waves where the items are too few to fill the chip or a frame's list leaves
+//    room for few blocks a CU: 8 up to one item a CU or past 256 steps (120 x 120, 8 items: 236 us
+//    against 256 with 4 and 417 with 2; 180 x 180, 1 000 items: 1 208, 1 337 and 2 505), else 4 past
+//    96 steps or up to two items a CU (120 x 120, 1 200 items: 798 us against 848 with 2 and 813
+//    with 8; 80 x 80, 400 items: 238, 294 and 244), else 2 (80 x 80, 4 000 items: 1 233, 1 308 with
+//    4, 1 392 with 8).
+// One wave an item took 725 us for 8 items of 120 x 120, 3 681 us for 40 of 240 x 240 (tiles: 567).
+struct RefLaunch {
+    int mode, waves;
+    size_t lds;
+};
+static RefLaunch ref_launch(RefArg& a, int n_px, long total) {
+    const size_t hist = (size_t)a.nmi_bins * a.nmi_bins * 4;
+    RefLaunch l;
+    if ((long)a.h * a.w <= 65536 && list_bytes(n_px) <= 60 * 1024) {
+        const int steps = (n_px + 63) / 64;
+        if (steps <= 4 * kHeld) {
+            l.mode = REF_HELD;
+            l.waves = std::max((steps + kHeld - 1) / kHeld, 2);
+        } else {
+            l.mode = REF_LIST;
+            l.waves = total <= 256 || steps > 256 ? 8 : total <= 512 || steps > 96 ? 4 : 2;
+        }
+        l.lds = hist + list_bytes(n_px);
+        return l;
+    }
+    const long tiles = (long)((a.h + 7) / 8) * ((a.w + 7) / 8);
+    // the tiles' list within 48 KB of LDS; past that every tile is walked
+    a.tiles = tiles <= 24 * 1024 ? (int)tiles : 0;
+    l.mode = REF_TILES;
+    l.waves = 16;
+    l.lds = hist + list_bytes(a.tiles);
+    return l;
+}
+
+// Blocks of k_refine_queue resident at once on the current device: CUs x blocks per CU, queried
+// once per device, form and LDS size (host queries only, so that a call under stream capture
+// records nothing else).
+static int queue_blocks(const RefLaunch& l) {
+    static std::mutex mu;
+    static std::map<std::tuple<int, int, size_t>, int> known;
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return 0;
+    std::lock_guard<std::mutex> g(mu);
+    const auto key = std::make_tuple(dev, l.mode * 64 + l.waves, l.lds);
+    auto it = known.find(key);
+    if (it != known.end()) return it->second;
+    int cus = 0, per_cu = 0;
+    const void* kern = nullptr;
+#define ZB_KERN(W, MODE) \
+    if (l.waves == W && l.mode == MODE) kern = (const void*)k_refine_queue<W, MODE>
+    ZB_KERN(3, REF_HELD);
+    ZB_KERN(2, REF_HELD);
+    ZB_KERN(2, REF_LIST);
+    ZB_KERN(4, REF_HELD);
+    ZB_KERN(4, REF_LIST);
+    ZB_KERN(8, REF_LIST);
+    ZB_KERN(16, REF_TILES);
+#undef ZB_KERN
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, 64 * l.waves, l.lds) != hipSuccess || per_cu < 1 || cus < 1)
+        return 0;
+    return known[key] = cus * per_cu;
+}
+
+// The refinement of n_phases phases launched (the arguments checked by the callers): block per
+// work item, or with `work` the persistent form.
+static int32_t refine_launch(const zb_refine_phase* phases, int n_phases, const zb_frame* frame, const float* pats, const float* items, int32_t n_items,
+                             const zb_refine_opts* o, int32_t out0, unsigned* queues, hipStream_t st, const char* who) {
+    RefArg a = {};
+    const int n_px = ref_frame(frame, phases[0].side, a, who);
+    if (n_px < 0) return n_px;
+    ref_opts(a, o, out0);
+    const long total = (long)n_items * n_phases;
+    const RefLaunch l = ref_launch(a, n_px, total);
+    // the phases' arrays as kernel arguments (phases past n_phases repeat the last: never read)
+    RefPhases ph = {};
+    const float* ms[kMaxRefinePhases];
+    const uint2* mgh[kMaxRefinePhases];
+    const float* sd[kMaxRefinePhases];
+    float* rec[kMaxRefinePhases];
+    for (int p = 0; p < kMaxRefinePhases; ++p) {
+        const zb_refine_phase& q = phases[std::min(p, n_phases - 1)];
+        ph.p[p] = RefPhase{q.order, q.side, q.seed_stride};
+        ms[p] = q.master;
+        mgh[p] = (const uint2*)q.mgrad_h;
+        sd[p] = q.seeds;
+        rec[p] = q.records;
+    }
+#define ZB_PHASES ms[0], mgh[0], sd[0], rec[0], ms[1], mgh[1], sd[1], rec[1], ms[2], mgh[2], sd[2], rec[2], ms[3], mgh[3], sd[3], rec[3]
+#define ZB_REFINE1(KERNEL, GRID, W, MODE, ...) \
+    if (l.waves == W && l.mode == MODE) ZB_LAUNCH("k_refine", (KERNEL<W, MODE>), dim3(GRID), dim3(64 * W), l.lds, st, a, ZB_PHASES, __VA_ARGS__)
+#define ZB_REFINE(KERNEL, GRID, ...)                         \
+    do {                                                     \
+        ZB_REFINE1(KERNEL, GRID, 2, REF_HELD, __VA_ARGS__);  \
+        ZB_REFINE1(KERNEL, GRID, 2, REF_LIST, __VA_ARGS__);  \
+        ZB_REFINE1(KERNEL, GRID, 3, REF_HELD, __VA_ARGS__);  \
+        ZB_REFINE1(KERNEL, GRID, 4, REF_HELD, __VA_ARGS__);  \
+        ZB_REFINE1(KERNEL, GRID, 4, REF_LIST, __VA_ARGS__);  \
+        ZB_REFINE1(KERNEL, GRID, 8, REF_LIST, __VA_ARGS__);  \
+        ZB_REFINE1(KERNEL, GRID, 16, REF_TILES, __VA_ARGS__); \
+    } while (0)
+    if (queues) {
+        // the queue counters cleared and the phase table written into the work buffer
+        ZB_LAUNCH("k_queue_setup", k_queue_setup, dim3(1), dim3(64), 0, st, ph, n_phases, queues);
+        if (int rc = check_launch("zb_refine_phases/setup")) return rc;
+        // as many blocks as stay resident at once (more would only wait for the queues to empty)
+        const int resident = queue_blocks(l);
+        if (resident < 1) {
+            set_error("%s: device or occupancy query failed", who);
+            return ZB_ELAUNCH;
+        }
+        const int grid = (int)std::min<long>(total, resident);
+        ZB_REFINE(k_refine_queue, grid, n_phases, pats, (const float4*)items, n_items, queues);
+    } else {
+        ZB_REFINE(k_refine_grid, total, pats, (const float4*)items, n_items, ph);
+    }
+#undef ZB_REFINE
+#undef ZB_REFINE1
+#undef ZB_PHASES
+    return check_launch(who);
+}
+
 extern "C" int32_t zb_refine(const float* master, const uint16_t* mgrad_h, int32_t side, const zb_frame* frame, const float* pats, const float* items,
                              const float* seeds, int32_t seed_stride, int32_t n_items, const zb_refine_opts* o, float* records, int32_t out0,
                              void* stream) {
@@ -774,46 +1158,8 @@ extern "C" int32_t zb_refine(const float* master, const uint16_t* mgrad_h, int32
         set_error("zb_refine: null pointer");
         return ZB_EINVAL;
     }
-    RefArg a = {};
-    size_t list_bytes = 0;
-    // the masked pixels (the list each block builds) and the LDS they take
-    const int n_px = ref_frame(frame, side, a, list_bytes, "zb_refine");
-    if (n_px < 0) return n_px;
-    ref_opts(a, o, out0);
-    a.seed_stride = seed_stride;
-    // the joint histogram, then the list (the histogram's size keeps the list 4-byte aligned)
-    const size_t lds = (size_t)o->nmi_bins * o->nmi_bins * 4 + list_bytes;
-    if (a.use_list && n_px <= 64 * 48)
-        ZB_LAUNCH("k_refine", (k_refine<48, true>), dim3(n_items), dim3(64), lds, (hipStream_t)stream, a, master, (const uint2*)mgrad_h, pats,
-                  (const float4*)items, seeds, n_items, (const int*)o->order, records);
-    else if (a.use_list)
-        ZB_LAUNCH("k_refine", (k_refine<0, true>), dim3(n_items), dim3(64), lds, (hipStream_t)stream, a, master, (const uint2*)mgrad_h, pats,
-                  (const float4*)items, seeds, n_items, (const int*)o->order, records);
-    else
-        ZB_LAUNCH("k_refine", (k_refine<0, false>), dim3(n_items), dim3(64), lds, (hipStream_t)stream, a, master, (const uint2*)mgrad_h, pats,
-                  (const float4*)items, seeds, n_items, (const int*)o->order, records);
-    return check_launch("zb_refine");
-}
-
-// Blocks of k_refine_queue (form `kind`, `lds` bytes of LDS) resident at once on the current
-// device: CUs x blocks per CU, queried once per device, form and LDS size (host queries only, so
-// that a call under stream capture records nothing else).
-static int queue_blocks(int kind, size_t lds) {
-    static std::mutex mu;
-    static std::map<std::tuple<int, int, size_t>, int> known;
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return 0;
-    std::lock_guard<std::mutex> g(mu);
-    const auto key = std::make_tuple(dev, kind, lds);
-    auto it = known.find(key);
-    if (it != known.end()) return it->second;
-    int cus = 0, per_cu = 0;
-    const void* kern = kind == 0 ? (const void*)k_refine_queue<48, true> : kind == 1 ? (const void*)k_refine_queue<0, true>
-                                                                                       : (const void*)k_refine_queue<0, false>;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, 64, lds) != hipSuccess || per_cu < 1 || cus < 1)
-        return 0;
-    return known[key] = cus * per_cu;
+    const zb_refine_phase one = {master, mgrad_h, side, seeds, seed_stride, o->order, records};
+    return refine_launch(&one, 1, frame, pats, items, n_items, o, out0, nullptr, (hipStream_t)stream, "zb_refine");
 }
 
 extern "C" int32_t zb_refine_phases(const zb_refine_phase* phases, int32_t n_phases, const zb_frame* frame, const float* pats, const float* items,
@@ -827,7 +1173,6 @@ extern "C" int32_t zb_refine_phases(const zb_refine_phase* phases, int32_t n_pha
         set_error("zb_refine_phases: null pointer");
         return ZB_EINVAL;
     }
-    RefPhases ph = {};
     for (int p = 0; p < n_phases; ++p) {
         const zb_refine_phase& q = phases[p];
         if (q.side < 2 || q.seed_stride < 4) {
@@ -838,7 +1183,6 @@ extern "C" int32_t zb_refine_phases(const zb_refine_phase* phases, int32_t n_pha
             set_error("zb_refine_phases: phase %d: null pointer", p);
             return ZB_EINVAL;
         }
-        ph.p[p] = RefPhase{q.order, q.side, q.seed_stride};
     }
     if (n_items == 0) return ZB_OK;
     if (!pats || !items || !work) {
@@ -853,64 +1197,8 @@ extern "C" int32_t zb_refine_phases(const zb_refine_phase* phases, int32_t n_pha
         set_error("zb_refine_phases: work not 8-byte aligned");
         return ZB_EINVAL;
     }
-    RefArg a = {};
-    size_t list_bytes = 0;
-    const int n_px = ref_frame(frame, phases[0].side, a, list_bytes, "zb_refine_phases");
-    if (n_px < 0) return n_px;
-    ref_opts(a, o, out0);
-    const size_t lds = (size_t)o->nmi_bins * o->nmi_bins * 4 + list_bytes;
-    const long total = (long)n_items * n_phases;
-    unsigned* queues = (unsigned*)work;
-    const hipStream_t st = (hipStream_t)stream;
-    // 0: the list and each lane's master values kept between the NMI's passes; 1: the list, the
-    // values looked up again (fewer registers: with the queue knob at 2); 2: the whole frame
-    const int kind = (a.use_list && n_px <= 64 * 48 && knob(KNOB_REFINE_QUEUE) != 2) ? 0 : a.use_list ? 1 : 2;
-    // phases past n_phases repeat the last one's entry (never read)
-    for (int p = n_phases; p < kMaxRefinePhases; ++p) ph.p[p] = ph.p[n_phases - 1];
-    // the phases' arrays as kernel arguments (phases past n_phases repeat the last: never read)
-    const float* ms[kMaxRefinePhases];
-    const uint2* mgh[kMaxRefinePhases];
-    const float* sd[kMaxRefinePhases];
-    float* rec[kMaxRefinePhases];
-    for (int p = 0; p < kMaxRefinePhases; ++p) {
-        const zb_refine_phase& q = phases[std::min(p, n_phases - 1)];
-        ms[p] = q.master;
-        mgh[p] = (const uint2*)q.mgrad_h;
-        sd[p] = q.seeds;
-        rec[p] = q.records;
-    }
-#define ZB_PHASES ms[0], mgh[0], sd[0], rec[0], ms[1], mgh[1], sd[1], rec[1], ms[2], mgh[2], sd[2], rec[2], ms[3], mgh[3], sd[3], rec[3]
-    if (knob(KNOB_REFINE_QUEUE)) {
-        // the queue counters cleared and the phase table written into the work buffer
-        ZB_LAUNCH("k_queue_setup", k_queue_setup, dim3(1), dim3(64), 0, st, ph, n_phases, queues);
-        if (int rc = check_launch("zb_refine_phases/setup")) return rc;
-        // as many blocks as stay resident at once (more would only wait for the queues to empty)
-        const int resident = queue_blocks(kind, lds);
-        if (resident < 1) {
-            set_error("zb_refine_phases: device or occupancy query failed");
-            return ZB_ELAUNCH;
-        }
-        const int grid = (int)std::min<long>(total, resident);
-        if (kind == 0)
-            ZB_LAUNCH("k_refine", (k_refine_queue<48, true>), dim3(grid), dim3(64), lds, st, a, ZB_PHASES, n_phases, pats, (const float4*)items,
-                      n_items, queues);
-        else if (kind == 1)
-            ZB_LAUNCH("k_refine", (k_refine_queue<0, true>), dim3(grid), dim3(64), lds, st, a, ZB_PHASES, n_phases, pats, (const float4*)items,
-                      n_items, queues);
-        else
-            ZB_LAUNCH("k_refine", (k_refine_queue<0, false>), dim3(grid), dim3(64), lds, st, a, ZB_PHASES, n_phases, pats, (const float4*)items,
-                      n_items, queues);
-    } else {
-        if (kind == 0)
-            ZB_LAUNCH("k_refine", (k_refine_grid<48, true>), dim3(total), dim3(64), lds, st, a, ZB_PHASES, pats, (const float4*)items, n_items, ph);
-        else if (kind == 1)
-            ZB_LAUNCH("k_refine", (k_refine_grid<0, true>), dim3(total), dim3(64), lds, st, a, ZB_PHASES, pats, (const float4*)items, n_items, ph);
-        else
-            ZB_LAUNCH("k_refine", (k_refine_grid<0, false>), dim3(total), dim3(64), lds, st, a, ZB_PHASES, pats, (const float4*)items, n_items,
-                      ph);
-    }
-#undef ZB_PHASES
-    return check_launch("zb_refine_phases");
+    return refine_launch(phases, n_phases, frame, pats, items, n_items, o, out0, knob(KNOB_REFINE_QUEUE) ? (unsigned*)work : nullptr,
+                         (hipStream_t)stream, "zb_refine_phases");
 }
 
 extern "C" int32_t zb_refine_order(const zb_frame* frame, const float* items, const float* seeds, int32_t seed_stride, int32_t n_items,
