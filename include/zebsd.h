@@ -308,7 +308,7 @@ int32_t zb_fit6_accept(const float* trial, const float* trial_sums, int32_t n, d
                        double* lambda, int32_t* state, void* stream);
 
 /* The same fit from each item's local model instead of its sums, so that the gradient can come
- * from elsewhere (zebsdsolve_amd/fit.py drives it with the gradient of its autograd function):
+ * from elsewhere (such as zebsdsolve_amd/fit.py's autograd function):
  * local [n][29] f64 = (NCC, ok (1.0 or 0.0), g[6], the Gauss-Newton matrix's upper triangle row
  * by row [21]) over the six directions of zb_sums. zb_local6 writes it from the sums
  * (planefit.zig:177-201 localOf; ok 0 and the rest 0 where the master is flat under the mask);
@@ -322,6 +322,18 @@ int32_t zb_fit6_step(const float* poses, const double* local, const double* lamb
                      float* trial, double* cur, int32_t* state, void* stream);
 int32_t zb_fit6_keep(const float* trial, const double* trial_local, int32_t n, double tol, const double* cur, float* poses, double* local,
                      double* lambda, int32_t* state, void* stream);
+
+/* The whole fit of n poses ([n][8] f32 = (t, pattern index, q), 16-byte aligned, moved in place): the
+ * local model at the poses, then iters times zb_fit6_step, the model at the trials of the items still
+ * moving and zb_fit6_keep, two launches a turn, the items in the order zb_refine_order gives them.
+ * The models are taken at the poses with q brought to unit length in 64 bits. Lambda starts at
+ * lambda0; unknowns 3 is the rotation alone; ncc [n] f64 (0 where flat) and scored (poses scored, added
+ * to what is there) may be NULL; state [n] as zb_fit6_step's. work: zb_fit6_workspace(n) bytes,
+ * 256-byte aligned. */
+int64_t zb_fit6_workspace(int32_t n);
+int32_t zb_fit6(const float* mgrad, int32_t side, const zb_frame* frame, const float* pats, float* poses, int32_t n, int32_t unknowns,
+                int32_t iters, double lambda0, double max_rot, double max_shift, double tol, void* work, int64_t work_bytes, double* ncc,
+                int64_t* scored, int32_t* state, void* stream);
 
 /* The pattern filters before the path. background: [h][w] f32 subtracted from every pattern
  * (the static background, e.g. the mean of patterns over the map), or NULL; dynamic: 0 none,

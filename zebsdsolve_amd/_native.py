@@ -79,6 +79,9 @@ _SIGS = {
     "zb_sums_active": ([vp, i32, ctypes.POINTER(Frame), vp, vp, i32, i32, vp, vp, vp], i32),
     "zb_fit6_step": ([vp, vp, vp, i32, i32, ctypes.c_double, ctypes.c_double, vp, vp, vp, vp], i32),
     "zb_fit6_keep": ([vp, vp, i32, ctypes.c_double, vp, vp, vp, vp, vp, vp], i32),
+    "zb_fit6_workspace": ([i32], i64),
+    "zb_fit6": ([vp, i32, ctypes.POINTER(Frame), vp, vp, i32, i32, i32, ctypes.c_double, ctypes.c_double, ctypes.c_double, ctypes.c_double,
+                 vp, i64, vp, vp, vp, vp], i32),
     "zb_sums": ([vp, i32, ctypes.POINTER(Frame), vp, vp, i32, i32, vp, vp], i32),
     "zb_project": ([vp, i32, ctypes.POINTER(Frame), vp, i32, vp, vp], i32),
     "zb_master_blur": ([vp, vp, i32, ctypes.c_float, vp], i32),

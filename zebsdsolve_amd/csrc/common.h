@@ -446,6 +446,13 @@ __device__ void fft_dif_fixed(float2* buf, int nlines, const float2* __restrict_
     fft_dif_stages<NT, LOG2N, LOG2N>(buf, nlines, tw, tid);
 }
 
+// zb_sums with the items taken in `order` (or NULL) and, unit, each pose's quaternion made a unit one;
+// zb_refine_order of items item_stride float4s apart (refine.hip).
+int32_t sums_run(const float* mgrad, int32_t side, const zb_frame* frame, const float* pats, const float* poses, int32_t n_items, int32_t flags,
+                 const int32_t* skip, const int32_t* order, int unit, float* sums, void* stream);
+int32_t order_run(const zb_frame* frame, const float* items, int item_stride, const float* seeds, int32_t seed_stride, int32_t n_items,
+                  int32_t* order, void* stream);
+
 __device__ __forceinline__ float warp_sum(float v) {
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
     return v;

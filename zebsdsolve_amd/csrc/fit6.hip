@@ -22,13 +22,16 @@ __device__ bool local6(const float* s, double& ncc, double* g, double* H) {
     const double inv = 1.0 / sqrt(var_n);
     ncc = (double)s[3] * inv;
     double sd[6], au[6];
+#pragma unroll
     for (int i = 0; i < 6; ++i) {
         sd[i] = (double)s[4 + i];
         au[i] = ((double)s[10 + i] - mean * sd[i]) * inv;
         g[i] = ((double)s[16 + i] - ncc * au[i]) * inv;
     }
     int o = 22;
+#pragma unroll
     for (int i = 0; i < 6; ++i)
+#pragma unroll
         for (int j = i; j < 6; ++j) {
             const double v = ((double)s[o] - sd[i] * sd[j] / n - au[i] * au[j]) * inv * inv;
             H[i * 6 + j] = v;
@@ -38,46 +41,71 @@ __device__ bool local6(const float* s, double& ncc, double* g, double* H) {
     return true;
 }
 
-// x = A^-1 b for the last k of the six unknowns, A damped by lambda; false on a zero pivot
-__device__ bool damped_solve(const double* H, const double* g, int k, double lambda, double* x) {
-    const int o = 6 - k;
-    double A[36], b[6];
+// x = A^-1 b for the last K of the six unknowns, A damped by lambda; false on a zero pivot. Every
+// index is a constant (a pivot's row changes place by value): a matrix in scratch memory took
+// k_fit6_step 54 us whatever the items' count.
+template <int K>
+__device__ __forceinline__ bool damped_solve(const double* H, const double* g, double lambda, double* x) {
+    constexpr int o = 6 - K;
+    double A[K][K], b[K];
     double tr = 0.0;
-    for (int i = 0; i < k; ++i) {
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
         b[i] = g[o + i];
-        for (int j = 0; j < k; ++j) A[i * 6 + j] = H[(o + i) * 6 + o + j];
-        tr += A[i * 6 + i];
+#pragma unroll
+        for (int j = 0; j < K; ++j) A[i][j] = H[(o + i) * 6 + o + j];
+        tr += A[i][i];
     }
-    for (int i = 0; i < k; ++i) A[i * 6 + i] = A[i * 6 + i] * (1.0 + lambda) + 1e-9 * tr + 1e-30;
-    for (int c = 0; c < k; ++c) {
+#pragma unroll
+    for (int i = 0; i < K; ++i) A[i][i] = A[i][i] * (1.0 + lambda) + 1e-9 * tr + 1e-30;
+    bool ok = true;
+#pragma unroll
+    for (int c = 0; c < K; ++c) {
         int piv = c;
-        for (int r = c + 1; r < k; ++r)
-            if (fabs(A[r * 6 + c]) > fabs(A[piv * 6 + c])) piv = r;
-        if (fabs(A[piv * 6 + c]) < 1e-300) return false;
-        if (piv != c) {
-            for (int q = 0; q < k; ++q) {
-                const double t = A[c * 6 + q];
-                A[c * 6 + q] = A[piv * 6 + q];
-                A[piv * 6 + q] = t;
+        double top = fabs(A[c][c]);
+#pragma unroll
+        for (int r = c + 1; r < K; ++r)
+            if (fabs(A[r][c]) > top) {
+                top = fabs(A[r][c]);
+                piv = r;
+            }
+        if (top < 1e-300) ok = false;
+#pragma unroll
+        for (int r = c + 1; r < K; ++r) {
+            const bool here = piv == r;
+#pragma unroll
+            for (int q = 0; q < K; ++q) {
+                const double t = A[c][q];
+                A[c][q] = here ? A[r][q] : t;
+                A[r][q] = here ? t : A[r][q];
             }
             const double t = b[c];
-            b[c] = b[piv];
-            b[piv] = t;
+            b[c] = here ? b[r] : t;
+            b[r] = here ? t : b[r];
         }
-        for (int r = c + 1; r < k; ++r) {
-            const double f = A[r * 6 + c] / A[c * 6 + c];
+#pragma unroll
+        for (int r = c + 1; r < K; ++r) {
+            const double f = A[r][c] / A[c][c];
             if (f == 0.0) continue;
-            for (int q = c; q < k; ++q) A[r * 6 + q] -= f * A[c * 6 + q];
+#pragma unroll
+            for (int q = c; q < K; ++q) A[r][q] -= f * A[c][q];
             b[r] -= f * b[c];
         }
     }
+#pragma unroll
     for (int i = 0; i < 6; ++i) x[i] = 0.0;
-    for (int r = k - 1; r >= 0; --r) {
+#pragma unroll
+    for (int r = K - 1; r >= 0; --r) {
         double acc = b[r];
-        for (int q = r + 1; q < k; ++q) acc -= A[r * 6 + q] * x[o + q];
-        x[o + r] = acc / A[r * 6 + r];
+#pragma unroll
+        for (int q = r + 1; q < K; ++q) acc -= A[r][q] * x[o + q];
+        x[o + r] = acc / A[r][r];
     }
-    return true;
+    return ok;
+}
+
+__device__ __forceinline__ bool damped_solve(const double* H, const double* g, int k, double lambda, double* x) {
+    return k == 6 ? damped_solve<6>(H, g, lambda, x) : damped_solve<3>(H, g, lambda, x);
 }
 
 struct Fit6Arg {
@@ -85,25 +113,11 @@ struct Fit6Arg {
     double max_rot, max_shift, tol;
 };
 
-// state: 0 fitting, 1 converged (its last step below tol), 2 flat (no NCC to fit)
-__global__ void __launch_bounds__(256) k_fit6_propose(const float* __restrict__ poses, const float* __restrict__ sums,
-                                                      const double* __restrict__ lambda, Fit6Arg a, float* __restrict__ trial,
-                                                      double* __restrict__ cur, int* __restrict__ state) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= a.n) return;
-    const float* p = poses + (size_t)i * 8;
-    float* t = trial + (size_t)i * 8;
-    double ncc, g[6], H[36], x[6];
-    const bool ok = local6(sums + (size_t)i * kSums, ncc, g, H);
-    if (!ok || state[i] == 2) {
-        state[i] = 2;
-        for (int k = 0; k < 8; ++k) t[k] = p[k];
-        cur[2 * i] = 0.0;
-        cur[2 * i + 1] = 0.0;
-        return;
-    }
+// the damped step of one item from its model, limited and applied: trial pose, cur = (NCC, step)
+__device__ void fit6_move(const float* p, double ncc, const double* g, const double* H, double lambda, const Fit6Arg& a, float* t, double* cur) {
+    double x[6];
     // the Newton step on the model NCC + g . x - x . H x / 2
-    if (!damped_solve(H, g, a.unknowns, lambda[i], x))
+    if (!damped_solve(H, g, a.unknowns, lambda, x))
         for (int k = 0; k < 6; ++k) x[k] = 0.0;
     // at most max_shift pixels and max_rot radians a step
     const double sh = sqrt(x[0] * x[0] + x[1] * x[1] + x[2] * x[2]);
@@ -134,8 +148,28 @@ __global__ void __launch_bounds__(256) k_fit6_propose(const float* __restrict__ 
     t[5] = (float)(nx * sg);
     t[6] = (float)(ny * sg);
     t[7] = (float)(nz * sg);
-    cur[2 * i] = ncc;
-    cur[2 * i + 1] = sqrt(sh * ks * sh * ks + th2);
+    cur[0] = ncc;
+    cur[1] = sqrt(sh * ks * sh * ks + th2);
+}
+
+// state: 0 fitting, 1 converged (its last step below tol), 2 flat (no NCC to fit)
+__global__ void __launch_bounds__(256) k_fit6_propose(const float* __restrict__ poses, const float* __restrict__ sums,
+                                                      const double* __restrict__ lambda, Fit6Arg a, float* __restrict__ trial,
+                                                      double* __restrict__ cur, int* __restrict__ state) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= a.n) return;
+    const float* p = poses + (size_t)i * 8;
+    float* t = trial + (size_t)i * 8;
+    double ncc, g[6], H[36];
+    const bool ok = local6(sums + (size_t)i * kSums, ncc, g, H);
+    if (!ok || state[i] == 2) {
+        state[i] = 2;
+        for (int k = 0; k < 8; ++k) t[k] = p[k];
+        cur[2 * i] = 0.0;
+        cur[2 * i + 1] = 0.0;
+        return;
+    }
+    fit6_move(p, ncc, g, H, lambda[i], a, t, cur + 2 * i);
 }
 
 __global__ void __launch_bounds__(256) k_fit6_accept(const float* __restrict__ trial, const float* __restrict__ tsums, Fit6Arg a,
@@ -188,42 +222,6 @@ __global__ void __launch_bounds__(256) k_local6(const float* __restrict__ sums, 
         for (int b = a; b < 6; ++b) l[o++] = ok ? H[a * 6 + b] : 0.0;
 }
 
-// the damped step of one item from its model, limited and applied: trial pose, cur = (NCC, step)
-__device__ void fit6_move(const float* p, double ncc, const double* g, const double* H, double lambda, const Fit6Arg& a, float* t, double* cur) {
-    double x[6];
-    if (!damped_solve(H, g, a.unknowns, lambda, x))
-        for (int k = 0; k < 6; ++k) x[k] = 0.0;
-    const double sh = sqrt(x[0] * x[0] + x[1] * x[1] + x[2] * x[2]);
-    const double th = sqrt(x[3] * x[3] + x[4] * x[4] + x[5] * x[5]);
-    const double ks = sh > a.max_shift ? a.max_shift / sh : 1.0;
-    const double kr = th > a.max_rot ? a.max_rot / th : 1.0;
-    for (int k = 0; k < 3; ++k) {
-        x[k] *= ks;
-        x[3 + k] *= kr;
-    }
-    const double th2 = x[3] * x[3] + x[4] * x[4] + x[5] * x[5];
-    const double h = sqrt(th2);
-    const double s = h < 1e-6 ? 0.5 - th2 / 48.0 : sin(0.5 * h) / h;
-    const double ew = cos(0.5 * h), ex = s * x[3], ey = s * x[4], ez = s * x[5];
-    const double qw = p[4], qx = p[5], qy = p[6], qz = p[7];
-    double nw = ew * qw - ex * qx - ey * qy - ez * qz;
-    double nx = ew * qx + ex * qw + ey * qz - ez * qy;
-    double ny = ew * qy - ex * qz + ey * qw + ez * qx;
-    double nz = ew * qz + ex * qy - ey * qx + ez * qw;
-    const double nn = sqrt(nw * nw + nx * nx + ny * ny + nz * nz);
-    const double sg = (nw < 0.0 ? -1.0 : 1.0) / (nn > 0.0 ? nn : 1.0);
-    t[0] = (float)((double)p[0] + x[0]);
-    t[1] = (float)((double)p[1] + x[1]);
-    t[2] = (float)((double)p[2] + x[2]);
-    t[3] = p[3];
-    t[4] = (float)(nw * sg);
-    t[5] = (float)(nx * sg);
-    t[6] = (float)(ny * sg);
-    t[7] = (float)(nz * sg);
-    cur[0] = ncc;
-    cur[1] = sqrt(sh * ks * sh * ks + th2);
-}
-
 __global__ void __launch_bounds__(256) k_fit6_step(const float* __restrict__ poses, const double* __restrict__ local,
                                                    const double* __restrict__ lambda, Fit6Arg a, float* __restrict__ trial,
                                                    double* __restrict__ cur, int* __restrict__ state) {
@@ -261,6 +259,75 @@ __global__ void __launch_bounds__(256) k_fit6_keep(const float* __restrict__ tri
         lambda[i] = fmin(lambda[i] * 10.0, 1e9);
     }
     state[i] = cur[2 * i + 1] < a.tol ? 1 : 0;
+}
+
+// The whole of one turn of the fit for each item, a thread an item: the sums at its trial decide
+// whether it is kept (k_local6, k_fit6_keep), then the next trial (k_fit6_step). first: the sums are
+// the start's and there is nothing to keep; last: no next trial. Blocks of one wave: the items are
+// few and every thread's work is a chain of divisions.
+// What bounded the fit was some eighty small launches a turn around k_sums6 (the poses moved, the
+// autograd pass and its copies as tensor operations): 4 000 poses of an 80 x 80 map, 20 turns:
+// 18.15 ms, 7.4 of them in k_sums6; with two launches a turn and the items ordered 5.04 ms.
+struct Fit6Turn {
+    int first, last;
+    double lambda0;
+    float *poses, *trial;
+    double *local, *lambda, *cur, *ncc;
+    int* state;
+    unsigned long long* scored;
+};
+
+__global__ void __launch_bounds__(64) k_fit6_turn(const float* __restrict__ sums, Fit6Arg a, Fit6Turn w) {
+    const int i = blockIdx.x * 64 + threadIdx.x;
+    if (i >= a.n) return;
+    double* kept = w.local + (size_t)i * kLocal;
+    float* p = w.poses + (size_t)i * 8;
+    float* t = w.trial + (size_t)i * 8;
+    int state = w.first ? 0 : w.state[i];
+    double lambda = w.first ? w.lambda0 : w.lambda[i];
+    double ncc = 0.0, g[6], H[36];
+    bool ok = false, fresh = false;  // fresh: ncc, g, H are the kept pose's already
+    if (state == 0) {
+        ok = local6(sums + (size_t)i * kSums, ncc, g, H);
+        fresh = w.first || (ok && ncc > w.cur[2 * i]);
+        if (!w.first) {
+            if (fresh) {
+#pragma unroll
+                for (int k = 0; k < 8; ++k) p[k] = t[k];
+                lambda = fmax(lambda * 0.1, 1e-9);
+            } else {
+                lambda = fmin(lambda * 10.0, 1e9);
+            }
+            state = w.cur[2 * i + 1] < a.tol ? 1 : 0;
+        }
+        if (fresh) {
+            kept[0] = ok ? ncc : 0.0;
+            kept[1] = ok ? 1.0 : 0.0;
+            int o = 8;
+#pragma unroll
+            for (int k = 0; k < 6; ++k) kept[2 + k] = ok ? g[k] : 0.0;
+#pragma unroll
+            for (int r = 0; r < 6; ++r)
+#pragma unroll
+                for (int c = r; c < 6; ++c) kept[o++] = ok ? H[r * 6 + c] : 0.0;
+        }
+    }
+    if (!w.last && state == 0) {
+        if (!fresh) ok = unpack_local(kept, ncc, g, H);
+        if (ok) {
+            fit6_move(p, ncc, g, H, lambda, a, t, w.cur + 2 * i);
+        } else {
+            state = 2;
+            w.cur[2 * i] = 0.0;
+            w.cur[2 * i + 1] = 0.0;
+        }
+    }
+    w.state[i] = state;
+    w.lambda[i] = lambda;
+    if (w.last && w.ncc) w.ncc[i] = kept[1] > 0.5 ? kept[0] : 0.0;
+    // the trials that are scored next
+    const unsigned long long on = __ballot(!w.last && state == 0);
+    if (w.scored && (threadIdx.x & 63) == 0) atomicAdd(w.scored, (unsigned long long)__popcll(on));
 }
 
 }  // namespace zb
@@ -344,4 +411,76 @@ extern "C" int32_t zb_fit6_keep(const float* trial, const double* trial_local, i
     ZB_LAUNCH("k_fit6_keep", k_fit6_keep, dim3((n + 255) / 256), dim3(256), 0, (hipStream_t)stream, trial, trial_local, a, cur, poses, local,
               lambda, (int*)state);
     return check_launch("zb_fit6_keep");
+}
+
+// The parts of zb_fit6's workspace, each 256-byte aligned.
+struct Fit6Work {
+    int64_t order, sums, trial, cur, lambda, local, bytes;
+    explicit Fit6Work(int64_t n) {
+        int64_t at = 0;
+        auto take = [&](int64_t b) {
+            const int64_t o = at;
+            at += (b + 255) / 256 * 256;
+            return o;
+        };
+        order = take(n * 4);
+        sums = take(n * kSums * 4);
+        trial = take(n * 32);
+        cur = take(n * 16);
+        lambda = take(n * 8);
+        local = take(n * kLocal * 8);
+        bytes = at;
+    }
+};
+
+extern "C" int64_t zb_fit6_workspace(int32_t n) {
+    if (n < 0) {
+        set_error("zb_fit6_workspace: n %d", n);
+        return ZB_EINVAL;
+    }
+    return Fit6Work(n).bytes;
+}
+
+extern "C" int32_t zb_fit6(const float* mgrad, int32_t side, const zb_frame* frame, const float* pats, float* poses, int32_t n, int32_t unknowns,
+                           int32_t iters, double lambda0, double max_rot, double max_shift, double tol, void* work, int64_t work_bytes, double* ncc,
+                           int64_t* scored, int32_t* state, void* stream) {
+    Fit6Arg a;
+    if (int rc = fit6_arg(n, unknowns, max_rot, max_shift, tol, a, "zb_fit6")) return rc;
+    if (iters < 0 || !frame || side < 2) {
+        set_error("zb_fit6: bad arguments (iters %d, side %d)", iters, side);
+        return ZB_EINVAL;
+    }
+    if (n == 0) return ZB_OK;
+    if (!mgrad || !pats || !poses || !work || !state || ((uintptr_t)work & 255) != 0 || ((uintptr_t)poses & 15) != 0) {
+        set_error("zb_fit6: null or misaligned pointer");
+        return ZB_EINVAL;
+    }
+    const Fit6Work at(n);
+    if (work_bytes < at.bytes) {
+        set_error("zb_fit6: workspace %lld bytes, need %lld", (long long)work_bytes, (long long)at.bytes);
+        return ZB_ESPACE;
+    }
+    char* base = (char*)work;
+    int32_t* order = (int32_t*)(base + at.order);
+    float* sums = (float*)(base + at.sums);
+    const int flags = unknowns == 3 ? ZB_SUMS_ROTATION_ONLY : 0;
+    Fit6Turn w = {};
+    w.lambda0 = lambda0;
+    w.poses = poses;
+    w.trial = (float*)(base + at.trial);
+    w.cur = (double*)(base + at.cur);
+    w.lambda = (double*)(base + at.lambda);
+    w.local = (double*)(base + at.local);
+    w.ncc = ncc;
+    w.state = (int*)state;
+    w.scored = (unsigned long long*)scored;
+    if (int rc = order_run(frame, poses, 2, poses + 4, 8, n, order, stream)) return rc;
+    for (int it = 0; it <= iters; ++it) {
+        w.first = it == 0;
+        w.last = it == iters;
+        const int rc = sums_run(mgrad, side, frame, pats, it ? w.trial : poses, n, flags, it ? state : nullptr, order, 1, sums, stream);
+        if (rc) return rc;
+        ZB_LAUNCH("k_fit6_turn", k_fit6_turn, dim3((n + 63) / 64), dim3(64), 0, (hipStream_t)stream, (const float*)sums, a, w);
+    }
+    return check_launch("zb_fit6");
 }

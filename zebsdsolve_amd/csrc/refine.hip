@@ -820,8 +820,8 @@ __device__ __forceinline__ int order_cell(const RefArg& a, float4 q, float3 t) {
 // A counting sort of the items by order_cell, one block: counts per cell in LDS, their exclusive
 // prefix, then each item placed at its cell's next slot (the order within a cell is arbitrary;
 // every item's record is the same whichever block computes it).
-__global__ void __launch_bounds__(1024) k_order(RefArg a, const float4* __restrict__ items, const float* __restrict__ seeds, int seed_stride,
-                                                int n_items, int* __restrict__ order) {
+__global__ void __launch_bounds__(1024) k_order(RefArg a, const float4* __restrict__ items, int item_stride, const float* __restrict__ seeds,
+                                                int seed_stride, int n_items, int* __restrict__ order) {
     __shared__ unsigned cnt[kOrderCells];
     __shared__ unsigned part[1024];
     const int tid = threadIdx.x;
@@ -829,7 +829,7 @@ __global__ void __launch_bounds__(1024) k_order(RefArg a, const float4* __restri
     __syncthreads();
     auto cell_of = [&](int b) {
         const float* sd = seeds + (size_t)b * seed_stride;
-        const float4 it = items[b];
+        const float4 it = items[(size_t)b * item_stride];
         return order_cell(a, make_float4(sd[0], sd[1], sd[2], sd[3]), make_float3(it.x, it.y, it.z));
     };
     for (int b = tid; b < n_items; b += 1024) atomicAdd(&cnt[cell_of(b)], 1u);
@@ -868,13 +868,18 @@ __global__ void __launch_bounds__(1024) k_order(RefArg a, const float4* __restri
 constexpr int kSums = 43;
 
 // skip (or NULL): items whose entry is not 0 are left out (their sums untouched). LIST: the masked
-// pixels as a list in LDS; else the whole frame walked with the mask tested a pixel.
+// pixels as a list in LDS; else the whole frame walked with the mask tested a pixel. order (or
+// NULL): block b takes item order[xcd_block(b)] rather than b, so the blocks of one XCD read one
+// region of the field: with 4 000 poses of an 80 x 80 map in flight the field's 8 MB (float4 a texel)
+// pass through every XCD's 4 MB of L2 in any order of the items (6.4 TB/s fetched past L2, the VALU
+// a quarter busy). unit: the quaternion is brought to unit length (in 64 bits) and w >= 0 first.
 template <bool LIST>
 __global__ void __launch_bounds__(64) k_sums6(RefArg a, const float4* __restrict__ mg, const float* __restrict__ pats, const float* __restrict__ poses,
-                                              int rotation_only, const int* __restrict__ skip, float* __restrict__ out) {
+                                              int rotation_only, const int* __restrict__ skip, const int* __restrict__ order, int unit,
+                                              float* __restrict__ out) {
     extern __shared__ unsigned lds[];
     unsigned short* list = (unsigned short*)lds;
-    const int b = blockIdx.x;
+    const int b = order ? __builtin_amdgcn_readfirstlane(order[xcd_block(blockIdx.x, gridDim.x)]) : blockIdx.x;
     if (skip && skip[b] != 0) return;
     const int lane = threadIdx.x;
     int n_px = a.h * a.w;
@@ -883,7 +888,12 @@ __global__ void __launch_bounds__(64) k_sums6(RefArg a, const float4* __restrict
     const float* ps = poses + (size_t)b * 8;
     const float3 t = make_float3(ps[0], ps[1], ps[2]);
     const float* pat = pats + (size_t)(int)ps[3] * a.h * a.w;
-    const float4 q = make_float4(ps[4], ps[5], ps[6], ps[7]);
+    float4 q = make_float4(ps[4], ps[5], ps[6], ps[7]);
+    if (unit) {
+        const double x = q.x, y = q.y, z = q.z, w = q.w;
+        const double len = sqrt(x * x + y * y + z * z + w * w), f = x / len < 0.0 ? -1.0 : 1.0;
+        q = make_float4((float)(f * (x / len)), (float)(f * (y / len)), (float)(f * (z / len)), (float)(f * (w / len)));
+    }
     const float4 qi = make_float4(q.x, -q.y, -q.z, -q.w);
     float s[kSums];
 #pragma unroll
@@ -961,12 +971,9 @@ static int ref_frame(const zb_frame* frame, int side, RefArg& a, const char* who
 // Bytes of a list of n 16-bit entries in LDS.
 static size_t list_bytes(long n) { return ((size_t)n * 2 + 15) / 16 * 16; }
 
-static int32_t sums_run(const float* mgrad, int32_t side, const zb_frame* frame, const float* pats, const float* poses, int32_t n_items,
-                        int32_t flags, const int32_t* skip, float* sums, void* stream);
-
 extern "C" int32_t zb_sums(const float* mgrad, int32_t side, const zb_frame* frame, const float* pats, const float* poses, int32_t n_items,
                            int32_t flags, float* sums, void* stream) {
-    return sums_run(mgrad, side, frame, pats, poses, n_items, flags, nullptr, sums, stream);
+    return zb::sums_run(mgrad, side, frame, pats, poses, n_items, flags, nullptr, nullptr, 0, sums, stream);
 }
 
 extern "C" int32_t zb_sums_active(const float* mgrad, int32_t side, const zb_frame* frame, const float* pats, const float* poses,
@@ -975,11 +982,11 @@ extern "C" int32_t zb_sums_active(const float* mgrad, int32_t side, const zb_fra
         set_error("zb_sums_active: null state");
         return ZB_EINVAL;
     }
-    return sums_run(mgrad, side, frame, pats, poses, n_items, flags, state, sums, stream);
+    return zb::sums_run(mgrad, side, frame, pats, poses, n_items, flags, state, nullptr, 0, sums, stream);
 }
 
-static int32_t sums_run(const float* mgrad, int32_t side, const zb_frame* frame, const float* pats, const float* poses, int32_t n_items,
-                        int32_t flags, const int32_t* skip, float* sums, void* stream) {
+int32_t zb::sums_run(const float* mgrad, int32_t side, const zb_frame* frame, const float* pats, const float* poses, int32_t n_items, int32_t flags,
+                     const int32_t* skip, const int32_t* order, int unit, float* sums, void* stream) {
     if (!frame || side < 2 || n_items < 0 || frame->pat_h < 2 || frame->pat_w < 2 || (flags & ~ZB_SUMS_ROTATION_ONLY)) {
         set_error("zb_sums: bad arguments");
         return ZB_EINVAL;
@@ -997,10 +1004,10 @@ static int32_t sums_run(const float* mgrad, int32_t side, const zb_frame* frame,
     const size_t lds = list_bytes(n_px);
     if ((long)a.h * a.w <= 65536 && lds <= 60 * 1024)
         ZB_LAUNCH("k_sums6", k_sums6<true>, dim3(n_items), dim3(64), lds, (hipStream_t)stream, a, (const float4*)mgrad, pats, poses,
-                  (flags & ZB_SUMS_ROTATION_ONLY) ? 1 : 0, (const int*)skip, sums);
+                  (flags & ZB_SUMS_ROTATION_ONLY) ? 1 : 0, (const int*)skip, (const int*)order, unit, sums);
     else
         ZB_LAUNCH("k_sums6", k_sums6<false>, dim3(n_items), dim3(64), 0, (hipStream_t)stream, a, (const float4*)mgrad, pats, poses,
-                  (flags & ZB_SUMS_ROTATION_ONLY) ? 1 : 0, (const int*)skip, sums);
+                  (flags & ZB_SUMS_ROTATION_ONLY) ? 1 : 0, (const int*)skip, (const int*)order, unit, sums);
     return check_launch("zb_sums");
 }
 
@@ -1212,6 +1219,11 @@ extern "C" int32_t zb_refine_order(const zb_frame* frame, const float* items, co
         set_error("zb_refine_order: null pointer");
         return ZB_EINVAL;
     }
+    return zb::order_run(frame, items, 1, seeds, seed_stride, n_items, order, stream);
+}
+
+int32_t zb::order_run(const zb_frame* frame, const float* items, int item_stride, const float* seeds, int32_t seed_stride, int32_t n_items,
+                      int32_t* order, void* stream) {
     RefArg a = {};
     for (int i = 0; i < 3; ++i) {
         a.c0[i] = frame->c0[i];
@@ -1221,6 +1233,7 @@ extern "C" int32_t zb_refine_order(const zb_frame* frame, const float* items, co
     }
     a.h = frame->pat_h;
     a.w = frame->pat_w;
-    ZB_LAUNCH("k_order", k_order, dim3(1), dim3(1024), 0, (hipStream_t)stream, a, (const float4*)items, seeds, seed_stride, n_items, order);
+    ZB_LAUNCH("k_order", k_order, dim3(1), dim3(1024), 0, (hipStream_t)stream, a, (const float4*)items, item_stride, seeds, seed_stride,
+              n_items, order);
     return check_launch("zb_refine_order");
 }

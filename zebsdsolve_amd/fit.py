@@ -9,8 +9,9 @@ rotation and the pattern centre (the detector position t(PC) of src/geometry.zig
 forward pass is zb_sums (the adjoint of the projection: the derivative of every masked pixel's
 master value along each direction, summed against the pattern) and zb_local6 (NCC, gradient,
 Gauss-Newton matrix) on the device, its backward pass the gradient from the same sums, chained
-through the left Jacobian of exp and dt/dPC. `fit6` takes its Levenberg-Marquardt steps with the
-gradient of a `PoseNcc` backward pass and the matrix of the same forward pass.
+through the left Jacobian of exp and dt/dPC. `fit6` takes its Levenberg-Marquardt steps from the
+same local model on the device (zb_fit6: at delta = 0 the left Jacobian is the identity, and the
+gradient of a `PoseNcc` backward pass is the model's own).
 """
 import numpy as np
 import torch
@@ -243,13 +244,11 @@ def local_with_autograd(field, poses, flags=0, state=None):
 
 def fit6(field, poses0, iters=20, unknowns=6, lambda0=1e-3, max_rot=np.radians(2.0), max_shift=2.0, tol=1e-7, with_ncc=True, counts=None):
     """Each pose fitted to its pattern by Levenberg-Marquardt steps over the six directions (or
-    the rotation alone, unknowns = 3), on the device: per step each item's damped Newton step
-    from its local model (zb_fit6_step, FP64: the gradient from a PoseNcc backward pass, the
-    Gauss-Newton matrix from the same forward pass), the model at the moved poses (PoseNcc
-    again, for the items still moving) deciding which are kept (zb_fit6_keep); an item whose
-    step fell below tol has converged and stays put. Returns (poses [n, 8] float32, NCC [n]
-    float64 (None without with_ncc), state [n]: 0 still moving after `iters` steps, 1
-    converged (the last step below tol), 2 flat), all on the device. `counts` (a dict), if
+    the rotation alone, unknowns = 3), on the device (zb_fit6): per step each item's damped Newton
+    step from its local model in FP64, the model at the moved poses (of the items still moving)
+    deciding which are kept; an item whose step fell below tol has converged and stays put.
+    Returns (poses [n, 8] float32, NCC [n] float64 (None without with_ncc), state [n]: 0 still
+    moving after `iters` steps, 1 converged (the last step below tol), 2 flat), all on the device. `counts` (a dict), if
     given, receives "scored": a device tensor of the poses scored (the start and every trial of
     an item still moving)."""
     from .engine import stream_ptr
@@ -257,24 +256,14 @@ def fit6(field, poses0, iters=20, unknowns=6, lambda0=1e-3, max_rot=np.radians(2
     dev = field.pats.device
     poses = torch.as_tensor(poses0, dtype=torch.float32, device=dev).clone().contiguous()
     n = poses.shape[0]
-    flags = ROTATION_ONLY if unknowns == 3 else 0
-    local = local_with_autograd(field, poses, flags)
-    scored = torch.full((), n, dtype=torch.int64, device=dev)
-    lam = torch.full((n,), float(lambda0), dtype=torch.float64, device=dev)
-    cur = torch.zeros((n, 2), dtype=torch.float64, device=dev)
+    scored = torch.full((), n, dtype=torch.int64, device=dev) if counts is not None else None
+    ncc = torch.empty((n,), dtype=torch.float64, device=dev) if with_ncc else None
     state = torch.zeros((n,), dtype=torch.int32, device=dev)
-    trial = torch.empty_like(poses)
-    st = stream_ptr()
-    for _ in range(iters):
-        nat.check(lib.zb_fit6_step(poses.data_ptr(), local.data_ptr(), lam.data_ptr(), n, unknowns, float(max_rot), float(max_shift),
-                                   trial.data_ptr(), cur.data_ptr(), state.data_ptr(), st), "fit6 step")
-        # only the items still moving are scored (converged ones stay put)
-        tlocal = local_with_autograd(field, trial, flags, state)
-        scored += (state == 0).sum()
-        nat.check(lib.zb_fit6_keep(trial.data_ptr(), tlocal.data_ptr(), n, float(tol), cur.data_ptr(), poses.data_ptr(), local.data_ptr(),
-                                   lam.data_ptr(), state.data_ptr(), st), "fit6 keep")
+    work = torch.empty((int(lib.zb_fit6_workspace(n)),), dtype=torch.uint8, device=dev)
+    nat.check(lib.zb_fit6(field.grad.data_ptr(), field.side, field.frame, field.pats.data_ptr(), poses.data_ptr(), n, int(unknowns), int(iters),
+                          float(lambda0), float(max_rot), float(max_shift), float(tol), work.data_ptr(), work.numel(),
+                          None if ncc is None else ncc.data_ptr(), None if scored is None else scored.data_ptr(), state.data_ptr(),
+                          stream_ptr()), "fit6")
     if counts is not None:
         counts["scored"] = scored
-    if not with_ncc:
-        return poses, None, state
-    return poses, torch.where(local[:, 1] > 0.5, local[:, 0], torch.zeros_like(local[:, 0])), state
+    return poses, ncc, state
