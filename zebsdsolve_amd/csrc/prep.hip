@@ -163,6 +163,7 @@ struct BlurArg {
     float reach;   // box: ceil(4 sigma_coarse), pixels
     float k0, k2;  // box: 1 / (2 sigma_coarse^2), 1 / (2 s^2)
     int hs, ws, hp, wp;
+    int nbx, nby;  // box: cells within reach of one, along the rows and the columns
 };
 
 struct PrepArg {
@@ -188,29 +189,29 @@ __device__ __forceinline__ float2 prep_cell(int j, int n, int s) {
     return make_float2(0.5f * (float)(lo + hi - 1), (float)(hi - lo));
 }
 
-// The Gaussian of the h x w image `img` (LDS, read only), through the scratch `aux` (LDS); the
-// last pass hands each pixel's blurred value to emit(i, value), pixel i on thread i mod 256.
-template <typename Emit>
-__device__ void gauss(const float* img, float* aux, int h, int w, const BlurArg& g, Emit emit) {
+// The Gaussian of the h x w image `img` (rows S apart, read only), through the scratch `aux`; the
+// last pass hands each pixel's blurred value to emit(row, col, value), pixel i on thread i mod NT.
+template <int NT, typename Emit>
+__device__ void gauss(const float* img, float* aux, int h, int w, int S, const BlurArg& g, Emit emit) {
     const int hw = h * w;
     const int tid = threadIdx.x;
     if (!g.box) {
         float* wt = aux + ((hw + 3) & ~3);  // exp(-d^2 k), d <= radius
-        for (int d = tid; d <= g.radius; d += 256) wt[d] = expf(-(float)(d * d) * g.k);
+        for (int d = tid; d <= g.radius; d += NT) wt[d] = expf(-(float)(d * d) * g.k);
         __syncthreads();
-        for (int i = tid; i < hw; i += 256) {
+        for (int i = tid; i < hw; i += NT) {
             const int r = i / w, c = i - (i / w) * w;
             float acc = 0.f, ws = 0.f;
             const int x1 = min(c + g.radius, w - 1);
             for (int x = max(c - g.radius, 0); x <= x1; ++x) {
                 const float q = wt[abs(x - c)];
-                acc += q * img[r * w + x];
+                acc += q * img[r * S + x];
                 ws += q;
             }
             aux[i] = acc / ws;
         }
         __syncthreads();
-        for (int i = tid; i < hw; i += 256) {
+        for (int i = tid; i < hw; i += NT) {
             const int r = i / w, c = i - (i / w) * w;
             float acc = 0.f, ws = 0.f;
             const int y1 = min(r + g.radius, h - 1);
@@ -219,7 +220,7 @@ __device__ void gauss(const float* img, float* aux, int h, int w, const BlurArg&
                 acc += q * aux[y * w + c];
                 ws += q;
             }
-            emit(i, acc / ws);
+            emit(r, c, acc / ws);
         }
         __syncthreads();
         return;
@@ -229,17 +230,17 @@ __device__ void gauss(const float* img, float* aux, int h, int w, const BlurArg&
     float2* c0 = reinterpret_cast<float2*>(aux);
     float2* c1 = c0 + big;
     // pixel sums and counts over the s x s boxes: [hs][ws]
-    for (int t = tid; t < g.hs * g.ws; t += 256) {
+    for (int t = tid; t < g.hs * g.ws; t += NT) {
         const int i = t / g.ws, j = t - (t / g.ws) * g.ws;
         const int r1 = min((i + 1) * s, h), q1 = min((j + 1) * s, w);
         float acc = 0.f;
         for (int r = i * s; r < r1; ++r)
-            for (int q = j * s; q < q1; ++q) acc += img[r * w + q];
+            for (int q = j * s; q < q1; ++q) acc += img[r * S + q];
         c0[t] = make_float2(acc, (float)((r1 - i * s) * (q1 - j * s)));
     }
     __syncthreads();
     // along the rows onto the coarse grid with its margin: [hs][wp]
-    for (int t = tid; t < g.hs * g.wp; t += 256) {
+    for (int t = tid; t < g.hs * g.wp; t += NT) {
         const int line = t / g.wp, tc = t - (t / g.wp) * g.wp;
         const float cc = prep_cell(tc - pad, w, s).x;
         const int j0 = max((int)floorf((cc - g.reach) / (float)s), 0);
@@ -255,7 +256,7 @@ __device__ void gauss(const float* img, float* aux, int h, int w, const BlurArg&
     }
     __syncthreads();
     // along the columns: [hp][wp]
-    for (int t = tid; t < g.hp * g.wp; t += 256) {
+    for (int t = tid; t < g.hp * g.wp; t += NT) {
         const int tr = t / g.wp, col = t - (t / g.wp) * g.wp;
         const float cc = prep_cell(tr - pad, h, s).x;
         const int i0 = max((int)floorf((cc - g.reach) / (float)s), 0);
@@ -271,7 +272,7 @@ __device__ void gauss(const float* img, float* aux, int h, int w, const BlurArg&
     }
     __syncthreads();
     // spread over the pixels of each row from the 2 pad + 1 cells around: [hp][w]
-    for (int t = tid; t < g.hp * w; t += 256) {
+    for (int t = tid; t < g.hp * w; t += NT) {
         const int tr = t / w, x = t - (t / w) * w;
         const int own = x / s;
         float2 acc = make_float2(0.f, 0.f);
@@ -286,7 +287,7 @@ __device__ void gauss(const float* img, float* aux, int h, int w, const BlurArg&
     }
     __syncthreads();
     // and of each column, into the pixels
-    for (int i = tid; i < hw; i += 256) {
+    for (int i = tid; i < hw; i += NT) {
         const int y = i / w, x = i - (i / w) * w;
         const int own = y / s;
         float2 acc = make_float2(0.f, 0.f);
@@ -297,7 +298,7 @@ __device__ void gauss(const float* img, float* aux, int h, int w, const BlurArg&
             const float2 v = c1[(own + q) * w + x];
             acc = make_float2(acc.x + e * v.x, acc.y + e * v.y);
         }
-        emit(i, acc.x / acc.y);
+        emit(y, x, acc.x / acc.y);
     }
     __syncthreads();
 }
@@ -317,6 +318,7 @@ __device__ void clahe_table(unsigned* hist, int B, float voxels, float clip) {
     const float nb = (float)B;
     const float limit = fmaxf(clip * voxels / nb, 1.f);
     float sumc = 0.f;
+#pragma unroll 8
     for (int i = 0; i < B; ++i) sumc += fminf((float)hist[i], limit);
     const float clipped = voxels - sumc;
     const int residual = (int)(clipped - nb * floorf(clipped / nb));
@@ -331,8 +333,8 @@ __device__ void clahe_table(unsigned* hist, int B, float voxels, float clip) {
 }
 
 // The equalized value of pixel (row, col) holding v (prep.wgsl:366-397): the four nearest
-// tiles' tables [T][T][B], each read between its two nearest levels.
-__device__ float clahe_value(float v, int row, int col, int h, int w, int T, int B, const float* cdf) {
+// tiles' tables [T][T] of B levels, `stride` words apart, each read between its two nearest levels.
+__device__ float clahe_value(float v, int row, int col, int h, int w, int T, int B, const float* cdf, int stride) {
     auto mix = [](float x, float y, float t) { return x * (1.f - t) + y * t; };
     v = fminf(fmaxf(v, 0.f), 1.f);
     const float gy = ((float)row + 0.5f) / (float)h * (float)(T - 1);
@@ -344,7 +346,7 @@ __device__ float clahe_value(float v, int row, int col, int h, int w, int T, int
     const int b0 = (int)fminf(fmaxf(floorf(bf), 0.f), (float)(B - 2));
     const float fb = bf - (float)b0;
     auto at = [&](int ty, int tx) {
-        const float* c = cdf + (ty * T + tx) * B;
+        const float* c = cdf + (ty * T + tx) * stride;
         return mix(c[b0], c[b0 + 1], fb);
     };
     return mix(mix(at(y0, x0), at(y0, x1), fx), mix(at(y1, x0), at(y1, x1), fx), fy);
@@ -392,7 +394,7 @@ __device__ void clahe_block(float* img, unsigned* hist, const PrepArg& a, float*
     const float* cdf = reinterpret_cast<const float*>(hist);
     for (int i = tid; i < hw; i += 256) {
         const int row = i / w, col = i - (i / w) * w;
-        img[i] = clahe_value(img[i], row, col, h, w, T, B, cdf);
+        img[i] = clahe_value(img[i], row, col, h, w, T, B, cdf, B);
     }
     __syncthreads();
 }
@@ -454,7 +456,7 @@ __global__ void __launch_bounds__(256) k_clahe_apply(float* __restrict__ img, Cl
     if (tid >= (long)a.n * hw) return;
     const int b = (int)(tid / hw);
     const int pix = (int)(tid - (long)b * hw);
-    img[tid] = clahe_value(img[tid], pix / a.w, pix % a.w, a.h, a.w, a.tiles, a.bins, cdf + (size_t)b * a.tiles * a.tiles * a.bins);
+    img[tid] = clahe_value(img[tid], pix / a.w, pix % a.w, a.h, a.w, a.tiles, a.bins, cdf + (size_t)b * a.tiles * a.tiles * a.bins, a.bins);
 }
 
 // The filter chain and the normalization of one pattern, the block's 256 threads over the
@@ -471,14 +473,17 @@ __device__ void prep_one(const T* __restrict__ src, const float* __restrict__ bg
     __syncthreads();
     if (a.dyn) {
         const int dyn = a.dyn;
-        gauss(img, aux, a.h, a.w, a.dynb, [&](int i, float b) { img[i] = dyn == 1 ? img[i] - b : img[i] / fmaxf(b, 1e-6f); });
+        gauss<256>(img, aux, a.h, a.w, a.w, a.dynb, [&](int r, int c, float b) {
+            float* p = img + r * a.w + c;
+            *p = dyn == 1 ? *p - b : *p / fmaxf(b, 1e-6f);
+        });
     }
     if (a.clahe) clahe_block(img, reinterpret_cast<unsigned*>(aux), a, red);
     if (a.bp) {
         // the coarse Gaussian into the output row (each pixel back on the thread that wrote it)
-        gauss(img, aux, a.h, a.w, a.coarse, [&](int i, float b) { dst[i] = b; });
+        gauss<256>(img, aux, a.h, a.w, a.w, a.coarse, [&](int r, int c, float b) { dst[r * a.w + c] = b; });
         if (a.bp_fine) {
-            gauss(img, aux, a.h, a.w, a.fine, [&](int i, float b) { img[i] = b - dst[i]; });
+            gauss<256>(img, aux, a.h, a.w, a.w, a.fine, [&](int r, int c, float b) { img[r * a.w + c] = b - dst[r * a.w + c]; });
         } else {
             for (int i = tid; i < hw; i += 256) img[i] -= dst[i];
             __syncthreads();
@@ -527,6 +532,522 @@ __global__ void __launch_bounds__(256) k_prep_g(const T* __restrict__ raw, const
     for (int b = blockIdx.x; b < n; b += gridDim.x) {
         prep_one(raw + (size_t)b * hw, bg, a, out + (size_t)b * hw, img, img + ((hw + 3) & ~3), red);
         __syncthreads();  // every thread done with the slot before the next pattern's loads
+    }
+}
+
+// ── the same chain, every sum in the same order, for what the fast forms take ──
+//
+// What bounded k_prep and k_prep_g (which stay for what these do not take): every tap of the direct
+// blur was two LDS reads and some eight instructions, the box path computed an exponential a tap and
+// pixel, an image in global memory had one wave a SIMD, and a tile's CLAHE table was read by lanes a
+// power of two apart. A pixel's last bit moves it from one NMI or CLAHE bin to the next, and records
+// with it, so every pixel here is the old kernels' bit for bit:
+// - the direct Gaussian is two products on the matrix cores, X Gx and Gy (X Gx), G the banded matrix
+//   of the taps. v_mfma_f32_32x32x2_f32 is fma(a1, b1, fma(a0, b0, c)) to the bit (checked against the
+//   VALU), so tap 2 s in the lower and 2 s + 1 in the upper lanes gives the serial sum's rounding; a
+//   tap outside the band adds 0. Taps come from one table of differences that each lane reads at an
+//   address of its own; groups of 8 taps outside the band are skipped.
+// - the box path's weights are tables made once a block (its sums and counts run as before).
+// - where the dynamic background by boxes is the whole chain, the image is not stored: the raw pixels
+//   are read for the boxes and again (from L2) where the background is subtracted (k_prep_box).
+// - the sums of the normalization stay on 256 threads, pixel i on thread i mod 256.
+// Blocks of 256 threads to 4 096 pixels, 512 to 16 384, 1 024 beyond.
+// 5 003 patterns of 60 x 60 in u8, the direct background: 436 -> 134 us; 160 of 240 x 320 in u16, by
+// boxes: 967 -> 116; 1 001 of 75 x 83 through background, CLAHE and band pass: 1 128 -> 329; 1 200 of
+// 120 x 120 in u16, by boxes: 870 -> 173. The outputs are the same bit for bit. (With the taps and sums
+// in another order the first three took 139, 86 and 228 us, but pixels a last bit away moved NMI bins:
+// a record's NMI by up to 0.5 %, and one cell of 6 035 past its acceptance.)
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+// row and column of pixel i in an image w wide (inv = 1 / w; exact to 2^22 pixels)
+__device__ __forceinline__ int2 pix_rc(int i, int w, float inv) {
+    int r = (int)(((float)i + 0.5f) * inv);
+    int c = i - r * w;
+    if (c < 0) {
+        c += w;
+        --r;
+    } else if (c >= w) {
+        c -= w;
+        ++r;
+    }
+    return make_int2(r, c);
+}
+
+// Words of LDS the direct Gaussian's tables take: the taps by difference, the sums of each column's
+// and row's taps.
+__host__ __device__ constexpr int tile_table_words(int radius, int h, int w) { return 2 * radius + 77 + w + h; }
+
+// The direct Gaussian of `img` (row stride S) through the scratch P (row stride S) on the matrix
+// cores; emit(row, col, value). `tab` (LDS) holds tile_table_words words. A wave takes 32 x 32 pixels
+// of the result; lane l of an A operand is row l % 32 and, of product s of a group of 8 taps, tap
+// 2 s + l / 32. A pixel that is not finite would reach pixels outside its radius through the zero
+// weights: such an image goes by gauss().
+template <int NT, typename Emit>
+__device__ void gauss_tiles(const float* img, int S, float* P, float* tab, int h, int w, const BlurArg& g, Emit emit) {
+    const int R = g.radius, off = R + 38;
+    const int tid = threadIdx.x;
+    float* wt = tab;
+    float* sx = wt + 2 * R + 77;
+    const float* sy = sx + w;
+    for (int t = tid; t < 2 * R + 77; t += NT) {
+        const int d = abs(t - off);
+        wt[t] = d <= R ? expf(-(float)(d * d) * g.k) : 0.f;
+    }
+    __syncthreads();
+    for (int p = tid; p < w + h; p += NT) {
+        const int n = p < w ? w : h, q = p < w ? p : p - w;
+        const int x1 = min(q + R, n - 1);
+        float ws = 0.f;
+#pragma unroll 8
+        for (int x = max(q - R, 0); x <= x1; ++x) ws += wt[off + x - q];
+        sx[p] = ws;
+    }
+    __syncthreads();
+    const int lane = tid & 63, l = lane & 31, hi = lane >> 5;
+    const int CT = (w + 31) >> 5, RT = (h + 31) >> 5;
+    for (int t = __builtin_amdgcn_readfirstlane(tid >> 6); t < CT * RT; t += NT / 64) {
+        const int rt = t / CT, ct = t - rt * CT;
+        const int c = 32 * ct + l;
+        const float* line = img + (size_t)min(32 * rt + l, h - 1) * S;
+        const float* wp = wt + off + hi - c;
+        const int g1 = min(32 * ct + 31 + R, w - 1) >> 3;
+        f32x16 acc = {};
+        for (int k = max(32 * ct - R, 0) >> 3; k <= g1; ++k) {
+            float a[4], b[4];
+            const int x = 8 * k + hi;
+#pragma unroll
+            for (int s = 0; s < 4; ++s) b[s] = wp[8 * k + 2 * s];
+            if (8 * k + 8 <= w) {
+#pragma unroll
+                for (int s = 0; s < 4; ++s) a[s] = line[x + 2 * s];
+            } else {
+#pragma unroll
+                for (int s = 0; s < 4; ++s) {
+                    const float v = line[min(x + 2 * s, w - 1)];
+                    a[s] = x + 2 * s < w ? v : 0.f;
+                }
+            }
+#pragma unroll
+            for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s], b[s], acc, 0, 0, 0);
+        }
+        const float ws = sx[min(c, w - 1)];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const int r = 32 * rt + 8 * (i >> 2) + 4 * hi + (i & 3);
+            if (r < h && c < w) P[(size_t)r * S + c] = acc[i] / ws;
+        }
+    }
+    __syncthreads();
+    for (int t = __builtin_amdgcn_readfirstlane(tid >> 6); t < CT * RT; t += NT / 64) {
+        const int rt = t / CT, ct = t - rt * CT;
+        const int c = 32 * ct + l;
+        const float* col = P + min(c, w - 1);
+        const float* wp = wt + off + hi - (32 * rt + l);
+        const int g1 = min(32 * rt + 31 + R, h - 1) >> 3;
+        f32x16 acc = {};
+        for (int k = max(32 * rt - R, 0) >> 3; k <= g1; ++k) {
+            float a[4], b[4];
+            const int y = 8 * k + hi;
+#pragma unroll
+            for (int s = 0; s < 4; ++s) a[s] = wp[8 * k + 2 * s];
+            if (8 * k + 8 <= h) {
+#pragma unroll
+                for (int s = 0; s < 4; ++s) b[s] = col[(size_t)(y + 2 * s) * S];
+            } else {
+#pragma unroll
+                for (int s = 0; s < 4; ++s) {
+                    const float v = col[(size_t)min(y + 2 * s, h - 1) * S];
+                    b[s] = y + 2 * s < h ? v : 0.f;
+                }
+            }
+#pragma unroll
+            for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s], b[s], acc, 0, 0, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const int r = 32 * rt + 8 * (i >> 2) + 4 * hi + (i & 3);
+            if (r < h && c < w) emit(r, c, acc[i] / sy[r]);
+        }
+    }
+    __syncthreads();
+}
+
+// Words of LDS the box path takes: the spread's weights of either axis, the cells [hp][wp] with their
+// counts, then in turn the boxes, the cells along the rows and the coarse weights, or each column's
+// cells [hp][w].
+__host__ __device__ inline long box_words(const BlurArg& g, int h, int w) {
+    const long coarse = 2L * g.hs * g.wp + (long)g.hs * g.ws + (long)g.wp * g.nbx + (long)g.hp * g.nby;
+    const long spread = 2L * g.hp * w;
+    return 2L * g.hp * g.wp + 7L * w + 7L * h + 1 + (coarse > spread ? coarse : spread);
+}
+
+// The Gaussian by boxes of the image whose pixels load(row, col) gives; emit(row, col, value). The
+// sums of gauss()'s box path, each weight read from a table. `aux` (LDS) 8-byte aligned.
+template <int NT, typename Load, typename Emit>
+__device__ void gauss_box(float* aux, int h, int w, const BlurArg& g, Load load, Emit emit) {
+    const int tid = threadIdx.x;
+    const int s = g.s, pad = g.pad, hs = g.hs, ws = g.ws, hp = g.hp, wp = g.wp;
+    float2* C2 = reinterpret_cast<float2*>(aux);                              // [hp][wp]
+    float* ex = aux + 2 * hp * wp;                                            // [w][7]
+    float* ey = ex + 7 * w;                                                   // [h][7]
+    float2* C1 = reinterpret_cast<float2*>(aux + ((2 * hp * wp + 7 * w + 7 * h + 1) & ~1));  // [hs][wp]
+    float* C0 = reinterpret_cast<float*>(C1 + hs * wp);                       // [hs][ws]
+    float* kx = C0 + hs * ws;                                                 // [wp][nbx]
+    float* ky = kx + wp * g.nbx;                                              // [hp][nby]
+    float2* A = C1;                                                           // [hp][w]
+    const float fs = (float)s;
+    auto first = [&](float cc) { return max((int)floorf((cc - g.reach) / fs), 0); };
+    auto last = [&](float cc, int cells) { return min((int)floorf((cc + g.reach) / fs), cells - 1); };
+    const float invw = 1.f / (float)w;
+    for (int t = tid; t < hs * ws; t += NT) {
+        const int i = t / ws, j = t - i * ws;
+        const int r1 = min((i + 1) * s, h), q1 = min((j + 1) * s, w);
+        float acc = 0.f;
+        for (int r = i * s; r < r1; ++r) {
+#pragma unroll 8
+            for (int q = j * s; q < q1; ++q) acc += load(r, q);
+        }
+        C0[t] = acc;
+    }
+    const int nkx = wp * g.nbx;
+    for (int t = tid; t < nkx + hp * g.nby; t += NT) {
+        const bool x = t < nkx;
+        const int u = x ? t : t - nkx, nb = x ? g.nbx : g.nby, n = x ? w : h;
+        const int to = u / nb;
+        const float cc = prep_cell(to - pad, n, s).x;
+        const float d = prep_cell(first(cc) + u - to * nb, n, s).x - cc;
+        kx[t] = expf(-d * d * g.k0);
+    }
+    for (int t = tid; t < 7 * (w + h); t += NT) {
+        const bool x = t < 7 * w;
+        const int u = x ? t : t - 7 * w, n = x ? w : h;
+        const int at = u / 7, q = u - at * 7;
+        const float2 cw = prep_cell(at / s + q - pad, n, s);
+        const float d = (float)at - cw.x;
+        ex[t] = cw.y * expf(-d * d * g.k2);
+    }
+    __syncthreads();
+    // along the rows onto the coarse grid with its margin: [hs][wp]
+    for (int t = tid; t < hs * wp; t += NT) {
+        const int line = t / wp, tc = t - line * wp;
+        const float cc = prep_cell(tc - pad, w, s).x;
+        const int j0 = first(cc), j1 = last(cc, ws);
+        const float* k = kx + tc * g.nbx - j0;
+        const float* v = C0 + line * ws;
+        const int rows = min((line + 1) * s, h) - line * s;
+        float2 acc = make_float2(0.f, 0.f);
+#pragma unroll 4
+        for (int j = j0; j <= j1; ++j) {
+            const float n = (float)(rows * (min((j + 1) * s, w) - j * s));
+            acc = make_float2(acc.x + k[j] * v[j], acc.y + k[j] * n);
+        }
+        C1[t] = acc;
+    }
+    __syncthreads();
+    // along the columns: [hp][wp]
+    for (int t = tid; t < hp * wp; t += NT) {
+        const int tr = t / wp, col = t - tr * wp;
+        const float cc = prep_cell(tr - pad, h, s).x;
+        const int i0 = first(cc), i1 = last(cc, hs);
+        const float* k = ky + tr * g.nby - i0;
+        float2 acc = make_float2(0.f, 0.f);
+#pragma unroll 4
+        for (int i = i0; i <= i1; ++i) {
+            const float2 v = C1[i * wp + col];
+            acc = make_float2(acc.x + k[i] * v.x, acc.y + k[i] * v.y);
+        }
+        C2[t] = acc;
+    }
+    __syncthreads();
+    // spread over the pixels of each row from the 7 cells around: [hp][w]
+    for (int t = tid; t < hp * w; t += NT) {
+        const int2 rx = pix_rc(t, w, invw);
+        const float2* v = C2 + rx.x * wp + rx.y / s;
+        float2 acc = make_float2(0.f, 0.f);
+#pragma unroll
+        for (int q = 0; q < 7; ++q) {
+            const float e = ex[7 * rx.y + q];
+            acc = make_float2(acc.x + e * v[q].x, acc.y + e * v[q].y);
+        }
+        A[t] = acc;
+    }
+    __syncthreads();
+    // and of each column, into the pixels of a cell's rows
+    for (int t = tid; t < hs * w; t += NT) {
+        const int2 ix = pix_rc(t, w, invw);
+        const int r0 = ix.x * s, r1 = min(r0 + s, h);
+        float2 v[7];
+#pragma unroll
+        for (int q = 0; q < 7; ++q) v[q] = A[t + q * w];
+#pragma unroll 4
+        for (int r = r0; r < r1; ++r) {
+            float2 acc = make_float2(0.f, 0.f);
+#pragma unroll
+            for (int q = 0; q < 7; ++q) {
+                const float e = ey[7 * r + q];
+                acc = make_float2(acc.x + e * v[q].x, acc.y + e * v[q].y);
+            }
+            emit(r, ix.y, acc.x / acc.y);
+        }
+    }
+    __syncthreads();
+}
+
+// clahe_block for an image of row stride S, the tiles' tables B + 1 words apart (a thread a tile makes
+// them, so that the threads of a wave read 64 banks).
+template <int NT>
+__device__ void clahe_tiles(float* img, int S, unsigned* hist, const PrepArg& a, float* red) {
+    const int h = a.h, w = a.w, hw = h * w;
+    const int tid = threadIdx.x;
+    const int T = a.tiles, B = a.bins;
+    const float invw = 1.f / (float)w;
+    float lo = 3.4e38f, hi = -3.4e38f;
+    for (int i = tid; i < hw; i += NT) {
+        const int2 rc = pix_rc(i, w, invw);
+        const float v = img[(size_t)rc.x * S + rc.y];
+        lo = fminf(lo, v);
+        hi = fmaxf(hi, v);
+    }
+    for (int o = 32; o >= 1; o >>= 1) {
+        lo = fminf(lo, __shfl_xor(lo, o, 64));
+        hi = fmaxf(hi, __shfl_xor(hi, o, 64));
+    }
+    if ((tid & 63) == 0) {
+        red[tid >> 6] = lo;
+        red[NT / 64 + (tid >> 6)] = hi;
+    }
+    for (int i = tid; i < T * T * (B + 1); i += NT) hist[i] = 0u;
+    __syncthreads();
+    for (int i = 0; i < NT / 64; ++i) {
+        lo = fminf(lo, red[i]);
+        hi = fmaxf(hi, red[NT / 64 + i]);
+    }
+    const float k = 1.f / fmaxf(hi - lo, 1e-20f);
+    const int hp = h + a.pad_h, wp = w + a.pad_w;
+    const float invp = 1.f / (float)wp;
+    for (int t = tid; t < hp * wp; t += NT) {
+        const int2 p = pix_rc(t, wp, invp);
+        const float v = (img[(size_t)clahe_reflect(p.x, h, a.pad_h) * S + clahe_reflect(p.y, w, a.pad_w)] - lo) * k;
+        const int tile = (p.x / a.tile_h) * T + p.y / a.tile_w;
+        atomicAdd(&hist[tile * (B + 1) + clahe_bin(v, B)], 1u);
+    }
+    __syncthreads();
+    for (int t = tid; t < T * T; t += NT) clahe_table(hist + t * (B + 1), B, (float)max(a.tile_h * a.tile_w, 1), a.clip);
+    __syncthreads();
+    const float* cdf = reinterpret_cast<const float*>(hist);
+    for (int i = tid; i < hw; i += NT) {
+        const int2 rc = pix_rc(i, w, invw);
+        float* p = img + (size_t)rc.x * S + rc.y;
+        *p = clahe_value((*p - lo) * k, rc.x, rc.y, h, w, T, B, cdf, B + 1);
+    }
+    __syncthreads();
+}
+
+// The sum of the first 256 threads' values (the others' are not counted) on every thread, as block_sum<256>.
+__device__ __forceinline__ float sum256(float v, float* red) {
+    v = warp_sum(v);
+    const int w = threadIdx.x >> 6;
+    if ((threadIdx.x & 63) == 0 && w < 4) red[w] = v;
+    __syncthreads();
+    float t = 0.f;
+    for (int i = 0; i < 4; ++i) t += red[i];
+    __syncthreads();
+    return t;
+}
+
+// A block a pattern with the image in LDS (row stride S, odd: the tiles' lanes read down the rows),
+// or, GLOB, in the block's slot of global memory (patterns blockIdx.x, + gridDim.x, ...; S = w) with
+// what is smaller than an image in LDS still. vec: four pixels a load and store (h w a multiple of
+// 4, raw, background and out aligned to four pixels).
+template <typename T, int NT, bool GLOB>
+__global__ void __launch_bounds__(NT, 4) k_prep_tiles(const T* __restrict__ raw, const float* __restrict__ bg, PrepArg a, int n, int S, int vec,
+                                                   float* __restrict__ work, long slot, float* __restrict__ out) {
+    extern __shared__ double lds64[];
+    __shared__ float red[2 * NT / 64];
+    float* lds = reinterpret_cast<float*>(lds64);
+    const int h = a.h, w = a.w, hw = h * w, tid = threadIdx.x;
+    const int area = (h * S + 3) & ~3;
+    const float invw = 1.f / (float)w;
+    float* img = GLOB ? work + (size_t)blockIdx.x * slot : lds;
+    float* P = img + area;                            // the direct Gaussian's scratch
+    float* near = GLOB ? lds : lds + area;            // the box path's, CLAHE's
+    float* tab = GLOB ? lds : lds + 2 * area;         // the direct Gaussian's tables
+    for (int b = blockIdx.x; b < n; b += gridDim.x) {
+        const T* src = raw + (size_t)b * hw;
+        float* dst = out + (size_t)b * hw;
+        bool odd = false;  // a pixel not finite, or too large to stay so
+        if (vec) {
+            for (int i = 4 * tid; i < hw; i += 4 * NT) {
+                float x[4];
+                PixVec<T, 4>::load(src + i, x);
+                if (bg) {
+                    const float4 q = *reinterpret_cast<const float4*>(bg + i);
+                    x[0] -= q.x, x[1] -= q.y, x[2] -= q.z, x[3] -= q.w;
+                }
+                int2 rc = pix_rc(i, w, invw);
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    odd |= !(fabsf(x[u]) < 1e30f);
+                    img[(size_t)rc.x * S + rc.y] = x[u];
+                    if (++rc.y == w) {
+                        rc.y = 0;
+                        ++rc.x;
+                    }
+                }
+            }
+        } else {
+            for (int i = tid; i < hw; i += NT) {
+                const float x = (float)src[i] - (bg ? bg[i] : 0.f);
+                const int2 rc = pix_rc(i, w, invw);
+                odd |= !(fabsf(x) < 1e30f);
+                img[(size_t)rc.x * S + rc.y] = x;
+            }
+        }
+        const bool loops = __syncthreads_or(odd);
+        // the dynamic background, then (after CLAHE) the band pass: its coarse Gaussian into the
+        // output row, its fine one less that. One copy of the code for the three.
+#pragma unroll 1
+        for (int stage = 0; stage < 3; ++stage) {
+            if (stage == 1 && a.clahe) clahe_tiles<NT>(img, S, reinterpret_cast<unsigned*>(near), a, red);
+            if (!(stage == 0 ? a.dyn : stage == 1 ? a.bp : a.bp && a.bp_fine)) continue;
+            const BlurArg g = stage == 0 ? a.dynb : stage == 1 ? a.coarse : a.fine;
+            auto emit = [&](int r, int c, float v) {
+                float* p = img + (size_t)r * S + c;
+                if (stage == 0)
+                    *p = a.dyn == 1 ? *p - v : *p / fmaxf(v, 1e-6f);
+                else if (stage == 1)
+                    dst[r * w + c] = v;
+                else
+                    *p = v - dst[r * w + c];
+            };
+            if (g.box)
+                gauss_box<NT>(near, h, w, g, [&](int r, int c) { return img[(size_t)r * S + c]; }, emit);
+            else if (loops)
+                gauss<NT>(img, P, h, w, S, g, emit);
+            else
+                gauss_tiles<NT>(img, S, P, tab, h, w, g, emit);
+        }
+        if (a.bp && !a.bp_fine) {
+            for (int i = tid; i < hw; i += NT) {
+                const int2 rc = pix_rc(i, w, invw);
+                img[(size_t)rc.x * S + rc.y] -= dst[i];
+            }
+            __syncthreads();
+        }
+        float sm = 0.f, cn = 0.f;
+        if (tid < 256) {
+#pragma unroll 4
+            for (int i = tid; i < hw; i += 256) {
+                const int2 rc = pix_rc(i, w, invw);
+                const float v = img[(size_t)rc.x * S + rc.y];
+                const bool in = in_mask((float)rc.x, (float)rc.y, a.mask);
+                sm += in ? v : 0.f;
+                cn += in ? 1.f : 0.f;
+            }
+        }
+        sm = sum256(sm, red);
+        cn = sum256(cn, red);
+        const float mean = sm / fmaxf(cn, 1.f);
+        float ss = 0.f;
+        if (tid < 256) {
+#pragma unroll 4
+            for (int i = tid; i < hw; i += 256) {
+                const int2 rc = pix_rc(i, w, invw);
+                const float x = img[(size_t)rc.x * S + rc.y];
+                const float v = in_mask((float)rc.x, (float)rc.y, a.mask) ? x - mean : 0.f;
+                img[(size_t)rc.x * S + rc.y] = v;
+                ss += v * v;
+            }
+        }
+        ss = sum256(ss, red);
+        const float inv = 1.f / sqrtf(fmaxf(ss, 1e-30f));
+        if (vec) {
+            for (int i = 4 * tid; i < hw; i += 4 * NT) {
+                int2 rc = pix_rc(i, w, invw);
+                float x[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    x[u] = img[(size_t)rc.x * S + rc.y] * inv;
+                    if (++rc.y == w) {
+                        rc.y = 0;
+                        ++rc.x;
+                    }
+                }
+                *reinterpret_cast<float4*>(dst + i) = make_float4(x[0], x[1], x[2], x[3]);
+            }
+        } else {
+            for (int i = tid; i < hw; i += NT) {
+                const int2 rc = pix_rc(i, w, invw);
+                dst[i] = img[(size_t)rc.x * S + rc.y] * inv;
+            }
+        }
+        __syncthreads();  // every thread done with the image before the next pattern's
+    }
+}
+
+// The dynamic background by boxes and the normalization alone, a block a pattern: the image is never
+// held. The background's difference goes to the output row and is scaled there.
+template <typename T, int NT>
+__global__ void __launch_bounds__(NT) k_prep_box(const T* __restrict__ raw, const float* __restrict__ bg, PrepArg a, int vec, float* __restrict__ out) {
+    extern __shared__ double lds64[];
+    __shared__ float red[NT / 64];
+    const int h = a.h, w = a.w, hw = h * w, tid = threadIdx.x;
+    const T* src = raw + (size_t)blockIdx.x * hw;
+    float* dst = out + (size_t)blockIdx.x * hw;
+    float sm = 0.f, cn = 0.f;
+    const int dyn = a.dyn;
+    auto load = [&](int r, int c) {
+        const int i = r * w + c;
+        return (float)src[i] - (bg ? bg[i] : 0.f);
+    };
+    gauss_box<NT>(reinterpret_cast<float*>(lds64), h, w, a.dynb, load, [&](int r, int c, float v) {
+        const float x = load(r, c);
+        const float y = dyn == 1 ? x - v : x / fmaxf(v, 1e-6f);
+        const bool in = in_mask((float)r, (float)c, a.mask);
+        dst[r * w + c] = in ? y : 0.f;
+        cn += in ? 1.f : 0.f;
+    });
+    if (tid < 256) {
+#pragma unroll 8
+        for (int i = tid; i < hw; i += 256) sm += dst[i];
+    }
+    sm = sum256(sm, red);
+    cn = block_sum<NT>(cn, red);
+    const float mean = sm / fmaxf(cn, 1.f);
+    const float invw = 1.f / (float)w;
+    float ss = 0.f;
+    if (tid < 256) {
+#pragma unroll 8
+        for (int i = tid; i < hw; i += 256) {
+            const int2 rc = pix_rc(i, w, invw);
+            const float x = dst[i];
+            const float v = in_mask((float)rc.x, (float)rc.y, a.mask) ? x - mean : 0.f;
+            ss += v * v;
+        }
+    }
+    ss = sum256(ss, red);
+    const float inv = 1.f / sqrtf(fmaxf(ss, 1e-30f));
+    if (vec) {
+        for (int i = 4 * tid; i < hw; i += 4 * NT) {
+            const float4 q = *reinterpret_cast<const float4*>(dst + i);
+            float x[4] = {q.x, q.y, q.z, q.w};
+            int2 rc = pix_rc(i, w, invw);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                x[u] = (in_mask((float)rc.x, (float)rc.y, a.mask) ? x[u] - mean : 0.f) * inv;
+                if (++rc.y == w) {
+                    rc.y = 0;
+                    ++rc.x;
+                }
+            }
+            *reinterpret_cast<float4*>(dst + i) = make_float4(x[0], x[1], x[2], x[3]);
+        }
+    } else {
+        for (int i = tid; i < hw; i += NT) {
+            const int2 rc = pix_rc(i, w, invw);
+            dst[i] = (in_mask((float)rc.x, (float)rc.y, a.mask) ? dst[i] - mean : 0.f) * inv;
+        }
     }
 }
 
@@ -693,6 +1214,8 @@ static size_t blur_arg(double sigma, int h, int w, BlurArg& g) {
     g.ws = (w + s - 1) / s;
     g.hp = g.hs + 2 * g.pad;
     g.wp = g.ws + 2 * g.pad;
+    g.nbx = std::min(g.ws, (int)(2 * g.reach / s) + 2);
+    g.nby = std::min(g.hs, (int)(2 * g.reach / s) + 2);
     return (size_t)2 * g.hp * (g.wp > w ? g.wp : w) * 2;
 }
 
@@ -753,13 +1276,63 @@ static long prep_slot(const PrepArg& a, long scratch) {
     return ((((hw + 3) & ~3L) + scratch) + 63) & ~63L;  // floats, slots 256-byte aligned
 }
 
+// Which kernel takes a call. `global`: the image is past a block's LDS in k_prep's form (or the
+// caller asked for global memory), which alone decides what is refused and which workspace it takes.
+enum PrepForm { kPrepLoops, kPrepLoopsG, kPrepTiles, kPrepTilesG, kPrepBoxes };
+
+// The fast forms wherever what they keep in LDS fits (their tables differ from k_prep's scratch,
+// so it doesn't for a few images near the limit, nor for long thin ones) and pix_rc is exact; `lds`
+// becomes the bytes of dynamic LDS, `S` the image's row stride.
+static PrepForm prep_form(const PrepArg& a, bool global, int limit, size_t& lds, int& S) {
+    const PrepForm loops = global ? kPrepLoopsG : kPrepLoops;
+    const long hw = (long)a.h * a.w, room = (long)(limit - 1024) / 4;
+    if (hw > (1L << 22)) return loops;
+    if (a.dyn && a.dynb.box && !a.clahe && !a.bp && box_words(a.dynb, a.h, a.w) <= room) {
+        lds = (size_t)box_words(a.dynb, a.h, a.w) * 4;
+        return kPrepBoxes;
+    }
+    S = global ? a.w : a.w | 1;
+    const long area = global ? 0 : ((long)a.h * S + 3) & ~3L;
+    long aux = a.clahe ? (long)a.tiles * a.tiles * (a.bins + 1) : 0;
+    auto need = [&](const BlurArg& g) { aux = std::max(aux, g.box ? box_words(g, a.h, a.w) : area + tile_table_words(g.radius, a.h, a.w)); };
+    if (a.dyn) need(a.dynb);
+    if (a.bp) need(a.coarse);
+    if (a.bp_fine) need(a.fine);
+    if (area + aux > room) return loops;
+    lds = (size_t)(area + aux) * 4;
+    return global ? kPrepTilesG : kPrepTiles;
+}
+
+// threads a block by the pixels (the text above the forms); a frame past LDS has its CU to itself
 template <typename T>
-static void prep_launch(const void* raw, const float* bg, const PrepArg& a, int n, bool global, size_t lds, float* work, long slot, int grid,
+static void prep_launch(const void* raw_, const float* bg, const PrepArg& a, int n, PrepForm form, size_t lds, int S, float* work, long slot, int grid,
                         float* out, hipStream_t s) {
-    if (global)
-        ZB_LAUNCH("k_prep", k_prep_g<T>, dim3(grid), dim3(256), 0, s, (const T*)raw, bg, a, n, work, slot, out);
+    const T* raw = (const T*)raw_;
+    const long hw = (long)a.h * a.w;
+    const int vec = hw % 4 == 0 && (uintptr_t)raw % (4 * sizeof(T)) == 0 && (uintptr_t)out % 16 == 0 && (uintptr_t)bg % 16 == 0;
+#define ZB_TILES(NT, G, GRID) \
+    ZB_LAUNCH("k_prep", (k_prep_tiles<T, NT, G>), dim3(GRID), dim3(NT), lds, s, raw, bg, a, n, S, vec, work, slot, out)
+    if (form == kPrepBoxes && hw <= 16384)
+        ZB_LAUNCH("k_prep", (k_prep_box<T, 512>), dim3(n), dim3(512), lds, s, raw, bg, a, vec, out);
+    else if (form == kPrepBoxes)
+        ZB_LAUNCH("k_prep", (k_prep_box<T, 1024>), dim3(n), dim3(1024), lds, s, raw, bg, a, vec, out);
+    else if (form == kPrepLoopsG)
+        ZB_LAUNCH("k_prep", k_prep_g<T>, dim3(grid), dim3(256), 0, s, raw, bg, a, n, work, slot, out);
+    else if (form == kPrepLoops)
+        ZB_LAUNCH("k_prep", k_prep<T>, dim3(n), dim3(256), lds, s, raw, bg, a, out);
+    else if (form == kPrepTilesG && hw <= 4096)
+        ZB_TILES(256, true, grid);
+    else if (form == kPrepTilesG && hw <= 16384)
+        ZB_TILES(512, true, grid);
+    else if (form == kPrepTilesG)
+        ZB_TILES(1024, true, grid);
+    else if (hw <= 4096)
+        ZB_TILES(256, false, n);
+    else if (hw <= 16384)
+        ZB_TILES(512, false, n);
     else
-        ZB_LAUNCH("k_prep", k_prep<T>, dim3(n), dim3(256), lds, s, (const T*)raw, bg, a, out);
+        ZB_TILES(1024, false, n);
+#undef ZB_TILES
 }
 
 static int32_t prep_run(const char* who, const void* raw, int32_t pixel, int32_t n, int32_t h, int32_t w, const float mask[3], const zb_prep_opts* o,
@@ -802,12 +1375,14 @@ static int32_t prep_run(const char* who, const void* raw, int32_t pixel, int32_t
     }
     hipStream_t s = (hipStream_t)stream;
     const float* bg = o->background;
+    int S = w;
+    const PrepForm form = prep_form(a, global, limit, lds, S);
     if (pixel == 0)
-        prep_launch<uint8_t>(raw, bg, a, n, global, lds, (float*)work, slot, grid, out, s);
+        prep_launch<uint8_t>(raw, bg, a, n, form, lds, S, (float*)work, slot, grid, out, s);
     else if (pixel == 1)
-        prep_launch<uint16_t>(raw, bg, a, n, global, lds, (float*)work, slot, grid, out, s);
+        prep_launch<uint16_t>(raw, bg, a, n, form, lds, S, (float*)work, slot, grid, out, s);
     else
-        prep_launch<float>(raw, bg, a, n, global, lds, (float*)work, slot, grid, out, s);
+        prep_launch<float>(raw, bg, a, n, form, lds, S, (float*)work, slot, grid, out, s);
     return check_launch(who);
 }
 
