@@ -77,6 +77,7 @@ struct VArg {
     // rows of b the GEMM computes (jg) and the peak searches (jp): all n/2 + 1, or with b_half
     // j <= n/4 searched and one row more computed for the peak's neighbour along b
     int jg, jp;
+    int jw;     // rows of b a GEMM block computes: blockIdx.y jw on (an even count, or all jg)
     int lp_gs;  // 16-bit products: the first group of 8 slots that takes the hi + lo product
     int vk;     // V's elements: 0 FP32 pairs (cols floats a row), 1 FP16 / 2 BF16 pairs (nc a row)
     // the items' best (value, index) keys, which the correlation's GEMM clears (its blocks of
@@ -189,6 +190,24 @@ __device__ __forceinline__ void vgemm_run(const VArg& a, int mp, int tile, int c
             dst[idx < F4 ? idx : F4] = pre[p];
         }
     };
+    const int j0 = blockIdx.y * a.jw, j1 = min(j0 + a.jw, a.jg);  // this block's rows of b
+    if (tile * MB * 32 >= a.n_items) {
+        // a wave whose items are all padding (nothing reads a tile past the last item's): it stages
+        // the rows with the others and neither multiplies nor stores
+        floatx4* dst[2] = {lds0, lds1};
+        stage_load(j0);
+        stage_store(lds0);
+        __syncthreads();
+        for (int j = j0; j < j1; j += 2) {
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                stage_load(min(j + u + 1, j1 - 1));
+                stage_store(dst[1 - u]);
+                __syncthreads();
+            }
+        }
+        return;
+    }
     // V row of one (j, m'): ni_pad items x cols floats (2 nc, or 32 when nc < 16: the table's
     // zero columns are stored too, so no store needs a predicate)
     const int w = a.cols;
@@ -206,7 +225,7 @@ __device__ __forceinline__ void vgemm_run(const VArg& a, int mp, int tile, int c
     // never wait for the stores of j to read their registers.
     auto step = [&](int j, Acc& acc, Acc& other, const floatx4* cur, floatx4* nxt) {
         // the last j stages its own rows again: no branch
-        stage_load(min(j + 1, a.jg - 1));
+        stage_load(min(j + 1, j1 - 1));
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
@@ -255,7 +274,7 @@ __device__ __forceinline__ void vgemm_run(const VArg& a, int mp, int tile, int c
         stage_store(nxt);
         __syncthreads();
     };
-    stage_load(0);
+    stage_load(j0);
     stage_store(lds0);
     __syncthreads();
     Acc acc0, acc1;
@@ -266,9 +285,9 @@ __device__ __forceinline__ void vgemm_run(const VArg& a, int mp, int tile, int c
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc1[mb][nb][0][r] = 0.f;
     // an odd count repeats the last j (the same values to the same place)
-    for (int j = 0; j < a.jg; j += 2) {
+    for (int j = j0; j < j1; j += 2) {
         step(j, acc0, acc1, lds0, lds1);
-        step(min(j + 1, a.jg - 1), acc1, acc0, lds1, lds0);
+        step(min(j + 1, j1 - 1), acc1, acc0, lds1, lds0);
     }
 }
 
@@ -393,6 +412,24 @@ __device__ __forceinline__ void vgemm16_run(const VArg& a, int mp, int tile, int
             dst[idx < F4 ? idx : F4] = pre[p];  // past the rows: the spare slot after them
         }
     };
+    const int j0 = blockIdx.y * a.jw, j1 = min(j0 + a.jw, a.jg);  // this block's rows of b
+    if (tile * MB * 32 >= a.n_items) {
+        // a wave whose items are all padding (nothing reads a tile past the last item's): it stages
+        // the rows with the others and neither multiplies nor stores
+        floatx4* dst[2] = {lds0, lds1};
+        stage_load(j0);
+        stage_store(lds0);
+        __syncthreads();
+        for (int j = j0; j < j1; j += 2) {
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                stage_load(min(j + u + 1, j1 - 1));
+                stage_store(dst[1 - u]);
+                __syncthreads();
+            }
+        }
+        return;
+    }
     // V row of one (j, m'): ni_pad items x nc 32-bit (re, im) pairs; the lane's complex column
     const int w = a.nc;
     const size_t vrow = (size_t)a.ni_pad * w;
@@ -401,7 +438,7 @@ __device__ __forceinline__ void vgemm16_run(const VArg& a, int mp, int tile, int
     for (int mb = 0; mb < MB; ++mb) loff[mb] = 4u * (unsigned)(((tile * MB + mb) * 32 + half * 4) * w + cg * 32 + r32);
     typedef floatx16 Acc[MB][NBLK][1];
     auto step = [&](int j, Acc& acc, Acc& other, const floatx4* cur, floatx4* nxt) {
-        stage_load(min(j + 1, a.jg - 1));
+        stage_load(min(j + 1, j1 - 1));
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
@@ -453,7 +490,7 @@ __device__ __forceinline__ void vgemm16_run(const VArg& a, int mp, int tile, int
         stage_store(nxt);
         __syncthreads();
     };
-    stage_load(0);
+    stage_load(j0);
     stage_store(lds0);
     __syncthreads();
     Acc acc0, acc1;
@@ -463,9 +500,9 @@ __device__ __forceinline__ void vgemm16_run(const VArg& a, int mp, int tile, int
         for (int nb = 0; nb < NBLK; ++nb)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc1[mb][nb][0][r] = 0.f;
-    for (int j = 0; j < a.jg; j += 2) {
+    for (int j = j0; j < j1; j += 2) {
         step(j, acc0, acc1, lds0, lds1);
-        step(min(j + 1, a.jg - 1), acc1, acc0, lds1, lds0);
+        step(min(j + 1, j1 - 1), acc1, acc0, lds1, lds0);
     }
 }
 
@@ -1048,6 +1085,17 @@ extern "C" int64_t zb_vcorr_workspace(const zb_vtable* t, int32_t n_items, int32
     return vcorr_ws(a, denominators != 0);
 }
 
+// Blocks along b: a block's rows are a chain (a row's staging, products and stores), so where the
+// tiles, orders and column groups alone leave the chip part empty (below three blocks a CU, what a
+// k_vgemm's registers allow) each takes fewer rows of b, two at the least. 3 items at L = 64: 64 blocks
+// of 34 rows 94 us, 576 of 4 rows (and no products and stores for waves of padding) 19. Beyond that one
+// block a range is as fast or faster (4 500 items: 0.223 us a pattern, 0.226 to 0.234 with 2 to 4).
+static int v_parts(VArg& b, long blocks) {
+    const int parts = (int)std::max(1L, std::min((long)(b.jg + 1) / 2, 768 / std::max(blocks, 1L)));
+    b.jw = parts == 1 ? b.jg : ((b.jg + parts - 1) / parts + 1) & ~1;
+    return (b.jg + b.jw - 1) / b.jw;
+}
+
 template <int MB, int NBLK, int S>
 static void launch_vgemm_t(const VArg& a, const float* q, const float* alm, float* v, hipStream_t s) {
     // a block takes kWaves tiles of 32 MB items (ni_pad is a multiple of that)
@@ -1056,7 +1104,9 @@ static void launch_vgemm_t(const VArg& a, const float* q, const float* alm, floa
     b.tiles = tiles;
     const int ncg = a.cols / (NBLK * 32);
     const size_t lds = 2 * ((size_t)(S / 4) * NBLK * 64 + 1) * 16;  // two buffers of one j's rows (and a spare slot)
-    ZB_LAUNCH("k_vgemm", (k_vgemm<MB, NBLK, S>), dim3((unsigned)(tiles * a.L * ncg)), dim3(64 * kWaves), lds, s, b, q, (const float2*)alm, v);
+    const int parts = v_parts(b, (long)tiles * a.L * ncg);
+    ZB_LAUNCH("k_vgemm", (k_vgemm<MB, NBLK, S>), dim3((unsigned)(tiles * a.L * ncg), parts), dim3(64 * kWaves), lds, s, b, q,
+              (const float2*)alm, v);
 }
 
 template <int NBLK, int G8, int GS, bool BF>
@@ -1066,7 +1116,8 @@ static void launch_vgemm16_t(const VArg& a, const void* q, const float* alm, voi
     b.tiles = tiles;
     const int ncg = a.cols / (NBLK * 32);
     const size_t lds = 2 * ((size_t)(2 * G8 - GS) * NBLK * 64 + 1) * 16;
-    ZB_LAUNCH("k_vgemm", (k_vgemm16<1, NBLK, G8, GS, BF>), dim3((unsigned)(tiles * a.L * ncg)), dim3(64 * kWaves), lds, s, b, (const floatx4*)q,
+    const int parts = v_parts(b, (long)tiles * a.L * ncg);
+    ZB_LAUNCH("k_vgemm", (k_vgemm16<1, NBLK, G8, GS, BF>), dim3((unsigned)(tiles * a.L * ncg), parts), dim3(64 * kWaves), lds, s, b, (const floatx4*)q,
               (const float2*)alm, (unsigned*)v);
 }
 
