@@ -930,14 +930,13 @@ __global__ void __launch_bounds__(64) k_sums6(RefArg a, const float4* __restrict
     }
 #pragma unroll
     for (int i = 0; i < kSums; ++i) s[i] = wave_sum(s[i]);
-    // lane i writes sum i (the shift's sums zero for orientation refinement)
+    // lane i writes sum i (the shift's sums zero for orientation refinement), picked by value: a store a
+    // sum under its lane's condition became a tree of some 900 branches, as long as 50 steps of the walk
+    float x = s[0];
 #pragma unroll
-    for (int i = 0; i < kSums; ++i) {
-        if (lane == i) {
-            const bool shift = (i >= 4 && i < 7) || (i >= 10 && i < 13) || (i >= 16 && i < 19) || (i >= 22 && i < 37);
-            out[(size_t)b * kSums + i] = (rotation_only && shift) ? 0.f : s[i];
-        }
-    }
+    for (int i = 1; i < kSums; ++i) x = lane == i ? s[i] : x;
+    const bool shift = (lane >= 4 && lane < 7) || (lane >= 10 && lane < 13) || (lane >= 16 && lane < 19) || (lane >= 22 && lane < 37);
+    if (lane < kSums) out[(size_t)b * kSums + lane] = (rotation_only && shift) ? 0.f : x;
 }
 
 }  // namespace zb
