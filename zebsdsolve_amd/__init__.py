@@ -47,9 +47,10 @@ def _unit_rand(x):
 
 def decoys(n, draw):
     """Uniform random orientations (Shoemake) for items 0..n-1 of draw `draw`, a different one
-    per item and draw (detector.wgsl decoy, 296-308)."""
+    per item and draw (detector.wgsl decoy, 296-308): [n, 4], or [d, n, 4] for d draws."""
     b = np.arange(n, dtype=np.uint64)
-    s = _hash_u32(b + 1) ^ ((draw * 0x9E3779B9) & 0xFFFFFFFF)
+    d = np.asarray(draw, np.uint64)[..., None]
+    s = _hash_u32(b + 1) ^ ((d * 0x9E3779B9) & 0xFFFFFFFF)
     u1 = _unit_rand(s)
     a2 = _unit_rand(s + 1) * 2 * np.pi
     a3 = _unit_rand(s + 2) * 2 * np.pi
@@ -342,11 +343,9 @@ class Solver:
         n = min(region, 256)
         cells = np.array([(2 * j + 1) * region // (2 * n) for j in range(n)], np.int64)
         med, spread = [], []
+        draws = decoys(n, np.arange(8))
         for pi in range(len(e.phases)):
-            vals = []
-            for d in range(8):
-                vals.append(e.nmi_at(pi, cells, decoys(n, d)))
-            c = np.sort(np.concatenate(vals).astype(np.float32))
+            c = np.sort(e.nmi_at(pi, cells, draws).astype(np.float32), axis=None)
             m = c[len(c) // 2]
             dev = np.sort(np.abs(c - m))
             med.append(float(m))
@@ -451,6 +450,9 @@ class Solver:
             handle = pend[1]
         else:
             handle = self._e.index_cells_begin(cells, L)
+        # (the first step's results need the calibration: its draws are made beside the step's kernels)
+        if self._chance is None:
+            self._calibrate()
         # the sweep's next step goes to the GPU before this one is read back and landed on the
         # host, so the device does not wait for the host between steps
         nd = self._done + n
