@@ -1,6 +1,7 @@
 // Patterns in, masters baked: per-pattern normalization under the mask, simulated patterns,
 // and the master's smoothing and gradient on the sphere (setup, once per master and geometry).
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 
@@ -552,9 +553,9 @@ __global__ void __launch_bounds__(256) k_prep_g(const T* __restrict__ raw, const
 //   are read for the boxes and again (from L2) where the background is subtracted (k_prep_box).
 // - the sums of the normalization stay on 256 threads, pixel i on thread i mod 256.
 // Blocks of 256 threads to 4 096 pixels, 512 to 16 384, 1 024 beyond.
-// 5 003 patterns of 60 x 60 in u8, the direct background: 436 -> 134 us; 160 of 240 x 320 in u16, by
-// boxes: 967 -> 116; 1 001 of 75 x 83 through background, CLAHE and band pass: 1 128 -> 329; 1 200 of
-// 120 x 120 in u16, by boxes: 870 -> 173. The outputs are the same bit for bit. (With the taps and sums
+// 5 003 patterns of 60 x 60 in u8, the direct background: 436 -> 117 us; 160 of 240 x 320 in u16, by
+// boxes: 967 -> 100; 1 001 of 75 x 83 through background, CLAHE and band pass: 1 128 -> 315; 1 200 of
+// 120 x 120 in u16, by boxes: 870 -> 143. The outputs are the same bit for bit. (With the taps and sums
 // in another order the first three took 139, 86 and 228 us, but pixels a last bit away moved NMI bins:
 // a record's NMI by up to 0.5 %, and one cell of 6 035 past its acceptance.)
 
@@ -574,9 +575,41 @@ __device__ __forceinline__ int2 pix_rc(int i, int w, float inv) {
     return make_int2(r, c);
 }
 
+// a / b to the bit, b's reciprocal made once: the steps of the division without its scaling, which
+// changes nothing while neither b nor the quotient is near the ends of the range (b: sums of taps)
+__device__ __forceinline__ float recip_of(float b) {
+    const float y = __builtin_amdgcn_rcpf(b);
+    return __builtin_fmaf(__builtin_fmaf(-b, y, 1.f), y, y);
+}
+__device__ __forceinline__ float div_by(float a, float b, float y) {
+    const float q0 = a * y;
+    const float q1 = __builtin_fmaf(__builtin_fmaf(-b, q0, a), y, q0);
+    return __builtin_fmaf(__builtin_fmaf(-b, q1, a), y, q1);
+}
+
+// A pixel outside the mask between the sums: a NaN that no sum gives.
+constexpr int kOutside = 0x7fdecade;
+__device__ __forceinline__ bool outside(float v) { return __float_as_int(v) == kOutside; }
+
+// Row and column of pixel i, 256 pixels on at a step.
+struct Walk {
+    int r, c, dr, dc, w;
+    __device__ __forceinline__ Walk(int i, int w_, float inv, int step) : w(w_) {
+        const int2 a = pix_rc(i, w, inv), d = pix_rc(step, w, inv);
+        r = a.x, c = a.y, dr = d.x, dc = d.y;
+    }
+    __device__ __forceinline__ void next() {
+        r += dr;
+        c += dc;
+        const bool over = c >= w;
+        c -= over ? w : 0;
+        r += over ? 1 : 0;
+    }
+};
+
 // Words of LDS the direct Gaussian's tables take: the taps by difference, the sums of each column's
-// and row's taps.
-__host__ __device__ constexpr int tile_table_words(int radius, int h, int w) { return 2 * radius + 77 + w + h; }
+// and row's taps, the rows' reciprocals.
+__host__ __device__ constexpr int tile_table_words(int radius, int h, int w) { return 2 * radius + 77 + w + 2 * h; }
 
 // The direct Gaussian of `img` (row stride S) through the scratch P (row stride S) on the matrix
 // cores; emit(row, col, value). `tab` (LDS) holds tile_table_words words. A wave takes 32 x 32 pixels
@@ -590,6 +623,7 @@ __device__ void gauss_tiles(const float* img, int S, float* P, float* tab, int h
     float* wt = tab;
     float* sx = wt + 2 * R + 77;
     const float* sy = sx + w;
+    float* iy = sx + w + h;
     for (int t = tid; t < 2 * R + 77; t += NT) {
         const int d = abs(t - off);
         wt[t] = d <= R ? expf(-(float)(d * d) * g.k) : 0.f;
@@ -602,6 +636,7 @@ __device__ void gauss_tiles(const float* img, int S, float* P, float* tab, int h
 #pragma unroll 8
         for (int x = max(q - R, 0); x <= x1; ++x) ws += wt[off + x - q];
         sx[p] = ws;
+        if (p >= w) iy[p - w] = recip_of(ws);
     }
     __syncthreads();
     const int lane = tid & 63, l = lane & 31, hi = lane >> 5;
@@ -631,11 +666,11 @@ __device__ void gauss_tiles(const float* img, int S, float* P, float* tab, int h
 #pragma unroll
             for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s], b[s], acc, 0, 0, 0);
         }
-        const float ws = sx[min(c, w - 1)];
+        const float ws = sx[min(c, w - 1)], inv = recip_of(ws);
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
             const int r = 32 * rt + 8 * (i >> 2) + 4 * hi + (i & 3);
-            if (r < h && c < w) P[(size_t)r * S + c] = acc[i] / ws;
+            if (r < h && c < w) P[(size_t)r * S + c] = div_by(acc[i], ws, inv);
         }
     }
     __syncthreads();
@@ -667,7 +702,7 @@ __device__ void gauss_tiles(const float* img, int S, float* P, float* tab, int h
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
             const int r = 32 * rt + 8 * (i >> 2) + 4 * hi + (i & 3);
-            if (r < h && c < w) emit(r, c, acc[i] / sy[r]);
+            if (r < h && c < w) emit(r, c, div_by(acc[i], sy[r], iy[r]));
         }
     }
     __syncthreads();
@@ -700,16 +735,35 @@ __device__ void gauss_box(float* aux, int h, int w, const BlurArg& g, Load load,
     auto first = [&](float cc) { return max((int)floorf((cc - g.reach) / fs), 0); };
     auto last = [&](float cc, int cells) { return min((int)floorf((cc + g.reach) / fs), cells - 1); };
     const float invw = 1.f / (float)w;
-    for (int t = tid; t < hs * ws; t += NT) {
-        const int i = t / ws, j = t - i * ws;
-        const int r1 = min((i + 1) * s, h), q1 = min((j + 1) * s, w);
-        float acc = 0.f;
-        for (int r = i * s; r < r1; ++r) {
-#pragma unroll 8
-            for (int q = j * s; q < q1; ++q) acc += load(r, q);
+    // the boxes row by row, E pixels' loads in flight before any is added
+    auto boxes = [&](auto chunk) {
+        constexpr int E = decltype(chunk)::value;
+        for (int t = tid; t < hs * ws; t += NT) {
+            const int i = t / ws, j = t - i * ws;
+            const int q0 = j * s, q1 = min(q0 + s, w), total = (q1 - q0) * (min((i + 1) * s, h) - i * s);
+            int r = i * s, q = q0;
+            float acc = 0.f;
+            for (int e = 0; e < total; e += E) {
+                float v[E];
+#pragma unroll
+                for (int u = 0; u < E; ++u) {
+                    v[u] = load(min(r, h - 1), q);
+                    const bool over = ++q == q1;
+                    q = over ? q0 : q;
+                    r += over ? 1 : 0;
+                }
+#pragma unroll
+                for (int u = 0; u < E; ++u) acc = e + u < total ? acc + v[u] : acc;
+            }
+            C0[t] = acc;
         }
-        C0[t] = acc;
-    }
+    };
+    if (s == 2)
+        boxes(std::integral_constant<int, 4>{});
+    else if (s == 3)
+        boxes(std::integral_constant<int, 9>{});
+    else
+        boxes(std::integral_constant<int, 16>{});
     const int nkx = wp * g.nbx;
     for (int t = tid; t < nkx + hp * g.nby; t += NT) {
         const bool x = t < nkx;
@@ -735,11 +789,13 @@ __device__ void gauss_box(float* aux, int h, int w, const BlurArg& g, Load load,
         const int j0 = first(cc), j1 = last(cc, ws);
         const float* k = kx + tc * g.nbx - j0;
         const float* v = C0 + line * ws;
+        // the boxes' counts: all of a line alike but the last
         const int rows = min((line + 1) * s, h) - line * s;
+        const float whole = (float)(rows * s), rest = (float)(rows * (w - (ws - 1) * s));
         float2 acc = make_float2(0.f, 0.f);
 #pragma unroll 4
         for (int j = j0; j <= j1; ++j) {
-            const float n = (float)(rows * (min((j + 1) * s, w) - j * s));
+            const float n = j < ws - 1 ? whole : rest;
             acc = make_float2(acc.x + k[j] * v[j], acc.y + k[j] * n);
         }
         C1[t] = acc;
@@ -780,7 +836,7 @@ __device__ void gauss_box(float* aux, int h, int w, const BlurArg& g, Load load,
         float2 v[7];
 #pragma unroll
         for (int q = 0; q < 7; ++q) v[q] = A[t + q * w];
-#pragma unroll 4
+#pragma unroll 8
         for (int r = r0; r < r1; ++r) {
             float2 acc = make_float2(0.f, 0.f);
 #pragma unroll
@@ -856,7 +912,8 @@ __device__ __forceinline__ float sum256(float v, float* red) {
     return t;
 }
 
-// A block a pattern with the image in LDS (row stride S, odd: the tiles' lanes read down the rows),
+// A block a pattern with the image in LDS (row stride S: w, or w + 1 where the lanes of a tile, which
+// read down the rows, would share fewer than 8 of the 64 banks),
 // or, GLOB, in the block's slot of global memory (patterns blockIdx.x, + gridDim.x, ...; S = w) with
 // what is smaller than an image in LDS still. vec: four pixels a load and store (h w a multiple of
 // 4, raw, background and out aligned to four pixels).
@@ -885,10 +942,15 @@ __global__ void __launch_bounds__(NT, 4) k_prep_tiles(const T* __restrict__ raw,
                     const float4 q = *reinterpret_cast<const float4*>(bg + i);
                     x[0] -= q.x, x[1] -= q.y, x[2] -= q.z, x[3] -= q.w;
                 }
+#pragma unroll
+                for (int u = 0; u < 4; ++u) odd |= !(fabsf(x[u]) < 1e30f);
+                if (S == w) {
+                    *reinterpret_cast<float4*>(img + i) = make_float4(x[0], x[1], x[2], x[3]);
+                    continue;
+                }
                 int2 rc = pix_rc(i, w, invw);
 #pragma unroll
                 for (int u = 0; u < 4; ++u) {
-                    odd |= !(fabsf(x[u]) < 1e30f);
                     img[(size_t)rc.x * S + rc.y] = x[u];
                     if (++rc.y == w) {
                         rc.y = 0;
@@ -937,13 +999,14 @@ __global__ void __launch_bounds__(NT, 4) k_prep_tiles(const T* __restrict__ raw,
         }
         float sm = 0.f, cn = 0.f;
         if (tid < 256) {
+            Walk at(tid, w, invw, 256);
 #pragma unroll 4
-            for (int i = tid; i < hw; i += 256) {
-                const int2 rc = pix_rc(i, w, invw);
-                const float v = img[(size_t)rc.x * S + rc.y];
-                const bool in = in_mask((float)rc.x, (float)rc.y, a.mask);
-                sm += in ? v : 0.f;
+            for (int i = tid; i < hw; i += 256, at.next()) {
+                float* p = img + (size_t)at.r * S + at.c;
+                const bool in = in_mask((float)at.r, (float)at.c, a.mask);
+                sm += in ? *p : 0.f;
                 cn += in ? 1.f : 0.f;
+                if (!in) *p = __int_as_float(kOutside);
             }
         }
         sm = sum256(sm, red);
@@ -951,12 +1014,13 @@ __global__ void __launch_bounds__(NT, 4) k_prep_tiles(const T* __restrict__ raw,
         const float mean = sm / fmaxf(cn, 1.f);
         float ss = 0.f;
         if (tid < 256) {
+            Walk at(tid, w, invw, 256);
 #pragma unroll 4
-            for (int i = tid; i < hw; i += 256) {
-                const int2 rc = pix_rc(i, w, invw);
-                const float x = img[(size_t)rc.x * S + rc.y];
-                const float v = in_mask((float)rc.x, (float)rc.y, a.mask) ? x - mean : 0.f;
-                img[(size_t)rc.x * S + rc.y] = v;
+            for (int i = tid; i < hw; i += 256, at.next()) {
+                float* p = img + (size_t)at.r * S + at.c;
+                const float x = *p;
+                const float v = outside(x) ? 0.f : x - mean;
+                *p = v;
                 ss += v * v;
             }
         }
@@ -964,6 +1028,11 @@ __global__ void __launch_bounds__(NT, 4) k_prep_tiles(const T* __restrict__ raw,
         const float inv = 1.f / sqrtf(fmaxf(ss, 1e-30f));
         if (vec) {
             for (int i = 4 * tid; i < hw; i += 4 * NT) {
+                if (S == w) {
+                    const float4 q = *reinterpret_cast<const float4*>(img + i);
+                    *reinterpret_cast<float4*>(dst + i) = make_float4(q.x * inv, q.y * inv, q.z * inv, q.w * inv);
+                    continue;
+                }
                 int2 rc = pix_rc(i, w, invw);
                 float x[4];
 #pragma unroll
@@ -1005,49 +1074,42 @@ __global__ void __launch_bounds__(NT) k_prep_box(const T* __restrict__ raw, cons
         const float x = load(r, c);
         const float y = dyn == 1 ? x - v : x / fmaxf(v, 1e-6f);
         const bool in = in_mask((float)r, (float)c, a.mask);
-        dst[r * w + c] = in ? y : 0.f;
+        dst[r * w + c] = in ? y : __int_as_float(kOutside);
         cn += in ? 1.f : 0.f;
     });
-    if (tid < 256) {
-#pragma unroll 8
-        for (int i = tid; i < hw; i += 256) sm += dst[i];
-    }
+    // (256 threads: 32 pixels' loads in flight before any is added)
+    auto serial = [&](auto add) {
+        if (tid >= 256) return;
+        for (int i = tid; i < hw; i += 256 * 32) {
+            float v[32];
+#pragma unroll
+            for (int u = 0; u < 32; ++u) v[u] = dst[min(i + 256 * u, hw - 1)];
+#pragma unroll
+            for (int u = 0; u < 32; ++u)
+                if (i + 256 * u < hw) add(v[u]);
+        }
+    };
+    serial([&](float x) { sm += outside(x) ? 0.f : x; });
     sm = sum256(sm, red);
     cn = block_sum<NT>(cn, red);
     const float mean = sm / fmaxf(cn, 1.f);
-    const float invw = 1.f / (float)w;
     float ss = 0.f;
-    if (tid < 256) {
-#pragma unroll 8
-        for (int i = tid; i < hw; i += 256) {
-            const int2 rc = pix_rc(i, w, invw);
-            const float x = dst[i];
-            const float v = in_mask((float)rc.x, (float)rc.y, a.mask) ? x - mean : 0.f;
-            ss += v * v;
-        }
-    }
+    serial([&](float x) {
+        const float v = outside(x) ? 0.f : x - mean;
+        ss += v * v;
+    });
     ss = sum256(ss, red);
     const float inv = 1.f / sqrtf(fmaxf(ss, 1e-30f));
+    auto scaled = [&](float x) { return (outside(x) ? 0.f : x - mean) * inv; };
     if (vec) {
+#pragma unroll 4
         for (int i = 4 * tid; i < hw; i += 4 * NT) {
             const float4 q = *reinterpret_cast<const float4*>(dst + i);
-            float x[4] = {q.x, q.y, q.z, q.w};
-            int2 rc = pix_rc(i, w, invw);
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                x[u] = (in_mask((float)rc.x, (float)rc.y, a.mask) ? x[u] - mean : 0.f) * inv;
-                if (++rc.y == w) {
-                    rc.y = 0;
-                    ++rc.x;
-                }
-            }
-            *reinterpret_cast<float4*>(dst + i) = make_float4(x[0], x[1], x[2], x[3]);
+            *reinterpret_cast<float4*>(dst + i) = make_float4(scaled(q.x), scaled(q.y), scaled(q.z), scaled(q.w));
         }
     } else {
-        for (int i = tid; i < hw; i += NT) {
-            const int2 rc = pix_rc(i, w, invw);
-            dst[i] = (in_mask((float)rc.x, (float)rc.y, a.mask) ? dst[i] - mean : 0.f) * inv;
-        }
+#pragma unroll 4
+        for (int i = tid; i < hw; i += NT) dst[i] = scaled(dst[i]);
     }
 }
 
@@ -1291,7 +1353,7 @@ static PrepForm prep_form(const PrepArg& a, bool global, int limit, size_t& lds,
         lds = (size_t)box_words(a.dynb, a.h, a.w) * 4;
         return kPrepBoxes;
     }
-    S = global ? a.w : a.w | 1;
+    S = !global && a.w % 16 == 0 ? a.w + 1 : a.w;
     const long area = global ? 0 : ((long)a.h * S + 3) & ~3L;
     long aux = a.clahe ? (long)a.tiles * a.tiles * (a.bins + 1) : 0;
     auto need = [&](const BlurArg& g) { aux = std::max(aux, g.box ? box_words(g, a.h, a.w) : area + tile_table_words(g.radius, a.h, a.w)); };
