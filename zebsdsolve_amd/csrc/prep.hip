@@ -553,9 +553,9 @@ __global__ void __launch_bounds__(256) k_prep_g(const T* __restrict__ raw, const
 //   are read for the boxes and again (from L2) where the background is subtracted (k_prep_box).
 // - the sums of the normalization stay on 256 threads, pixel i on thread i mod 256.
 // Blocks of 256 threads to 4 096 pixels, 512 to 16 384, 1 024 beyond.
-// 5 003 patterns of 60 x 60 in u8, the direct background: 436 -> 117 us; 160 of 240 x 320 in u16, by
-// boxes: 967 -> 100; 1 001 of 75 x 83 through background, CLAHE and band pass: 1 128 -> 315; 1 200 of
-// 120 x 120 in u16, by boxes: 870 -> 143. The outputs are the same bit for bit. (With the taps and sums
+// 5 003 patterns of 60 x 60 in u8, the direct background: 436 -> 100 us; 160 of 240 x 320 in u16, by
+// boxes: 967 -> 99; 1 001 of 75 x 83 through background, CLAHE and band pass: 1 128 -> 208; 1 200 of
+// 120 x 120 in u16, by boxes: 870 -> 131. The outputs are the same bit for bit. (With the taps and sums
 // in another order the first three took 139, 86 and 228 us, but pixels a last bit away moved NMI bins:
 // a record's NMI by up to 0.5 %, and one cell of 6 035 past its acceptance.)
 
@@ -712,7 +712,7 @@ __device__ void gauss_tiles(const float* img, int S, float* P, float* tab, int h
 // counts, then in turn the boxes, the cells along the rows and the coarse weights, or each column's
 // cells [hp][w].
 __host__ __device__ inline long box_words(const BlurArg& g, int h, int w) {
-    const long coarse = 2L * g.hs * g.wp + (long)g.hs * g.ws + (long)g.wp * g.nbx + (long)g.hp * g.nby;
+    const long coarse = (g.hs + 2L) * g.wp + (long)g.hs * g.ws + (long)g.wp * g.nbx + (long)g.hp * g.nby;
     const long spread = 2L * g.hp * w;
     return 2L * g.hp * g.wp + 7L * w + 7L * h + 1 + (coarse > spread ? coarse : spread);
 }
@@ -726,11 +726,12 @@ __device__ void gauss_box(float* aux, int h, int w, const BlurArg& g, Load load,
     float2* C2 = reinterpret_cast<float2*>(aux);                              // [hp][wp]
     float* ex = aux + 2 * hp * wp;                                            // [w][7]
     float* ey = ex + 7 * w;                                                   // [h][7]
-    float2* C1 = reinterpret_cast<float2*>(aux + ((2 * hp * wp + 7 * w + 7 * h + 1) & ~1));  // [hs][wp]
-    float* C0 = reinterpret_cast<float*>(C1 + hs * wp);                       // [hs][ws]
+    float2* A = reinterpret_cast<float2*>(aux + ((2 * hp * wp + 7 * w + 7 * h + 1) & ~1));  // [hp][w], after:
+    float* C1 = reinterpret_cast<float*>(A);                                  // [hs][wp]
+    float* N1 = C1 + hs * wp;                                                 // [2][wp] counts: whole lines, the last
+    float* C0 = N1 + 2 * wp;                                                  // [hs][ws]
     float* kx = C0 + hs * ws;                                                 // [wp][nbx]
     float* ky = kx + wp * g.nbx;                                              // [hp][nby]
-    float2* A = C1;                                                           // [hp][w]
     const float fs = (float)s;
     auto first = [&](float cc) { return max((int)floorf((cc - g.reach) / fs), 0); };
     auto last = [&](float cc, int cells) { return min((int)floorf((cc + g.reach) / fs), cells - 1); };
@@ -782,23 +783,40 @@ __device__ void gauss_box(float* aux, int h, int w, const BlurArg& g, Load load,
         ex[t] = cw.y * expf(-d * d * g.k2);
     }
     __syncthreads();
-    // along the rows onto the coarse grid with its margin: [hs][wp]
-    for (int t = tid; t < hs * wp; t += NT) {
-        const int line = t / wp, tc = t - line * wp;
+    // along the rows onto the coarse grid with its margin, [hs][wp], four lines a thread (one weight
+    // for the four); the counts are of two kinds of line, whole ones and the last
+    const int groups = (hs + 3) >> 2;
+    for (int t = tid; t < (groups + 2) * wp; t += NT) {
+        const int group = t / wp, tc = t - group * wp;
         const float cc = prep_cell(tc - pad, w, s).x;
         const int j0 = first(cc), j1 = last(cc, ws);
         const float* k = kx + tc * g.nbx - j0;
-        const float* v = C0 + line * ws;
-        // the boxes' counts: all of a line alike but the last
-        const int rows = min((line + 1) * s, h) - line * s;
-        const float whole = (float)(rows * s), rest = (float)(rows * (w - (ws - 1) * s));
-        float2 acc = make_float2(0.f, 0.f);
+        if (group < groups) {
+            const int l0 = 4 * group;
+            const float* v0 = C0 + l0 * ws;
+            const float* v1 = C0 + min(l0 + 1, hs - 1) * ws;
+            const float* v2 = C0 + min(l0 + 2, hs - 1) * ws;
+            const float* v3 = C0 + min(l0 + 3, hs - 1) * ws;
+            float acc[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
-        for (int j = j0; j <= j1; ++j) {
-            const float n = j < ws - 1 ? whole : rest;
-            acc = make_float2(acc.x + k[j] * v[j], acc.y + k[j] * n);
+            for (int j = j0; j <= j1; ++j) {
+                const float q = k[j];
+                acc[0] = acc[0] + q * v0[j];
+                acc[1] = acc[1] + q * v1[j];
+                acc[2] = acc[2] + q * v2[j];
+                acc[3] = acc[3] + q * v3[j];
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (l0 + u < hs) C1[(l0 + u) * wp + tc] = acc[u];
+        } else {
+            const int rows = group == groups ? s : h - (hs - 1) * s;
+            const float whole = (float)(rows * s), rest = (float)(rows * (w - (ws - 1) * s));
+            float acc = 0.f;
+#pragma unroll 4
+            for (int j = j0; j <= j1; ++j) acc = acc + k[j] * (j < ws - 1 ? whole : rest);
+            N1[(group - groups) * wp + tc] = acc;
         }
-        C1[t] = acc;
     }
     __syncthreads();
     // along the columns: [hp][wp]
@@ -807,12 +825,11 @@ __device__ void gauss_box(float* aux, int h, int w, const BlurArg& g, Load load,
         const float cc = prep_cell(tr - pad, h, s).x;
         const int i0 = first(cc), i1 = last(cc, hs);
         const float* k = ky + tr * g.nby - i0;
+        const float* v = C1 + col;
+        const float whole = N1[col], rest = N1[wp + col];
         float2 acc = make_float2(0.f, 0.f);
 #pragma unroll 4
-        for (int i = i0; i <= i1; ++i) {
-            const float2 v = C1[i * wp + col];
-            acc = make_float2(acc.x + k[i] * v.x, acc.y + k[i] * v.y);
-        }
+        for (int i = i0; i <= i1; ++i) acc = make_float2(acc.x + k[i] * v[i * wp], acc.y + k[i] * (i < hs - 1 ? whole : rest));
         C2[t] = acc;
     }
     __syncthreads();
@@ -917,8 +934,8 @@ __device__ __forceinline__ float sum256(float v, float* red) {
 // or, GLOB, in the block's slot of global memory (patterns blockIdx.x, + gridDim.x, ...; S = w) with
 // what is smaller than an image in LDS still. vec: four pixels a load and store (h w a multiple of
 // 4, raw, background and out aligned to four pixels).
-template <typename T, int NT, bool GLOB>
-__global__ void __launch_bounds__(NT, 4) k_prep_tiles(const T* __restrict__ raw, const float* __restrict__ bg, PrepArg a, int n, int S, int vec,
+template <typename T, int NT, bool GLOB, bool FULL>
+__global__ void __launch_bounds__(NT, FULL ? 4 : 5) k_prep_tiles(const T* __restrict__ raw, const float* __restrict__ bg, PrepArg a, int n, int S, int vec,
                                                    float* __restrict__ work, long slot, float* __restrict__ out) {
     extern __shared__ double lds64[];
     __shared__ float red[2 * NT / 64];
@@ -971,7 +988,7 @@ __global__ void __launch_bounds__(NT, 4) k_prep_tiles(const T* __restrict__ raw,
         // output row, its fine one less that. One copy of the code for the three.
 #pragma unroll 1
         for (int stage = 0; stage < 3; ++stage) {
-            if (stage == 1 && a.clahe) clahe_tiles<NT>(img, S, reinterpret_cast<unsigned*>(near), a, red);
+            if (FULL && stage == 1 && a.clahe) clahe_tiles<NT>(img, S, reinterpret_cast<unsigned*>(near), a, red);
             if (!(stage == 0 ? a.dyn : stage == 1 ? a.bp : a.bp && a.bp_fine)) continue;
             const BlurArg g = stage == 0 ? a.dynb : stage == 1 ? a.coarse : a.fine;
             auto emit = [&](int r, int c, float v) {
@@ -983,7 +1000,7 @@ __global__ void __launch_bounds__(NT, 4) k_prep_tiles(const T* __restrict__ raw,
                 else
                     *p = v - dst[r * w + c];
             };
-            if (g.box)
+            if (FULL && g.box)
                 gauss_box<NT>(near, h, w, g, [&](int r, int c) { return img[(size_t)r * S + c]; }, emit);
             else if (loops)
                 gauss<NT>(img, P, h, w, S, g, emit);
@@ -1372,8 +1389,11 @@ static void prep_launch(const void* raw_, const float* bg, const PrepArg& a, int
     const T* raw = (const T*)raw_;
     const long hw = (long)a.h * a.w;
     const int vec = hw % 4 == 0 && (uintptr_t)raw % (4 * sizeof(T)) == 0 && (uintptr_t)out % 16 == 0 && (uintptr_t)bg % 16 == 0;
-#define ZB_TILES(NT, G, GRID) \
-    ZB_LAUNCH("k_prep", (k_prep_tiles<T, NT, G>), dim3(GRID), dim3(NT), lds, s, raw, bg, a, n, S, vec, work, slot, out)
+#define ZB_TILES(NT, G, F, GRID) \
+    ZB_LAUNCH("k_prep", (k_prep_tiles<T, NT, G, F>), dim3(GRID), dim3(NT), lds, s, raw, bg, a, n, S, vec, work, slot, out)
+    // without CLAHE and box sums the code for them is left out (its registers hold 60 x 60 to four blocks
+    // a CU where LDS allows five)
+    const bool full = a.clahe || (a.dyn && a.dynb.box) || (a.bp && (a.coarse.box || (a.bp_fine && a.fine.box)));
     if (form == kPrepBoxes && hw <= 16384)
         ZB_LAUNCH("k_prep", (k_prep_box<T, 512>), dim3(n), dim3(512), lds, s, raw, bg, a, vec, out);
     else if (form == kPrepBoxes)
@@ -1383,17 +1403,19 @@ static void prep_launch(const void* raw_, const float* bg, const PrepArg& a, int
     else if (form == kPrepLoops)
         ZB_LAUNCH("k_prep", k_prep<T>, dim3(n), dim3(256), lds, s, raw, bg, a, out);
     else if (form == kPrepTilesG && hw <= 4096)
-        ZB_TILES(256, true, grid);
+        ZB_TILES(256, true, true, grid);
     else if (form == kPrepTilesG && hw <= 16384)
-        ZB_TILES(512, true, grid);
+        ZB_TILES(512, true, true, grid);
     else if (form == kPrepTilesG)
-        ZB_TILES(1024, true, grid);
+        ZB_TILES(1024, true, true, grid);
+    else if (hw <= 4096 && !full)
+        ZB_TILES(256, false, false, n);
     else if (hw <= 4096)
-        ZB_TILES(256, false, n);
+        ZB_TILES(256, false, true, n);
     else if (hw <= 16384)
-        ZB_TILES(512, false, n);
+        ZB_TILES(512, false, true, n);
     else
-        ZB_TILES(1024, false, n);
+        ZB_TILES(1024, false, true, n);
 #undef ZB_TILES
 }
 
