@@ -12,6 +12,8 @@
 //   k_legendre a_lm = sum_y wplm[y, pair] (sum or difference by the parity of l + m): per order
 //              m and tile of 16 items, two GEMMs on the matrix cores (one per parity)
 //   k_norm     unit harmonic norm and the item's stats
+// The window covers some fifth of the sphere: k_sums notes the ring pairs with a sample in it, and the
+// later stages leave the others out (their samples and spectra are zeros).
 // Workspace: per item the window sums (float2), and the ring spectra [L][items][n/2] float4
 // (order-major, so that a k_legendre block's items lie side by side, not a power-of-two stride
 // apart).
@@ -101,11 +103,27 @@ __device__ __forceinline__ void sample_pair(const SphArg& a, const ItemGeom& g, 
     south = sample_dir(a, g, h2 - z2, h0 - z0, h1 - z1);
 }
 
+// The first and one past the last ring pair of an item with a sample in the window: the spectra of the
+// pairs outside are neither written nor read. k_sums leaves the two numbers where the item's four
+// stats go, which k_norm writes at the end.
+__device__ __forceinline__ int2 live_range(const int* live, int item) { return make_int2(live[4 * (size_t)item], live[4 * (size_t)item + 1]); }
+
+// The range that holds those of a wave's lanes.
+__device__ __forceinline__ int2 wave_range(int2 r) {
+    for (int o = 1; o < 64; o <<= 1) {
+        r.x = min(r.x, __shfl_xor(r.x, o, 64));
+        r.y = max(r.y, __shfl_xor(r.y, o, 64));
+    }
+    return make_int2(__builtin_amdgcn_readfirstlane(r.x), __builtin_amdgcn_readfirstlane(r.y));
+}
+
 // Per item: sum of w wq value and of w wq over its whole grid (sphere.wgsl:114-151). Each thread
 // keeps grid columns (phi) and walks the ring pairs (y, n - 1 - y), whose weights are equal.
 __global__ void __launch_bounds__(256) k_sums(SphArg a, const float* __restrict__ ring, const float2* __restrict__ tw,
-                                              const float* __restrict__ pats, const float4* __restrict__ items, float2* __restrict__ sums) {
+                                              const float* __restrict__ pats, const float4* __restrict__ items, float2* __restrict__ sums,
+                                              int* __restrict__ live) {
     __shared__ float2 red[4];
+    __shared__ int2 seen[4];
     __shared__ float4 rt[ZB_TW / 4];  // the ring pairs' entries (n / 2 <= ZB_TW / 4)
     const int b = blockIdx.x;
     const ItemGeom g = item_geom(a, pats, items[b]);
@@ -117,25 +135,36 @@ __global__ void __launch_bounds__(256) k_sums(SphArg a, const float* __restrict_
     for (int y = tid; y < nh; y += 256) rt[y] = ring_entry(ring, y);
     __syncthreads();
     float sv = 0.f, sw = 0.f;
+    // a wave's lanes share y (64 columns at least, else every pair counts as live)
+    const bool alike = cols >= 64;
+    int2 on = alike ? make_int2(nh, 0) : make_int2(0, nh);
+    const int yfirst = alike ? __builtin_amdgcn_readfirstlane(tid / cols) : tid / cols;
     for (int j = tid % cols; j < nphi; j += cols) {
         const ColGeom cg = col_geom(a, tw[j << (10 - a.log2nphi)]);
-        for (int y = tid / cols; y < nh; y += rows) {
+        for (int y = yfirst; y < nh; y += rows) {
             float2 gn, gs;
             const float4 r = rt[y];
             sample_pair(a, g, cg, r.x, r.y, gn, gs);
             const float wq = r.z;
             sv += (gn.x * gn.y + gs.x * gs.y) * wq;
             sw += (gn.y + gs.y) * wq;
+            if (__ballot(gn.y + gs.y != 0.f)) on = make_int2(min(on.x, y), max(on.y, y + 1));
         }
     }
     sv = warp_sum(sv);
     sw = warp_sum(sw);
-    if ((tid & 63) == 0) red[tid >> 6] = make_float2(sv, sw);
+    if ((tid & 63) == 0) {
+        red[tid >> 6] = make_float2(sv, sw);
+        seen[tid >> 6] = on;
+    }
     __syncthreads();
     if (tid == 0) {
         float2 t = red[0];
         for (int i = 1; i < 4; ++i) t = make_float2(t.x + red[i].x, t.y + red[i].y);
         sums[b] = t;
+        for (int i = 0; i < 4; ++i) on = make_int2(min(on.x, seen[i].x), max(on.y, seen[i].y));
+        live[4 * (size_t)b] = on.x;
+        live[4 * (size_t)b + 1] = on.y;
     }
 }
 
@@ -149,14 +178,22 @@ __device__ __forceinline__ float window_mean(const SphArg& a, float2 tot) {
 template <int LOG2NPHI>
 __global__ void __launch_bounds__(256) k_rings(SphArg a, int G, const float* __restrict__ ring, const float2* __restrict__ tw,
                                                const float* __restrict__ pats, const float4* __restrict__ items,
-                                               const float2* __restrict__ sums, float4* __restrict__ spectra) {
+                                               const float2* __restrict__ sums, const int* __restrict__ live, float4* __restrict__ spectra) {
     extern __shared__ float2 buf[];  // [G][nphi] lines, then the group's G ring entries
     if constexpr (LOG2NPHI > 0) a.log2nphi = LOG2NPHI;
     const int nh = a.n >> 1;
     const int groups = nh / G;
     const int b = blockIdx.x / groups;
-    const int y0 = (blockIdx.x - b * groups) * G;
+    // (an item's groups rotated by the item: blocks are dealt to the 8 XCDs in turn, so one group of
+    // every item, empty or not, would fall to one XCD)
+    const int y0 = ((blockIdx.x - b * groups + b) & (groups - 1)) * G;
     const int nphi = 1 << a.log2nphi;
+    const int lg = __builtin_ctz((unsigned)G);  // G is a power of two
+    const int n_items = gridDim.x / groups;
+    // nothing of these rings in the window: 2 groups in 8 at L = 64, the detector tilted 70 degrees and
+    // half a frame from its centre to its edge at the distance 0.55
+    const int2 on = live_range(live, b);
+    if (y0 >= on.y || y0 + G <= on.x) return;
     float4* rt = reinterpret_cast<float4*>(buf + G * nphi);
     for (int i = threadIdx.x; i < G; i += 256) rt[i] = ring_entry(ring, y0 + i);
     __syncthreads();
@@ -181,8 +218,6 @@ __global__ void __launch_bounds__(256) k_rings(SphArg a, int G, const float* __r
         fft_dif<256>(buf, a.log2nphi, G, nphi, 1, tw, threadIdx.x);
     // Z = N + i S for real N, S: N_m = (Z_m + conj Z_{-m}) / 2, S_m = (Z_m - conj Z_{-m}) / 2i
     const int L = a.L;
-    const int lg = __builtin_ctz((unsigned)G);  // G is a power of two
-    const int n_items = gridDim.x / groups;
     for (int e = threadIdx.x; e < G * L; e += 256) {
         const int m = e >> lg;
         const int i = e & (G - 1);
@@ -202,7 +237,7 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 // v_mfma_f32_32x32x2_f32: A lane -> (row lane % 32, k lane / 32), B lane -> (k lane / 32,
 // column lane % 32), C register r -> (row (r / 4) 8 + (lane / 32) 4 + r % 4, column lane % 32).
 __global__ void __launch_bounds__(64) k_legendre(SphArg a, int n_items, const float* __restrict__ wplm, const float4* __restrict__ spectra,
-                                                 float2* __restrict__ alm) {
+                                                 const int* __restrict__ live, float2* __restrict__ alm) {
     const int lane = threadIdx.x;
     const int half = lane >> 5;
     const int r32 = lane & 31;
@@ -216,6 +251,9 @@ __global__ void __launch_bounds__(64) k_legendre(SphArg a, int n_items, const fl
     const bool im = (r32 & 1) != 0;
     const bool iok = item < n_items;
     const float4* sp = spectra + ((size_t)m * n_items + (iok ? item : 0)) * nh;
+    const int2 own = iok ? live_range(live, item) : make_int2(nh, 0);
+    const int2 on = wave_range(own);
+    const unsigned own_n = (unsigned)max(own.y - own.x, 0);
     const int ncol = (L - m + 1) / 2;  // degrees l = m, m + 2, ...
     for (int ct = 0; ct * 32 < ncol; ++ct) {
         const int le = m + 2 * (ct * 32 + r32);  // this lane's column: even l + m
@@ -223,9 +261,10 @@ __global__ void __launch_bounds__(64) k_legendre(SphArg a, int n_items, const fl
         floatx16 ce, co;
 #pragma unroll
         for (int r = 0; r < 16; ++r) ce[r] = co[r] = 0.f;
-        for (int ks = 0; ks < nh / 2; ++ks) {
+        for (int ks = on.x >> 1; ks < (on.y + 1) >> 1; ++ks) {
             const int y = 2 * ks + half;
-            const float4 v = iok ? sp[y] : make_float4(0.f, 0.f, 0.f, 0.f);
+            float4 v = sp[y];
+            if ((unsigned)(y - own.x) >= own_n) v = make_float4(0.f, 0.f, 0.f, 0.f);
             const float* wy = wplm + (size_t)y * a.pairs + base;
             const float be = le < L ? wy[le] : 0.f;
             const float bo = lo < L ? wy[lo] : 0.f;
@@ -270,8 +309,8 @@ struct Leg16<true> {
 };
 
 template <bool BF>
-__global__ void __launch_bounds__(64) k_legendre16(SphArg a, int n_items, int split, const float* __restrict__ wplm,
-                                                   const float4* __restrict__ spectra, float2* __restrict__ alm) {
+__global__ void __launch_bounds__(64, 3) k_legendre16(SphArg a, int n_items, int split, const float* __restrict__ wplm,
+                                                   const float4* __restrict__ spectra, const int* __restrict__ live, float2* __restrict__ alm) {
     typedef typename Leg16<BF>::T T;
     typedef typename Leg16<BF>::V8 V8;
     const int lane = threadIdx.x;
@@ -286,6 +325,9 @@ __global__ void __launch_bounds__(64) k_legendre16(SphArg a, int n_items, int sp
     const bool im = (r32 & 1) != 0;
     const bool iok = item < n_items;
     const float4* sp = spectra + ((size_t)m * n_items + (iok ? item : 0)) * nh;
+    const int2 own = iok ? live_range(live, item) : make_int2(nh, 0);
+    const int2 on = wave_range(own);
+    const unsigned own_n = (unsigned)max(own.y - own.x, 0);
     const int ncol = (L - m + 1) / 2;
     constexpr float kScale = BF ? 1.f : 4096.f;
     for (int ct = 0; ct * 32 < ncol; ++ct) {
@@ -296,12 +338,13 @@ __global__ void __launch_bounds__(64) k_legendre16(SphArg a, int n_items, int sp
         floatx16 ce, co;
 #pragma unroll
         for (int r = 0; r < 16; ++r) ce[r] = co[r] = 0.f;
-        for (int ks = 0; ks < nh / 16; ++ks) {
+        for (int ks = on.x >> 4; ks < (on.y + 15) >> 4; ++ks) {
             V8 aeh, aol, ael, aoh, beh, bel, boh, bol;
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 const int y = 16 * ks + 8 * half + i;
-                const float4 v = iok ? sp[y] : make_float4(0.f, 0.f, 0.f, 0.f);
+                float4 v = sp[y];
+                if ((unsigned)(y - own.x) >= own_n) v = make_float4(0.f, 0.f, 0.f, 0.f);
                 const float xe = im ? v.y : v.x, xo = im ? v.w : v.z;
                 const float* wy = wplm + (size_t)y * a.pairs + base;
                 const float we = le < L ? kScale * wy[le] : 0.f, wo = lo < L ? kScale * wy[lo] : 0.f;
@@ -518,9 +561,10 @@ static int32_t sh_run(const zb_band* band, const zb_frame* frame, const float* p
     char* ws = work;
     float2* sums = (float2*)ws;
     float4* spectra = (float4*)(ws + ((int64_t)n_items * 8 + 255) / 256 * 256);
+    int* live = (int*)stats;
     const float2* tw = (const float2*)band->twiddle;
     const float4* its = (const float4*)items;
-    ZB_LAUNCH("k_sums", k_sums, dim3(n_items), dim3(256), 0, s, a, band->ring, tw, pats, its, sums);
+    ZB_LAUNCH("k_sums", k_sums, dim3(n_items), dim3(256), 0, s, a, band->ring, tw, pats, its, sums, live);
     if (int rc = check_launch("zb_sh_coefficients/sums")) return rc;
     const int nh = n / 2;
     const int nphi = 2 * n;
@@ -534,26 +578,26 @@ static int32_t sh_run(const zb_band* band, const zb_frame* frame, const float* p
     const dim3 rgrid(n_items * (nh / G));
     const size_t rlds = (size_t)G * nphi * 8 + (size_t)G * 16;
     if (a.log2nphi == 7)
-        ZB_LAUNCH("k_rings", k_rings<7>, rgrid, dim3(256), rlds, s, a, G, band->ring, tw, pats, its, (const float2*)sums, spectra);
+        ZB_LAUNCH("k_rings", k_rings<7>, rgrid, dim3(256), rlds, s, a, G, band->ring, tw, pats, its, (const float2*)sums, (const int*)live, spectra);
     else if (a.log2nphi == 8)
-        ZB_LAUNCH("k_rings", k_rings<8>, rgrid, dim3(256), rlds, s, a, G, band->ring, tw, pats, its, (const float2*)sums, spectra);
+        ZB_LAUNCH("k_rings", k_rings<8>, rgrid, dim3(256), rlds, s, a, G, band->ring, tw, pats, its, (const float2*)sums, (const int*)live, spectra);
     else if (a.log2nphi == 9)
-        ZB_LAUNCH("k_rings", k_rings<9>, rgrid, dim3(256), rlds, s, a, G, band->ring, tw, pats, its, (const float2*)sums, spectra);
+        ZB_LAUNCH("k_rings", k_rings<9>, rgrid, dim3(256), rlds, s, a, G, band->ring, tw, pats, its, (const float2*)sums, (const int*)live, spectra);
     else
-        ZB_LAUNCH("k_rings", k_rings<0>, rgrid, dim3(256), rlds, s, a, G, band->ring, tw, pats, its, (const float2*)sums, spectra);
+        ZB_LAUNCH("k_rings", k_rings<0>, rgrid, dim3(256), rlds, s, a, G, band->ring, tw, pats, its, (const float2*)sums, (const int*)live, spectra);
     if (int rc = check_launch("zb_sh_coefficients/rings")) return rc;
     if ((flags & (ZB_FLAG_FP16 | ZB_FLAG_BF16)) && nh >= 16) {
         // 16-bit products, 16 rings a product (below n = 32 the FP32 sums stand in)
         const int split = (flags >> ZB_FLAG_SPLIT_SHIFT) & 0xff;
         if (flags & ZB_FLAG_BF16)
             ZB_LAUNCH("k_legendre", k_legendre16<true>, dim3((n_items + 15) / 16, L), dim3(64), 0, s, a, n_items, split, band->wplm,
-                      (const float4*)spectra, (float2*)alm);
+                      (const float4*)spectra, (const int*)live, (float2*)alm);
         else
             ZB_LAUNCH("k_legendre", k_legendre16<false>, dim3((n_items + 15) / 16, L), dim3(64), 0, s, a, n_items, split, band->wplm,
-                      (const float4*)spectra, (float2*)alm);
+                      (const float4*)spectra, (const int*)live, (float2*)alm);
     } else {
         ZB_LAUNCH("k_legendre", k_legendre, dim3((n_items + 15) / 16, L), dim3(64), 0, s, a, n_items, band->wplm, (const float4*)spectra,
-                  (float2*)alm);
+                  (const int*)live, (float2*)alm);
     }
     if (int rc = check_launch("zb_sh_coefficients/legendre")) return rc;
     if (a.pairs <= 256 * 10)
