@@ -394,44 +394,78 @@ __device__ void fft_dif(float2* buf, int log2n, int nlines, int lstride, int pst
     }
 }
 
-// fft_dif for contiguous lines (pstride 1, lstride 2^LOG2N) of a size known at compile time:
-// the same butterflies in the same order (bit-identical results), with the stage sizes, strides
-// and twiddle steps constants, so that the index arithmetic folds away.
+// fft_dif for lines of a size known at compile time, 2^7 to 2^9: the same butterflies in the same order
+// (bit-identical results), with the stage sizes, strides and twiddle steps constants, so that the
+// index arithmetic folds away.
+//
+// Every stage of a line of 2^k points meets powers of two, and so few of the 64 LDS banks (4-way
+// conflicts in the stages, 32-way in the bit-reversed gather after them: two thirds of the LDS
+// cycles of a kernel that LDS bound). So point p sits at fft_at(p) = p + p / 64, a line takes
+// fft_line<LOG2N> = 2^LOG2N + 2^LOG2N / 64 points, and neighbouring threads take neighbouring lines
+// and then F = 2^LOG2N / 64 butterflies of one, neighbours or (where q < F) an eighth of the line or
+// so apart: with 32 / F lines 32 threads meet every bank once. With p's digits disjoint fft_at adds
+// up, so the four points of a butterfly stay a constant apart.
+// (The ring transforms at L = 64, 3 001 items: conflicts 44 of 67 M LDS cycles, k_rings 186 us; 18 of 41
+// and 145 with the padding, the vector units busy for 115 of them.)
+__host__ __device__ constexpr int fft_at(int p) { return p + (p >> 6); }
+template <int LOG2N>
+constexpr int fft_line = fft_at(1 << LOG2N);
+
+// The butterfly (of 2^BITS of a line) that index rr takes in a stage of step 2^LQ.
+template <int LOG2N, int BITS, int LQ>
+__device__ __forceinline__ int fft_turn(int rr) {
+    constexpr int LF = LOG2N - 6;  // log2 F
+    if constexpr (LQ >= LF) {
+        return rr;
+    } else {
+        const int j = rr & ((1 << LQ) - 1), top = (rr >> LQ) & ((1 << (LF - LQ)) - 1), rest = rr >> LF;
+        return (top << (BITS - (LF - LQ))) | (rest << LQ) | j;
+    }
+}
+
+// d w and -i d w, each component's fused product named (left to the compiler, which of the two is fused
+// changes with the code around it, and the last bits of the harmonics with it)
+__device__ __forceinline__ float2 twist(float2 d, float2 w) {
+    return make_float2(__builtin_fmaf(w.x, d.x, -(w.y * d.y)), __builtin_fmaf(w.y, d.x, w.x * d.y));
+}
+__device__ __forceinline__ float2 twist_mi(float2 d, float2 w) {
+    return make_float2(__builtin_fmaf(w.y, d.x, w.x * d.y), __builtin_fmaf(w.y, d.y, -(w.x * d.x)));
+}
+
 template <int NT, int LOG2N, int S>
-__device__ __forceinline__ void fft_dif_stages(float2* buf, int nlines, const float2* __restrict__ tw, int tid) {
+__device__ __forceinline__ void fft_dif_stages(float2* buf, int lg_lines, const float2* __restrict__ tw, int tid) {
+    const int lmask = (1 << lg_lines) - 1;
     if constexpr (S >= 2) {
-        constexpr int lq = S - 2, q = 1 << lq, nq = 1 << (LOG2N - 2);
+        constexpr int lq = S - 2, q = 1 << lq;
         constexpr int t4 = ZB_TW >> S, t2 = ZB_TW >> (S - 1);
-        const int total = nlines * nq;
+        const int total = 1 << (lg_lines + LOG2N - 2);
         for (int e = tid; e < total; e += NT) {
-            const int line = e >> (LOG2N - 2);
-            const int r = e & (nq - 1);
+            const int line = e & lmask;
+            const int r = fft_turn<LOG2N, LOG2N - 2, lq>(e >> lg_lines);
             const int j = r & (q - 1);
-            float2* b = buf + (line << LOG2N) + ((r >> lq) << S) + j;
+            float2* b = buf + line * fft_line<LOG2N> + fft_at(((r >> lq) << S) + j);
             float2 x0 = b[0];
-            float2 x1 = b[q];
-            float2 x2 = b[2 * q];
-            float2 x3 = b[3 * q];
+            float2 x1 = b[fft_at(q)];
+            float2 x2 = b[fft_at(2 * q)];
+            float2 x3 = b[fft_at(3 * q)];
             float2 w4 = tw[j * t4];
             float2 w2 = tw[j * t2];
             float2 a0 = cadd(x0, x2);
-            float2 a2 = cmul(csub(x0, x2), w4);
+            float2 a2 = twist(csub(x0, x2), w4);
             float2 a1 = cadd(x1, x3);
-            float2 a3 = cmul(cmul_mi(csub(x1, x3)), w4);
+            float2 a3 = twist_mi(csub(x1, x3), w4);
             b[0] = cadd(a0, a1);
-            b[q] = cmul(csub(a0, a1), w2);
-            b[2 * q] = cadd(a2, a3);
-            b[3 * q] = cmul(csub(a2, a3), w2);
+            b[fft_at(q)] = twist(csub(a0, a1), w2);
+            b[fft_at(2 * q)] = cadd(a2, a3);
+            b[fft_at(3 * q)] = twist(csub(a2, a3), w2);
         }
         __syncthreads();
-        fft_dif_stages<NT, LOG2N, S - 2>(buf, nlines, tw, tid);
+        fft_dif_stages<NT, LOG2N, S - 2>(buf, lg_lines, tw, tid);
     } else if constexpr (S == 1) {
-        constexpr int half = 1 << (LOG2N - 1);
-        const int total = nlines * half;
+        const int total = 1 << (lg_lines + LOG2N - 1);
         for (int e = tid; e < total; e += NT) {
-            const int line = e >> (LOG2N - 1);
-            const int r = e & (half - 1);
-            float2* b = buf + (line << LOG2N) + 2 * r;
+            const int line = e & lmask;
+            float2* b = buf + line * fft_line<LOG2N> + fft_at(2 * fft_turn<LOG2N, LOG2N - 1, 0>(e >> lg_lines));
             float2 x0 = b[0];
             float2 x1 = b[1];
             b[0] = cadd(x0, x1);
@@ -441,9 +475,11 @@ __device__ __forceinline__ void fft_dif_stages(float2* buf, int nlines, const fl
     }
 }
 
+// 2^lg_lines lines, fft_line points apart.
 template <int NT, int LOG2N>
-__device__ void fft_dif_fixed(float2* buf, int nlines, const float2* __restrict__ tw, int tid) {
-    fft_dif_stages<NT, LOG2N, LOG2N>(buf, nlines, tw, tid);
+__device__ void fft_dif_fixed(float2* buf, int lg_lines, const float2* __restrict__ tw, int tid) {
+    static_assert(LOG2N >= 7 && LOG2N <= 9, "fft_at pads for 128 to 512 points");
+    fft_dif_stages<NT, LOG2N, LOG2N>(buf, lg_lines, tw, tid);
 }
 
 // zb_sums with the items taken in `order` (or NULL) and, unit, each pose's quaternion made a unit one;

@@ -194,7 +194,11 @@ __global__ void __launch_bounds__(256) k_rings(SphArg a, int G, const float* __r
     // half a frame from its centre to its edge at the distance 0.55
     const int2 on = live_range(live, b);
     if (y0 >= on.y || y0 + G <= on.x) return;
-    float4* rt = reinterpret_cast<float4*>(buf + G * nphi);
+    // a line's points in LDS: padded for the lengths known here (fft_at)
+    int stride = nphi;
+    if constexpr (LOG2NPHI > 0) stride = fft_line<LOG2NPHI>;
+    auto at = [&](int i, int p) -> float2& { return buf[i * stride + (LOG2NPHI > 0 ? fft_at(p) : p)]; };
+    float4* rt = reinterpret_cast<float4*>(buf + G * stride);
     for (int i = threadIdx.x; i < G; i += 256) rt[i] = ring_entry(ring, y0 + i);
     __syncthreads();
     const ItemGeom g = item_geom(a, pats, items[b]);
@@ -208,12 +212,12 @@ __global__ void __launch_bounds__(256) k_rings(SphArg a, int G, const float* __r
             float2 gn, gs;
             const float4 r = rt[i];
             sample_pair(a, g, cg, r.x, r.y, gn, gs);
-            buf[i * nphi + j] = make_float2((gn.x - mean) * gn.y, (gs.x - mean) * gs.y);
+            at(i, j) = make_float2((gn.x - mean) * gn.y, (gs.x - mean) * gs.y);
         }
     }
     __syncthreads();
     if constexpr (LOG2NPHI > 0)
-        fft_dif_fixed<256, LOG2NPHI>(buf, G, tw, threadIdx.x);
+        fft_dif_fixed<256, LOG2NPHI>(buf, lg, tw, threadIdx.x);
     else
         fft_dif<256>(buf, a.log2nphi, G, nphi, 1, tw, threadIdx.x);
     // Z = N + i S for real N, S: N_m = (Z_m + conj Z_{-m}) / 2, S_m = (Z_m - conj Z_{-m}) / 2i
@@ -221,8 +225,8 @@ __global__ void __launch_bounds__(256) k_rings(SphArg a, int G, const float* __r
     for (int e = threadIdx.x; e < G * L; e += 256) {
         const int m = e >> lg;
         const int i = e & (G - 1);
-        const float2 z = buf[i * nphi + bitrev(m, a.log2nphi)];
-        const float2 zr = buf[i * nphi + bitrev((nphi - m) & (nphi - 1), a.log2nphi)];
+        const float2 z = at(i, bitrev(m, a.log2nphi));
+        const float2 zr = at(i, bitrev((nphi - m) & (nphi - 1), a.log2nphi));
         const float2 rn = make_float2(0.5f * (z.x + zr.x), 0.5f * (z.y - zr.y));
         const float2 rs = make_float2(0.5f * (z.y + zr.y), -0.5f * (z.x - zr.x));
         spectra[((size_t)m * n_items + b) * nh + y0 + i] = make_float4(rn.x + rs.x, rn.y + rs.y, rn.x - rs.x, rn.y - rs.y);
@@ -576,7 +580,8 @@ static int32_t sh_run(const zb_band* band, const zb_frame* frame, const float* p
     if (G < 1) G = 1;
     if (G > nh) G = nh;
     const dim3 rgrid(n_items * (nh / G));
-    const size_t rlds = (size_t)G * nphi * 8 + (size_t)G * 16;
+    const int points = a.log2nphi >= 7 && a.log2nphi <= 9 ? fft_at(nphi) : nphi;
+    const size_t rlds = (size_t)G * points * 8 + (size_t)G * 16;
     if (a.log2nphi == 7)
         ZB_LAUNCH("k_rings", k_rings<7>, rgrid, dim3(256), rlds, s, a, G, band->ring, tw, pats, its, (const float2*)sums, (const int*)live, spectra);
     else if (a.log2nphi == 8)
