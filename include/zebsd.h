@@ -441,7 +441,8 @@ int32_t zb_profile_select(const char* names);
  *   "refine_queue" 0..2 (0): zb_refine_phases as one block per work item (0) or as a persistent
  *                            grid draining device-side queues (1; 2: the same)
  *   "rings_group"  0..64 (0): ring pairs per block of the sphere stage's ring transforms, a power
- *                            of two (0: 16 KB of LDS worth; at most n / 2 and 64 KB)
+ *                            of two (0: 16, 4 and 4 for rings of 128, 256 and 512 points, else 16 KB of
+ *                            LDS worth; at most n / 2 and 64 KB)
  *   "prep_global"  0..1 (0): zb_prep_work's filters through global memory even where LDS holds
  *                            the image (1)
  * The reference fixes the ring lines a workgroup transforms at TW_LEN / n

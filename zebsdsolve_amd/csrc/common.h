@@ -400,21 +400,28 @@ __device__ void fft_dif(float2* buf, int log2n, int nlines, int lstride, int pst
 //
 // Every stage of a line of 2^k points meets powers of two, and so few of the 64 LDS banks (4-way
 // conflicts in the stages, 32-way in the bit-reversed gather after them: two thirds of the LDS
-// cycles of a kernel that LDS bound). So point p sits at fft_at(p) = p + p / 64, a line takes
-// fft_line<LOG2N> = 2^LOG2N + 2^LOG2N / 64 points, and neighbouring threads take neighbouring lines
-// and then F = 2^LOG2N / 64 butterflies of one, neighbours or (where q < F) an eighth of the line or
-// so apart: with 32 / F lines 32 threads meet every bank once. With p's digits disjoint fft_at adds
+// cycles of a kernel that LDS bound). So point p sits at fft_at(p) = p + p / 2^shift, a line takes
+// fft_line<LOG2N> = 2^LOG2N + F points, F = 2^(LOG2N - shift), and neighbouring threads take
+// neighbouring lines and then F butterflies of one, neighbours or (where q < F) a part of the line
+// apart: with 32 / F lines 32 threads meet every bank once. With p's digits disjoint fft_at adds
 // up, so the four points of a butterfly stay a constant apart.
-// (The ring transforms at L = 64, 3 001 items: conflicts 44 of 67 M LDS cycles, k_rings 186 us; 18 of 41
-// and 145 with the padding, the vector units busy for 115 of them.)
-__host__ __device__ constexpr int fft_at(int p) { return p + (p >> 6); }
+// (The ring transforms at L = 64, 3 001 items, 8 lines a block: conflicts 44 of 67 M LDS cycles, k_rings
+// 186 us; 18 of 41 and 145 padded by one in 64, the vector units busy for 115 of them. Then 4 lines and
+// one in 32: a batch of 4 500 at 60 x 60 1 960 -> 1 944 us.)
+constexpr int fft_shift(int log2n) { return log2n == 8 ? 5 : 6; }
 template <int LOG2N>
-constexpr int fft_line = fft_at(1 << LOG2N);
+__host__ __device__ constexpr int fft_at(int p) {
+    return p + (p >> fft_shift(LOG2N));
+}
+template <int LOG2N>
+constexpr int fft_line = fft_at<LOG2N>(1 << LOG2N);
+// the lines for which a wave meets every bank once: 16, 4 and 4 of 128, 256 and 512 points
+constexpr int fft_lines(int log2n) { return 32 >> (log2n - fft_shift(log2n)); }
 
 // The butterfly (of 2^BITS of a line) that index rr takes in a stage of step 2^LQ.
 template <int LOG2N, int BITS, int LQ>
 __device__ __forceinline__ int fft_turn(int rr) {
-    constexpr int LF = LOG2N - 6;  // log2 F
+    constexpr int LF = LOG2N - fft_shift(LOG2N);  // log2 F
     if constexpr (LQ >= LF) {
         return rr;
     } else {
@@ -443,11 +450,11 @@ __device__ __forceinline__ void fft_dif_stages(float2* buf, int lg_lines, const 
             const int line = e & lmask;
             const int r = fft_turn<LOG2N, LOG2N - 2, lq>(e >> lg_lines);
             const int j = r & (q - 1);
-            float2* b = buf + line * fft_line<LOG2N> + fft_at(((r >> lq) << S) + j);
+            float2* b = buf + line * fft_line<LOG2N> + fft_at<LOG2N>(((r >> lq) << S) + j);
             float2 x0 = b[0];
-            float2 x1 = b[fft_at(q)];
-            float2 x2 = b[fft_at(2 * q)];
-            float2 x3 = b[fft_at(3 * q)];
+            float2 x1 = b[fft_at<LOG2N>(q)];
+            float2 x2 = b[fft_at<LOG2N>(2 * q)];
+            float2 x3 = b[fft_at<LOG2N>(3 * q)];
             float2 w4 = tw[j * t4];
             float2 w2 = tw[j * t2];
             float2 a0 = cadd(x0, x2);
@@ -455,9 +462,9 @@ __device__ __forceinline__ void fft_dif_stages(float2* buf, int lg_lines, const 
             float2 a1 = cadd(x1, x3);
             float2 a3 = twist_mi(csub(x1, x3), w4);
             b[0] = cadd(a0, a1);
-            b[fft_at(q)] = twist(csub(a0, a1), w2);
-            b[fft_at(2 * q)] = cadd(a2, a3);
-            b[fft_at(3 * q)] = twist(csub(a2, a3), w2);
+            b[fft_at<LOG2N>(q)] = twist(csub(a0, a1), w2);
+            b[fft_at<LOG2N>(2 * q)] = cadd(a2, a3);
+            b[fft_at<LOG2N>(3 * q)] = twist(csub(a2, a3), w2);
         }
         __syncthreads();
         fft_dif_stages<NT, LOG2N, S - 2>(buf, lg_lines, tw, tid);
@@ -465,7 +472,7 @@ __device__ __forceinline__ void fft_dif_stages(float2* buf, int lg_lines, const 
         const int total = 1 << (lg_lines + LOG2N - 1);
         for (int e = tid; e < total; e += NT) {
             const int line = e & lmask;
-            float2* b = buf + line * fft_line<LOG2N> + fft_at(2 * fft_turn<LOG2N, LOG2N - 1, 0>(e >> lg_lines));
+            float2* b = buf + line * fft_line<LOG2N> + fft_at<LOG2N>(2 * fft_turn<LOG2N, LOG2N - 1, 0>(e >> lg_lines));
             float2 x0 = b[0];
             float2 x1 = b[1];
             b[0] = cadd(x0, x1);

@@ -197,7 +197,10 @@ __global__ void __launch_bounds__(256) k_rings(SphArg a, int G, const float* __r
     // a line's points in LDS: padded for the lengths known here (fft_at)
     int stride = nphi;
     if constexpr (LOG2NPHI > 0) stride = fft_line<LOG2NPHI>;
-    auto at = [&](int i, int p) -> float2& { return buf[i * stride + (LOG2NPHI > 0 ? fft_at(p) : p)]; };
+    auto at = [&](int i, int p) -> float2& {
+        if constexpr (LOG2NPHI > 0) return buf[i * stride + fft_at<LOG2NPHI>(p)];
+        else return buf[i * stride + p];
+    };
     float4* rt = reinterpret_cast<float4*>(buf + G * stride);
     for (int i = threadIdx.x; i < G; i += 256) rt[i] = ring_entry(ring, y0 + i);
     __syncthreads();
@@ -587,15 +590,18 @@ static int32_t sh_run(const zb_band* band, const zb_frame* frame, const float* p
     if (int rc = check_launch("zb_sh_coefficients/sums")) return rc;
     const int nh = n / 2;
     const int nphi = 2 * n;
-    // ring pairs a block transforms: the knob's (a power of two), else 16 KB of LDS worth; at
-    // most n / 2 and 64 KB of LDS
-    int G = knob(KNOB_RINGS_GROUP) > 0 ? knob(KNOB_RINGS_GROUP) : 2048 / nphi;
+    // ring pairs a block transforms: the knob's (a power of two), else what meets every LDS bank once
+    // (fft_lines; k_rings over 100 000 patterns: L = 64, 8, 4 and 2 pairs 6.3, 4.1 and 5.8 ms; L = 96, 8, 4 and 2: 25.6,
+    // 16.6 and 20.4; L = 32, 16, 8 and 4: 1.39, 1.41 and 1.79), 16 KB of LDS worth past these lengths; at most
+    // n / 2 and 64 KB of LDS
+    const bool padded = a.log2nphi >= 7 && a.log2nphi <= 9;
+    int G = knob(KNOB_RINGS_GROUP) > 0 ? knob(KNOB_RINGS_GROUP) : padded ? fft_lines(a.log2nphi) : 2048 / nphi;
     while (G & (G - 1)) G &= G - 1;
     if (G > 8192 / nphi) G = 8192 / nphi;
     if (G < 1) G = 1;
     if (G > nh) G = nh;
     const dim3 rgrid(n_items * (nh / G));
-    const int points = a.log2nphi >= 7 && a.log2nphi <= 9 ? fft_at(nphi) : nphi;
+    const int points = a.log2nphi == 7 ? fft_line<7> : a.log2nphi == 8 ? fft_line<8> : a.log2nphi == 9 ? fft_line<9> : nphi;
     const size_t rlds = (size_t)G * points * 8 + (size_t)G * 16;
     if (a.log2nphi == 7)
         ZB_LAUNCH("k_rings", k_rings<7>, rgrid, dim3(256), rlds, s, a, G, band->ring, tw, pats, its, (const float2*)sums, (const int*)live, spectra);
