@@ -119,6 +119,15 @@ class DevicePhase:
         return self._vt16[key][0]
 
 
+def _gather(patterns, cells):
+    """Patterns [n, h, w] (a tensor) of the given cells. (torch has no gather of uint16 on a device:
+    the same bits as int16.)"""
+    at = torch.as_tensor(cells, device=patterns.device)
+    if patterns.dtype == torch.uint16:
+        return patterns.view(torch.int16)[at].view(torch.uint16)
+    return patterns[at]
+
+
 def lattice(rows, cols, want):
     """About `want` cells spread evenly over a rows x cols map, row-major (src/engine.zig:1325-1341):
     every cell when the map has no more."""
@@ -587,7 +596,7 @@ class Engine:
                 # (sums of whole numbers, exact in any order; of floats only in the host's)
                 flat = self._resident.reshape(rows * cols, h, w)
             if isinstance(flat, torch.Tensor):
-                sel = flat[torch.as_tensor(cells, device=flat.device)].to(torch.float64)
+                sel = _gather(flat, cells).to(torch.float64)
                 tot = sel.sum(0)
             else:
                 tot = torch.from_numpy(np.asarray(flat)[cells].astype(np.float64).sum(0))
@@ -781,7 +790,7 @@ class Engine:
             out.record_stream(cur)
             return out
         if isinstance(flat, torch.Tensor):
-            part = flat[int(cells[0]):int(cells[-1]) + 1] if run else flat[torch.as_tensor(cells, device=flat.device)]
+            part = flat[int(cells[0]):int(cells[-1]) + 1] if run else _gather(flat, cells)
             return part.to(dev).contiguous()
         part = flat[cells[0]:cells[-1] + 1] if run else flat[cells]
         return torch.from_numpy(np.ascontiguousarray(part)).to(dev)
