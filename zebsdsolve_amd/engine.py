@@ -899,11 +899,17 @@ class Engine:
     def nmi_at(self, pi, cells, quats):
         """NMI of each cell's pattern with phase pi's master at the given orientation (no
         refinement): zb_refine with no iterations. quats [n, 4], or several draws [d, n, 4] in one
-        launch; returns float32 [n] or [d, n]."""
+        launch; returns float32 [n] or [d, n]. ValueError for a count that does not fit the cells:
+        every orientation is an item of the launch, with the pattern of its cell."""
         lib = nat.load()
         dev = self._device()
         cells = np.asarray(cells, np.int64).reshape(-1)
         n = len(cells)
+        quats = np.asarray(quats, np.float32)
+        if quats.ndim == 3 and quats.shape[1:] == (n, 4):
+            shape = quats.shape[:2]
+        else:
+            quats, shape = quats.reshape(n, 4), (n,)
         raw = self._raw_for(cells)
         h, w = self.pattern_hw()
         pats = torch.empty((n, h, w), dtype=torch.float32, device=dev)
@@ -911,8 +917,6 @@ class Engine:
         st = stream_ptr()
         self.prep_into(raw, n, h, w, pats, st)
         t = self.positions(cells)
-        quats = np.asarray(quats, np.float32)
-        shape = quats.shape[:-1]
         total = quats.size // 4
         items = np.concatenate([t, np.arange(n, dtype=np.float32)[:, None]], 1)
         items = torch.from_numpy(np.tile(items, (total // max(n, 1), 1))).to(dev)
