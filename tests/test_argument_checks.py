@@ -58,3 +58,17 @@ def test_nmi_at_launches_an_item_an_orientation(n, shape, launched, result, monk
     monkeypatch.setattr(engine, "stream_ptr", lambda: None)
     out = e.nmi_at(0, np.arange(n), np.zeros(shape, np.float32))
     assert seen == [launched] and out.shape == result
+
+
+@pytest.mark.parametrize("shape", [(5, 7), (8,), (5, 9), (2, 5, 8), ()])
+def test_fit6_refuses_poses_that_are_not_rows_of_eight(shape, monkeypatch):
+    import torch
+    from zebsdsolve_amd import fit
+
+    def launched(*a):
+        raise Launched
+
+    monkeypatch.setattr(fit.nat, "load", lambda: types.SimpleNamespace(zb_fit6=launched, zb_fit6_workspace=launched))
+    field = types.SimpleNamespace(pats=torch.zeros((1, 4, 4)))
+    with pytest.raises(ValueError):
+        fit.fit6(field, np.zeros(shape, np.float32))

@@ -255,6 +255,8 @@ def fit6(field, poses0, iters=20, unknowns=6, lambda0=1e-3, max_rot=np.radians(2
     lib = nat.load()
     dev = field.pats.device
     poses = torch.as_tensor(poses0, dtype=torch.float32, device=dev).clone().contiguous()
+    if poses.dim() != 2 or poses.shape[1] != 8:
+        raise ValueError(f"fit6: poses of shape {tuple(poses.shape)}, not [n, 8]")
     n = poses.shape[0]
     scored = torch.full((), n, dtype=torch.int64, device=dev) if counts is not None else None
     ncc = torch.empty((n,), dtype=torch.float64, device=dev) if with_ncc else None
