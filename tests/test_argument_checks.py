@@ -72,3 +72,25 @@ def test_fit6_refuses_poses_that_are_not_rows_of_eight(shape, monkeypatch):
     field = types.SimpleNamespace(pats=torch.zeros((1, 4, 4)))
     with pytest.raises(ValueError):
         fit.fit6(field, np.zeros(shape, np.float32))
+
+
+@pytest.mark.parametrize("cells", [[6], [5, 6], [0, 9, 2], [-7, 0], [3, -8, 1]])
+@pytest.mark.parametrize("resident", [True, False])
+def test_cells_outside_the_map_are_refused(cells, resident):
+    import torch
+    e = _engine(2, 3)
+    # (a tensor on the meta device checks no index, as one on a GPU before its kernel runs)
+    e._resident = torch.empty(e.shape, device="meta") if resident else None
+    e._device = lambda: torch.device("meta" if resident else "cpu")
+    with pytest.raises(IndexError):
+        e._raw_for(cells)
+
+
+@pytest.mark.parametrize("cells", [[5], [0, 1, 2], [4, 0, 5], [-1], [-2, -1], [-1, 0, 1], [-6, 3], []])
+@pytest.mark.parametrize("resident", [True, False])
+def test_cells_of_the_map_give_their_patterns(cells, resident):
+    import torch
+    e = _engine(2, 3)
+    e._resident = torch.from_numpy(e.patterns) if resident else None
+    got = e._raw_for(cells)
+    assert np.array_equal(got.numpy(), e.patterns.reshape(6, 8, 8)[np.asarray(cells, np.int64)])

@@ -777,7 +777,12 @@ class Engine:
         flat = (self.patterns if resident is None else resident).reshape(rows * cols, h, w)
         cells = np.asarray(cells, np.int64)
         # a run of consecutive cells (the usual request) is a slice: no gather copy
-        run = len(cells) > 0 and cells[-1] - cells[0] == len(cells) - 1 and bool(np.all(np.diff(cells) == 1))
+        run = len(cells) > 0 and 0 <= cells[0] and cells[-1] - cells[0] == len(cells) - 1 and bool(np.all(np.diff(cells) == 1))
+        # (refused here: a gather on the device would abort, a slice give fewer patterns than there are items)
+        if len(cells):
+            lo, hi = (cells[0], cells[-1]) if run else (cells.min(), cells.max())
+            if lo < -rows * cols or hi >= rows * cols:
+                raise IndexError(f"cell {int(lo if lo < -rows * cols else hi)} of a map of {rows * cols} cells")
         pinned = getattr(self, "_pinned", None)
         if run and pinned is not None:
             # page-locked and never written again: the upload goes on a copy stream of its own,
