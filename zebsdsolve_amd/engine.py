@@ -209,7 +209,7 @@ class Engine:
         # streams a large index_cells request is spread over (1: one; more measured no faster
         # through Solver.index, whose steps each wait for their records)
         self.index_lanes = 1
-        self._bg = None           # (key, static background on the device)
+        self._bg = None           # (key, static background on the device, the stream that made it, its event there)
         self.file_background = None  # [h, w] the scan file's static background (static_background "file")
 
     # ── state ──
@@ -583,13 +583,14 @@ class Engine:
         rows, cols, h, w = self.shape
         kind = self.settings["static_background"]
         key = (id(self.patterns), self.shape, int(self.settings["static_patterns"]), kind, id(self.file_background))
-        if kind == "file":
-            if self.file_background is None:
-                raise ValueError('static_background "file": the scan stores no background')
-            if self._bg is None or self._bg[0] != key:
-                self._bg = (key, torch.as_tensor(np.asarray(self.file_background, np.float32)).reshape(h, w).to(self._device()).contiguous())
+        if kind == "file" and self.file_background is None:
+            raise ValueError('static_background "file": the scan stores no background')
+        if self._bg is not None and self._bg[0] == key:
+            self._join_background()
             return self._bg[1]
-        if self._bg is None or self._bg[0] != key:
+        if kind == "file":
+            avg = torch.as_tensor(np.asarray(self.file_background, np.float32)).reshape(h, w).to(self._device()).contiguous()
+        else:
             cells = lattice(rows, cols, int(self.settings["static_patterns"]))
             flat = self.patterns.reshape(rows * cols, h, w)
             if getattr(self, "_resident", None) is not None and self._resident.dtype != torch.float32:
@@ -601,8 +602,24 @@ class Engine:
             else:
                 tot = torch.from_numpy(np.asarray(flat)[cells].astype(np.float64).sum(0))
             avg = (tot * (1.0 / len(cells))).to(torch.float32).to(self._device()).contiguous()
-            self._bg = (key, avg)
-        return self._bg[1]
+        stream = done = None
+        if avg.is_cuda:
+            stream = torch.cuda.current_stream(avg.device)
+            done = torch.cuda.Event()
+            done.record(stream)
+        self._bg = (key, avg, stream, done)
+        return avg
+
+    def _join_background(self):
+        """The current stream, where it is not the one that made the static background, waits for it,
+        and the background's memory for the stream."""
+        _, avg, made, done = self._bg
+        if made is None:
+            return
+        cur = torch.cuda.current_stream(avg.device)
+        if cur != made and not torch.cuda.is_current_stream_capturing():
+            cur.wait_event(done)
+            avg.record_stream(cur)
 
     def prep_into(self, raw, n, h, w, out, st, lane=None):
         """Raw patterns [n, h, w] (device) to the normalized ones in `out`: the pattern filters the
@@ -714,7 +731,11 @@ class Engine:
             if workspace is None or workspace.numel() < need:
                 workspace = torch.empty((need,), dtype=torch.uint8, device=dev)
         else:
+            # (the background too is made before the lane waits for this stream: the filters read it there)
+            bg = self.static_background() if s["static_background"] != "none" else None
             lane.stream.wait_stream(torch.cuda.current_stream(dev))
+            if bg is not None:
+                bg.record_stream(lane.stream)
             st = lane.stream.cuda_stream
             pats = lane.buf("pats", (n_raw, h, w), torch.float32)
             alm = lane.buf("alm", (big, pairs, 2), torch.float32)
