@@ -71,3 +71,28 @@ def test_a_second_stream_waits_for_the_background(slow_background):
         got = s._e.index_cells(np.arange(600))
     torch.cuda.synchronize()
     assert np.array_equal(want[..., :7], got[..., :7])
+
+
+def test_the_scan_outlives_its_engine_for_a_stream_that_reads_it():
+    import gc
+    import torch
+    print("scan read by a stream after its engine is closed", flush=True)
+    scan = _scan(64, 130, np.uint8)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    s = _solver()
+    s.set_patterns(scan)
+    assert s._e._resident is not None
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        raw = s._e._raw_for(np.arange(64 * 130))
+        torch.cuda._sleep(50_000_000)
+        got = raw.clone()
+    del raw
+    s.close()
+    del s
+    gc.collect()
+    # memory of the scan's size from the stream that uploaded it, written while the other one idles
+    other = [torch.full(scan.shape, 255, dtype=torch.uint8, device="cuda") for _ in range(2)]
+    torch.cuda.synchronize()
+    assert np.array_equal(got.cpu().numpy().reshape(scan.shape), scan) and int(other[0].min()) == 255

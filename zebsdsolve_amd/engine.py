@@ -243,7 +243,9 @@ class Engine:
                 a = a.astype(np.float32)
             self.patterns = np.ascontiguousarray(a)
         if getattr(self, "_resident", None) is not None:
-            torch.cuda.synchronize()  # a batch launched ahead on another stream may still read it
+            # (its memory is free for the next scan once every batch that reads it is done)
+            if self._resident.is_cuda:
+                torch.cuda.synchronize(self._resident.device)
             self._resident = None
         if getattr(self, "_pinned", None) is not None:
             # the previous scan's page-locked copy goes back to the system, not to torch's cache
@@ -268,6 +270,14 @@ class Engine:
         if a.nbytes > torch.cuda.mem_get_info(dev)[0] // 4:
             return None
         return torch.from_numpy(a).to(dev)
+
+    def _scan_on_device(self):
+        """The scan uploaded by set_patterns, or None. The current stream is about to read it: its memory,
+        which belongs to the stream that was current at the upload, is not given on before that is done."""
+        scan = getattr(self, "_resident", None)
+        if scan is not None and scan.is_cuda:
+            scan.record_stream(torch.cuda.current_stream(scan.device))
+        return scan
 
     @staticmethod
     def _pin(a):
@@ -593,9 +603,10 @@ class Engine:
         else:
             cells = lattice(rows, cols, int(self.settings["static_patterns"]))
             flat = self.patterns.reshape(rows * cols, h, w)
-            if getattr(self, "_resident", None) is not None and self._resident.dtype != torch.float32:
+            resident = self._scan_on_device()
+            if resident is not None and resident.dtype != torch.float32:
                 # (sums of whole numbers, exact in any order; of floats only in the host's)
-                flat = self._resident.reshape(rows * cols, h, w)
+                flat = resident.reshape(rows * cols, h, w)
             if isinstance(flat, torch.Tensor):
                 sel = _gather(flat, cells).to(torch.float64)
                 tot = sel.sum(0)
@@ -794,7 +805,7 @@ class Engine:
     def _raw_for(self, cells):
         dev = self._device()
         rows, cols, h, w = self.shape
-        resident = getattr(self, "_resident", None)
+        resident = self._scan_on_device()
         flat = (self.patterns if resident is None else resident).reshape(rows * cols, h, w)
         cells = np.asarray(cells, np.int64)
         # a run of consecutive cells (the usual request) is a slice: no gather copy
