@@ -15,6 +15,8 @@ on torch's current stream; there is no CPU path.
 Conventions (as the reference's): quaternions (w, x, y, z) map sample directions to crystal
 directions; Bunge angles in radians; map cells numbered row-major.
 """
+import operator
+
 import numpy as np
 
 from . import _native
@@ -49,8 +51,8 @@ def decoys(n, draw):
     """Uniform random orientations (Shoemake) for items 0..n-1 of draw `draw`, a different one
     per item and draw (detector.wgsl decoy, 296-308): [n, 4], or [d, n, 4] for d draws."""
     b = np.arange(n, dtype=np.uint64)
-    d = np.asarray(draw, np.uint64)[..., None]
-    s = _hash_u32(b + 1) ^ ((d * 0x9E3779B9) & 0xFFFFFFFF)
+    d = np.array([(operator.index(k) * 0x9E3779B9) & 0xFFFFFFFF for k in np.ravel(draw)], np.uint64).reshape(np.shape(draw) + (1,))
+    s = _hash_u32(b + 1) ^ d
     u1 = _unit_rand(s)
     a2 = _unit_rand(s + 1) * 2 * np.pi
     a3 = _unit_rand(s + 2) * 2 * np.pi
