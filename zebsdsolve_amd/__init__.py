@@ -60,6 +60,16 @@ def decoys(n, draw):
     return np.stack([ra * np.sin(a2), ra * np.cos(a2), rb * np.sin(a3), rb * np.cos(a3)], -1).astype(np.float32)
 
 
+def rings_group(knob, n):
+    """The ring pairs a block of the sphere stage's ring transforms takes for the knob "rings_group" and
+    rings of 2 n points, as the library works them out (csrc/sphere.hip sh_run): the knob's, else 16, 4 and 4
+    of 128, 256 and 512 points (a wave meets every LDS bank once), else 16 KB of LDS worth."""
+    points = 2 * n
+    g = knob if knob > 0 else {128: 16, 256: 4, 512: 4}.get(points, 2048 // points)
+    g = 1 << (max(g, 1).bit_length() - 1)
+    return max(1, min(g, 8192 // points, n // 2))
+
+
 class Solver:
     """One engine on one GPU. Use as a context manager or call close()."""
 
@@ -689,10 +699,7 @@ class Solver:
         n = sh.fft_size(L)
 
         def group_of(v):
-            # k_rings' ring pairs a block, as the library derives them from the knob
-            g = v if v > 0 else 2048 // (2 * n)
-            g = 1 << (max(g, 1).bit_length() - 1)
-            return max(1, min(g, 8192 // (2 * n), n // 2))
+            return rings_group(v, n)
 
         choices = {"refine_queue": ((0, 1, 2), lambda v: v), "rings_group": ((0, 4, 8, 16, 32), group_of)}
         for name, (values, launch) in choices.items():
