@@ -4,16 +4,15 @@ import re
 import time
 import types
 
-import numpy as np
 import pytest
 
 from zebsdsolve_amd import Solver, _native, rings_group, sh
 
 
-def _tried(monkeypatch, L):
+def _tried(monkeypatch, L, refine_queue=0):
     """The values tune sets each of the library's knobs to, and not the ones it puts back."""
     import torch
-    knobs = {"refine_queue": 0, "rings_group": 0}
+    knobs = {"refine_queue": refine_queue, "rings_group": 0}
     sets = {k: [] for k in knobs}
 
     def put(name, v):
@@ -52,3 +51,9 @@ def test_the_default_group_is_the_librarys():
     for L in (8, 16, 200, 256):
         n = sh.fft_size(L)
         assert rings_group(0, n) == max(1, min(2048 // (2 * n), n // 2))
+
+
+@pytest.mark.parametrize("present,values", [(0, [1]), (1, [0]), (2, [0])])
+def test_tune_times_the_two_refinement_forms(monkeypatch, present, values):
+    """refine_queue 2 is the form 1 is."""
+    assert _tried(monkeypatch, 64, present)["refine_queue"] == values

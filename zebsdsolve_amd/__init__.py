@@ -701,7 +701,7 @@ class Solver:
         def group_of(v):
             return rings_group(v, n)
 
-        choices = {"refine_queue": ((0, 1, 2), lambda v: v), "rings_group": ((0, 4, 8, 16, 32), group_of)}
+        choices = {"refine_queue": ((0, 1), lambda v: min(v, 1)), "rings_group": ((0, 4, 8, 16, 32), group_of)}
         for name, (values, launch) in choices.items():
             before[name] = lib.zb_knob_get(name.encode())
             for v in values:
