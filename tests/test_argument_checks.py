@@ -1,5 +1,6 @@
 """Arguments that do not fit are refused on the host, before any launch: a kernel takes its counts and
 indices as they come. No GPU: the engine's device side is replaced by stand-ins that note a call."""
+import ctypes
 import types
 
 import numpy as np
@@ -43,7 +44,7 @@ def test_nmi_at_launches_an_item_an_orientation(n, shape, launched, result, monk
     e.phases = [types.SimpleNamespace(master=types.SimpleNamespace(side=5))]
     e.mask_tuple = lambda: (0.0, 0.0, 0.0)
     e.prep_into = lambda *a: None
-    e.refine_opts = lambda: types.SimpleNamespace(iters=1)
+    e.refine_opts = lambda: types.SimpleNamespace(iters=1, stamp=1)
     e.positions = lambda cells: np.zeros((len(cells), 3), np.float32)
     e.baked = lambda pi: (None, (torch.zeros(1), None, None))
     e.grad_half = lambda pi: torch.zeros(1)
@@ -52,6 +53,7 @@ def test_nmi_at_launches_an_item_an_orientation(n, shape, launched, result, monk
 
     def refine(*a):
         seen.append(a[8])
+        (ctypes.c_float * (8 * a[8])).from_address(a[10])[7::8] = [1.0] * a[8]  # the records' stamps
         return 0
 
     monkeypatch.setattr(engine.nat, "load", lambda: types.SimpleNamespace(zb_refine=refine))

@@ -25,7 +25,7 @@ struct RefArg {
     float c0[3], c1[3], c2[3];
     float mask[3];
     int h, w, side;
-    int iters, nmi_bins, seed_stride, out0;
+    int iters, nmi_bins, seed_stride, out0, polls;
     float max_step, scale0, scale_min, scale_max;
     float stamp;
     int tiles;  // 8 x 8 tiles of the frame the tile walk lists (0: every tile is walked)
@@ -138,6 +138,8 @@ struct alignas(16) Shared {
     Gn gn;
     int cnt[W];
     int turn;  // the chunk whose sums are to be added next, counted over the item's passes
+    int polls;  // how often a wave looks for its turn
+    int late;   // a wave gave up waiting for its turn: the record is not valid
 };
 
 struct Held {
@@ -160,12 +162,18 @@ __device__ __forceinline__ Chunks chunks_of(int n_px) {
 }
 
 // Waits until the chain reaches chunk `id` (its turn comes after finitely many chunks of other
-// waves of the block, all resident; the bound only keeps a wave from waiting for ever).
-__device__ __forceinline__ void wait_turn(int* turn, int id) {
-    for (int k = 0; k < (1 << 22); ++k) {
-        if (__builtin_amdgcn_readfirstlane(__hip_atomic_load(turn, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP)) == id) break;
+// waves of the block, all resident; the bound only keeps a wave from waiting for ever: one that
+// gives up marks the item's record as not valid).
+// (The bound comes from LDS with the first look: 4 500 items at 60 x 60, L = 64, 1 945 us a batch, as with a
+// bound known to the compiler; held in a scalar register over the passes 1 955, read at each look 1 947.)
+template <int W>
+__device__ __forceinline__ void wait_turn(Shared<W>& sh, int id) {
+    int left = __builtin_amdgcn_readfirstlane(sh.polls);
+    do {
+        if (__builtin_amdgcn_readfirstlane(__hip_atomic_load(&sh.turn, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP)) == id) break;
         __builtin_amdgcn_s_sleep(1);
-    }
+    } while (--left > 0);
+    if (left <= 0) sh.late = 1;
 }
 __device__ __forceinline__ void pass_turn(int* turn, int id, int lane) {
     if (lane == 0) __hip_atomic_store(turn, id + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -408,6 +416,8 @@ __device__ __forceinline__ void refine_item(const RefArg& a, const float* __rest
         if (lane == 0) {
             sh.gn = g;
             sh.turn = 0;
+            sh.late = 0;
+            sh.polls = a.polls;
         }
     }
     __syncthreads();
@@ -446,7 +456,7 @@ __device__ __forceinline__ void refine_item(const RefArg& a, const float* __rest
                         m[i] = v.w;
                         e[i] = ev;
                     });
-                wait_turn(&sh.turn, base + id);
+                wait_turn(sh, base + id);
                 if (id > 0) {
 #pragma unroll
                     for (int j = 0; j < kPart / 4; ++j) {
@@ -555,7 +565,7 @@ __device__ __forceinline__ void refine_item(const RefArg& a, const float* __rest
                 if constexpr (MODE == REF_HELD) simv[decltype(rc)::value * kChunk + i] = sv[i];
                 if (i < cnt && 64 * (step0 + i) + lane < n_px) extremes(ev[i], sv[i]);
             }
-            wait_turn(&sh.turn, base + id);
+            wait_turn(sh, base + id);
             if (id > 0) f = sh.acc[0][lane];
 #pragma unroll
             for (int i = 0; i < kChunk; ++i)
@@ -672,7 +682,7 @@ __device__ __forceinline__ void refine_item(const RefArg& a, const float* __rest
         r[4] = ncc_best;
         r[5] = nmi;
         r[6] = sh.gn.last_step;
-        r[7] = a.stamp;
+        r[7] = sh.late ? __int_as_float(0x7fc00000) : a.stamp;  // (no stamp equals a NaN)
     }
 }
 
@@ -1013,6 +1023,7 @@ int32_t zb::sums_run(const float* mgrad, int32_t side, const zb_frame* frame, co
 static void ref_opts(RefArg& a, const zb_refine_opts* o, int out0) {
     a.iters = o->iters;
     a.nmi_bins = o->nmi_bins;
+    a.polls = knob(KNOB_REFINE_POLLS);
     a.out0 = out0;
     a.max_step = o->max_step;
     a.scale0 = o->scale0;

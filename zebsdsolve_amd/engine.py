@@ -964,7 +964,10 @@ class Engine:
         _, (sheets, _, _) = self.baked(pi)
         nat.check(lib.zb_refine(sheets.data_ptr(), self.grad_half(pi).data_ptr(), self.phases[pi].master.side, self.frame(), pats.data_ptr(), items.data_ptr(),
                                 seeds.data_ptr(), 4, total, o, rec.data_ptr(), 0, st), "nmi")
-        return rec[:, 5].cpu().numpy().reshape(shape)
+        rec = rec.cpu().numpy()
+        if not np.all(rec[:, 7] == np.float32(o.stamp)):
+            raise RuntimeError("DeviceSkippedBatch: records without this batch's stamp")
+        return np.ascontiguousarray(rec[:, 5]).reshape(shape)
 
     def simulate(self, pi, cells, quats):
         """Simulated patterns of phase pi at the given orientations, as cells would record them
