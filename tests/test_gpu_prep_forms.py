@@ -1,0 +1,55 @@
+"""The filters' forms give the same bits: whatever the alignment of the workspace, the kernel that a size and a
+chain of filters take, and the switches that force another."""
+import numpy as np
+import pytest
+
+from tests.conftest import gpu_available
+from tests.test_gpu_prep_tiles import _raw
+
+pytestmark = [pytest.mark.gpu, pytest.mark.skipif(not gpu_available(), reason="needs a GPU")]
+
+CHAINS = {"direct": dict(dynamic=1, dynamic_sigma=4.0), "boxes": dict(dynamic=1, dynamic_sigma=14.5), "divided boxes": dict(dynamic=2, dynamic_sigma=12.5),
+          "clahe": dict(clahe=1, clahe_grid=4, clahe_bins=64, clahe_clip=2.0),
+          "all": dict(dynamic=2, dynamic_sigma=9.3, clahe=1, clahe_grid=3, clahe_bins=65, clahe_clip=2.5, bandpass=1, bp_fine=1.5, bp_coarse=6.0),
+          "all by boxes": dict(dynamic=2, dynamic_sigma=13.0, clahe=1, clahe_grid=5, clahe_bins=32, clahe_clip=1.5, bandpass=1, bp_fine=12.0, bp_coarse=16.0),
+          "band pass": dict(bandpass=1, bp_fine=0.0, bp_coarse=13.0)}
+
+
+def _call(raw, chain, shift=0, background=False, **knobs):
+    """The patterns through zb_prep_work, the workspace `shift` bytes past 256, with the knobs set; and the
+    workspace's bytes that the call wrote."""
+    import torch
+    from zebsdsolve_amd import _native as nat, engine
+    lib = nat.load()
+    n, h, w = raw.shape
+    o = nat.PrepOpts()
+    for k, v in CHAINS[chain].items():
+        setattr(o, k, v)
+    kind = {"float32": 2, "uint16": 1, "uint8": 0}[raw.dtype.name]
+    dev = torch.from_numpy(raw.view(np.int16) if kind == 1 else raw).cuda()
+    bg = torch.from_numpy(raw.astype(np.float64).mean(0).astype(np.float32)).cuda()
+    o.background = bg.data_ptr() if background else None
+    out = torch.full((n, h, w), float("nan"), device="cuda")
+    m = (nat.ctypes.c_float * 3)((h - 1) / 2, (w - 1) / 2, (min(h, w) / 2) ** 2)
+    before = {k: lib.zb_knob_set(k.encode(), v) for k, v in knobs.items()}
+    assert min(before.values(), default=0) >= 0
+    try:
+        need = int(lib.zb_prep_workspace(n, h, w, nat.ctypes.byref(o)))
+        ws = torch.full((max(need, 8) + shift,), 171, dtype=torch.uint8, device="cuda")
+        nat.check(lib.zb_prep_work(dev.data_ptr(), kind, n, h, w, m, nat.ctypes.byref(o), ws.data_ptr() + shift, ws.numel() - shift, out.data_ptr(),
+                                   engine.stream_ptr()), "prep")
+        return out.cpu().numpy(), int((ws != 171).sum())
+    finally:
+        for k, v in before.items():
+            lib.zb_knob_set(k.encode(), v)
+
+
+@pytest.mark.parametrize("chain", ["direct", "all", "all by boxes"])
+@pytest.mark.parametrize("h,w", [(60, 60), (44, 64), (120, 120)])
+def test_a_workspace_of_eight_bytes_alignment(chain, h, w):
+    print(f"prep workspace alignment {chain} {h}x{w}", flush=True)
+    raw = _raw(5, h, w, h + w)
+    want, _ = _call(raw, chain, 0, prep_global=1)
+    for shift in (8, 16, 24):
+        got, wrote = _call(raw, chain, shift, prep_global=1)
+        assert wrote > 0 and np.array_equal(got, want), shift

@@ -933,7 +933,7 @@ __device__ __forceinline__ float sum256(float v, float* red) {
 // read down the rows, would share fewer than 8 of the 64 banks),
 // or, GLOB, in the block's slot of global memory (patterns blockIdx.x, + gridDim.x, ...; S = w) with
 // what is smaller than an image in LDS still. vec: four pixels a load and store (h w a multiple of
-// 4, raw, background and out aligned to four pixels).
+// 4, raw, background, out and GLOB's slots aligned to four pixels).
 template <typename T, int NT, bool GLOB, bool FULL>
 __global__ void __launch_bounds__(NT, FULL ? 4 : 5) k_prep_tiles(const T* __restrict__ raw, const float* __restrict__ bg, PrepArg a, int n, int S, int vec,
                                                    float* __restrict__ work, long slot, float* __restrict__ out) {
@@ -1388,7 +1388,9 @@ static void prep_launch(const void* raw_, const float* bg, const PrepArg& a, int
                         float* out, hipStream_t s) {
     const T* raw = (const T*)raw_;
     const long hw = (long)a.h * a.w;
-    const int vec = hw % 4 == 0 && (uintptr_t)raw % (4 * sizeof(T)) == 0 && (uintptr_t)out % 16 == 0 && (uintptr_t)bg % 16 == 0;
+    // (the global form's image lies in the workspace, which a caller aligns to 8 bytes; its slots are multiples of 256)
+    const int vec = hw % 4 == 0 && (uintptr_t)raw % (4 * sizeof(T)) == 0 && (uintptr_t)out % 16 == 0 && (uintptr_t)bg % 16 == 0 &&
+                    (form != kPrepTilesG || (uintptr_t)work % 16 == 0);
 #define ZB_TILES(NT, G, F, GRID) \
     ZB_LAUNCH("k_prep", (k_prep_tiles<T, NT, G, F>), dim3(GRID), dim3(NT), lds, s, raw, bg, a, n, S, vec, work, slot, out)
     // without CLAHE and box sums the code for them is left out (its registers hold 60 x 60 to four blocks
