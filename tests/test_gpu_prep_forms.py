@@ -53,3 +53,16 @@ def test_a_workspace_of_eight_bytes_alignment(chain, h, w):
     for shift in (8, 16, 24):
         got, wrote = _call(raw, chain, shift, prep_global=1)
         assert wrote > 0 and np.array_equal(got, want), shift
+
+
+@pytest.mark.parametrize("chain", list(CHAINS))
+@pytest.mark.parametrize("h,w,dtype", [(60, 60, np.uint8), (75, 83, np.float32), (120, 120, np.uint16)])
+def test_prep_global_goes_through_global_memory(chain, h, w, dtype):
+    """With the knob prep_global every chain's image lies in the workspace, and every pixel is the same."""
+    print(f"prep forced global {chain} {h}x{w} {np.dtype(dtype).name}", flush=True)
+    raw = _raw(5, h, w, h + w)
+    raw = (raw / 4 if dtype == np.uint8 else raw).astype(dtype)
+    want, _ = _call(raw, chain, background=True, prep_global=0)
+    got, wrote = _call(raw, chain, background=True, prep_global=1)
+    assert wrote > 0
+    assert np.array_equal(got, want)

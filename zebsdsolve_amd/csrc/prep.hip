@@ -1361,12 +1361,13 @@ enum PrepForm { kPrepLoops, kPrepLoopsG, kPrepTiles, kPrepTilesG, kPrepBoxes };
 
 // The fast forms wherever what they keep in LDS fits (their tables differ from k_prep's scratch,
 // so it doesn't for a few images near the limit, nor for long thin ones) and pix_rc is exact; `lds`
-// becomes the bytes of dynamic LDS, `S` the image's row stride.
-static PrepForm prep_form(const PrepArg& a, bool global, int limit, size_t& lds, int& S) {
+// becomes the bytes of dynamic LDS, `S` the image's row stride. forced: the caller asked for global
+// memory, which k_prep_box would not go through.
+static PrepForm prep_form(const PrepArg& a, bool global, bool forced, int limit, size_t& lds, int& S) {
     const PrepForm loops = global ? kPrepLoopsG : kPrepLoops;
     const long hw = (long)a.h * a.w, room = (long)(limit - 1024) / 4;
     if (hw > (1L << 22)) return loops;
-    if (a.dyn && a.dynb.box && !a.clahe && !a.bp && box_words(a.dynb, a.h, a.w) <= room) {
+    if (!forced && a.dyn && a.dynb.box && !a.clahe && !a.bp && box_words(a.dynb, a.h, a.w) <= room) {
         lds = (size_t)box_words(a.dynb, a.h, a.w) * 4;
         return kPrepBoxes;
     }
@@ -1441,7 +1442,8 @@ static int32_t prep_run(const char* who, const void* raw, int32_t pixel, int32_t
         set_error("%s: no device", who);
         return ZB_ELAUNCH;
     }
-    const bool global = lds > (size_t)limit || (may_global && knob(KNOB_PREP_GLOBAL) != 0);
+    const bool forced = may_global && knob(KNOB_PREP_GLOBAL) != 0;
+    const bool global = lds > (size_t)limit || forced;
     if (global && !may_global) {
         set_error("%s: a %d x %d pattern with these filters needs %zu bytes of LDS, the device gives a block %d (zb_prep_work takes it "
                   "through global memory)",
@@ -1462,7 +1464,7 @@ static int32_t prep_run(const char* who, const void* raw, int32_t pixel, int32_t
     hipStream_t s = (hipStream_t)stream;
     const float* bg = o->background;
     int S = w;
-    const PrepForm form = prep_form(a, global, limit, lds, S);
+    const PrepForm form = prep_form(a, global, forced, limit, lds, S);
     if (pixel == 0)
         prep_launch<uint8_t>(raw, bg, a, n, form, lds, S, (float*)work, slot, grid, out, s);
     else if (pixel == 1)
