@@ -445,6 +445,8 @@ int32_t zb_profile_select(const char* names);
  *                            LDS worth; at most n / 2 and 64 KB)
  *   "prep_global"  0..1 (0): zb_prep_work's filters through global memory even where LDS holds
  *                            the image (1)
+ *   "prep_loops"   0..1 (0): zb_prep and zb_prep_work by the kernels that take every call (1), also
+ *                            where a faster form's tables fit LDS
  *   "refine_polls" 1..4194304 (4194304): how often a refinement block's wave looks whether its turn to
  *                            add its sums has come; a record for which one gave up carries NaN in
  *                            place of the stamp (the default is some 0.2 s, the turn comes within

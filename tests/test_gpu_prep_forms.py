@@ -66,3 +66,45 @@ def test_prep_global_goes_through_global_memory(chain, h, w, dtype):
     got, wrote = _call(raw, chain, background=True, prep_global=1)
     assert wrote > 0
     assert np.array_equal(got, want)
+
+
+SIZES = [(2, 2), (5, 7), (8, 64), (31, 33), (32, 32), (33, 65), (44, 64), (60, 60), (64, 48), (75, 83), (97, 96), (120, 120), (129, 128), (240, 320)]
+
+
+@pytest.mark.parametrize("chain", list(CHAINS))
+@pytest.mark.parametrize("forced", [0, 1])
+def test_the_fast_forms_give_the_general_kernels_bits(chain, forced):
+    """Every pixel of k_prep_tiles and k_prep_box is that of k_prep and k_prep_g: their sums run in the same order."""
+    for k, (h, w) in enumerate(SIZES):
+        dtype = (np.uint8, np.uint16, np.float32)[k % 3]
+        print(f"prep forms {chain} {h}x{w} {np.dtype(dtype).name} global {forced}", flush=True)
+        raw = _raw(4, h, w, 100 * h + w)
+        raw = (raw / 4 if dtype == np.uint8 else raw).astype(dtype)
+        for background in (False, True):
+            want, _ = _call(raw, chain, background=background, prep_global=forced, prep_loops=1)
+            got, _ = _call(raw, chain, background=background, prep_global=forced)
+            assert np.isfinite(want).all()
+            assert np.array_equal(got, want), (h, w, background, np.abs(got - want).max())
+
+
+@pytest.mark.parametrize("sigma", [0.3, 0.7, 2.0, 5.5, 9.0, 11.99, 12.0, 17.3, 30.5, 60.0])
+@pytest.mark.parametrize("dynamic", [1, 2])
+def test_every_deviation_gives_the_general_kernels_bits(sigma, dynamic, monkeypatch):
+    monkeypatch.setitem(CHAINS, "one", dict(dynamic=dynamic, dynamic_sigma=sigma))
+    for h, w in ((40, 40), (61, 90), (128, 129)):
+        print(f"prep forms sigma {sigma} dynamic {dynamic} {h}x{w}", flush=True)
+        raw = _raw(4, h, w, h * w)
+        want, _ = _call(raw, "one", prep_loops=1)
+        got, _ = _call(raw, "one")
+        assert np.array_equal(got, want), (h, w, np.abs(got - want).max())
+
+
+@pytest.mark.parametrize("value", [np.nan, np.inf, -np.inf, 3e38, 1e-42, -0.0])
+@pytest.mark.parametrize("chain", list(CHAINS))
+def test_odd_pixels_give_the_general_kernels_bits(value, chain):
+    print(f"prep forms {chain} a pixel of {value}", flush=True)
+    raw = _raw(3, 60, 60, 9)
+    raw[0, 0, 0] = raw[1, 30, 31] = raw[2, 59, 59] = value
+    want, _ = _call(raw, chain, prep_loops=1)
+    got, _ = _call(raw, chain)
+    assert np.array_equal(got, want, equal_nan=True)

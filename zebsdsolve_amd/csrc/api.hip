@@ -87,6 +87,7 @@ static Knob g_knobs[] = {
     {"rings_group", 0, 64, 0, {0}},  // ring pairs per k_rings block (0: 2048 / (2n), at most n / 2)
     {"prep_global", 0, 1, 0, {0}},   // zb_prep_work: 1 the filters through global memory even where LDS holds the image
     {"refine_polls", 1, 1 << 22, 1 << 22, {1 << 22}},  // k_refine: polls of a wave's wait for its turn before its record goes unstamped
+    {"prep_loops", 0, 1, 0, {0}},    // zb_prep, zb_prep_work: 1 the kernels that take every call, also where a faster form holds
 };
 static_assert(sizeof g_knobs / sizeof g_knobs[0] == KNOB_COUNT, "a knob per id");
 

@@ -1366,7 +1366,7 @@ enum PrepForm { kPrepLoops, kPrepLoopsG, kPrepTiles, kPrepTilesG, kPrepBoxes };
 static PrepForm prep_form(const PrepArg& a, bool global, bool forced, int limit, size_t& lds, int& S) {
     const PrepForm loops = global ? kPrepLoopsG : kPrepLoops;
     const long hw = (long)a.h * a.w, room = (long)(limit - 1024) / 4;
-    if (hw > (1L << 22)) return loops;
+    if (hw > (1L << 22) || knob(KNOB_PREP_LOOPS) != 0) return loops;
     if (!forced && a.dyn && a.dynb.box && !a.clahe && !a.bp && box_words(a.dynb, a.h, a.w) <= room) {
         lds = (size_t)box_words(a.dynb, a.h, a.w) * 4;
         return kPrepBoxes;
