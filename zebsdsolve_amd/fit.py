@@ -242,11 +242,45 @@ def local_with_autograd(field, poses, flags=0, state=None):
     return local
 
 
+# (what zb_fit6 computes on the device)
+_OWN_MODEL = (PoseField.sums, PoseField.local6)
+
+
+def _own_model(field):
+    """Whether the field's local model is PoseField's: neither its sums nor its local6 replaced."""
+    mine = (getattr(type(field), "sums", None), getattr(type(field), "local6", None))
+    return mine == _OWN_MODEL and not {"sums", "local6"} & set(getattr(field, "__dict__", ()))
+
+
+def _fit6_by_turns(lib, field, poses, iters, unknowns, lambda0, max_rot, max_shift, tol, st):
+    """fit6 of a field with a model of its own: its local6 at each turn's poses, the gradient through
+    PoseNcc, the steps by zb_fit6_step and zb_fit6_keep. Returns (NCC, state, poses scored)."""
+    dev = field.pats.device
+    n = poses.shape[0]
+    flags = ROTATION_ONLY if unknowns == 3 else 0
+    local = local_with_autograd(field, poses, flags)
+    scored = torch.full((), n, dtype=torch.int64, device=dev)
+    lam = torch.full((n,), float(lambda0), dtype=torch.float64, device=dev)
+    cur = torch.zeros((n, 2), dtype=torch.float64, device=dev)
+    state = torch.zeros((n,), dtype=torch.int32, device=dev)
+    trial = torch.empty_like(poses)
+    for _ in range(iters):
+        nat.check(lib.zb_fit6_step(poses.data_ptr(), local.data_ptr(), lam.data_ptr(), n, unknowns, float(max_rot), float(max_shift),
+                                   trial.data_ptr(), cur.data_ptr(), state.data_ptr(), st), "fit6 step")
+        # only the items still moving are scored (converged ones stay put)
+        tlocal = local_with_autograd(field, trial, flags, state)
+        scored += (state == 0).sum()
+        nat.check(lib.zb_fit6_keep(trial.data_ptr(), tlocal.data_ptr(), n, float(tol), cur.data_ptr(), poses.data_ptr(), local.data_ptr(),
+                                   lam.data_ptr(), state.data_ptr(), st), "fit6 keep")
+    return torch.where(local[:, 1] > 0.5, local[:, 0], torch.zeros_like(local[:, 0])), state, scored
+
+
 def fit6(field, poses0, iters=20, unknowns=6, lambda0=1e-3, max_rot=np.radians(2.0), max_shift=2.0, tol=1e-7, with_ncc=True, counts=None):
     """Each pose fitted to its pattern by Levenberg-Marquardt steps over the six directions (or
     the rotation alone, unknowns = 3), on the device (zb_fit6): per step each item's damped Newton
     step from its local model in FP64, the model at the moved poses (of the items still moving)
-    deciding which are kept; an item whose step fell below tol has converged and stays put.
+    deciding which are kept; an item whose step fell below tol has converged and stays put. A field
+    whose sums or local6 are its own is fitted by those, turn by turn.
     Returns (poses [n, 8] float32, NCC [n] float64 (None without with_ncc), state [n]: 0 still
     moving after `iters` steps, 1 converged (the last step below tol), 2 flat), all on the device. `counts` (a dict), if
     given, receives "scored": a device tensor of the poses scored (the start and every trial of
@@ -258,6 +292,11 @@ def fit6(field, poses0, iters=20, unknowns=6, lambda0=1e-3, max_rot=np.radians(2
     if poses.dim() != 2 or poses.shape[1] != 8:
         raise ValueError(f"fit6: poses of shape {tuple(poses.shape)}, not [n, 8]")
     n = poses.shape[0]
+    if not _own_model(field):
+        ncc, state, scored = _fit6_by_turns(lib, field, poses, iters, unknowns, lambda0, max_rot, max_shift, tol, stream_ptr())
+        if counts is not None:
+            counts["scored"] = scored
+        return poses, ncc if with_ncc else None, state
     scored = torch.full((), n, dtype=torch.int64, device=dev) if counts is not None else None
     ncc = torch.empty((n,), dtype=torch.float64, device=dev) if with_ncc else None
     state = torch.zeros((n,), dtype=torch.int32, device=dev)
