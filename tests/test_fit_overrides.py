@@ -73,3 +73,17 @@ def test_fit6_of_a_plain_field_is_one_call(sub, monkeypatch):
     f = _field(type("Named", (fit.PoseField,), {"name": "mine"}) if sub else fit.PoseField)
     with pytest.raises(WholeFit):
         fit.fit6(f, torch.zeros((3, 8)))
+
+
+@pytest.mark.parametrize("iters,turns", [(0, 0), (7, 7), (-3, 0), (True, 1)])
+def test_fit6_takes_whole_numbers_of_turns(iters, turns, monkeypatch):
+    import torch
+    seen = []
+    lib = _lib([])
+    lib.zb_fit6 = lambda *a: seen.append(a[7]) or 0
+    monkeypatch.setattr(fit.nat, "load", lambda: lib)
+    monkeypatch.setattr(engine, "stream_ptr", lambda: None)
+    fit.fit6(_field(fit.PoseField), torch.zeros((3, 8)), iters=iters)
+    assert seen == [turns]
+    with pytest.raises(TypeError):
+        fit.fit6(_field(fit.PoseField), torch.zeros((3, 8)), iters=2.5)

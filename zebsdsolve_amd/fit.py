@@ -292,6 +292,7 @@ def fit6(field, poses0, iters=20, unknowns=6, lambda0=1e-3, max_rot=np.radians(2
     if poses.dim() != 2 or poses.shape[1] != 8:
         raise ValueError(f"fit6: poses of shape {tuple(poses.shape)}, not [n, 8]")
     n = poses.shape[0]
+    iters = len(range(iters))  # (a whole number; none below 0)
     if not _own_model(field):
         ncc, state, scored = _fit6_by_turns(lib, field, poses, iters, unknowns, lambda0, max_rot, max_shift, tol, stream_ptr())
         if counts is not None:
@@ -301,7 +302,7 @@ def fit6(field, poses0, iters=20, unknowns=6, lambda0=1e-3, max_rot=np.radians(2
     ncc = torch.empty((n,), dtype=torch.float64, device=dev) if with_ncc else None
     state = torch.zeros((n,), dtype=torch.int32, device=dev)
     work = torch.empty((int(lib.zb_fit6_workspace(n)),), dtype=torch.uint8, device=dev)
-    nat.check(lib.zb_fit6(field.grad.data_ptr(), field.side, field.frame, field.pats.data_ptr(), poses.data_ptr(), n, int(unknowns), int(iters),
+    nat.check(lib.zb_fit6(field.grad.data_ptr(), field.side, field.frame, field.pats.data_ptr(), poses.data_ptr(), n, int(unknowns), iters,
                           float(lambda0), float(max_rot), float(max_shift), float(tol), work.data_ptr(), work.numel(),
                           None if ncc is None else ncc.data_ptr(), None if scored is None else scored.data_ptr(), state.data_ptr(),
                           stream_ptr()), "fit6")
