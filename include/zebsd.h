@@ -329,7 +329,8 @@ int32_t zb_fit6_keep(const float* trial, const double* trial_local, int32_t n, d
  * The models are taken at the poses with q brought to unit length in 64 bits. Lambda starts at
  * lambda0; unknowns 3 is the rotation alone; ncc [n] f64 (0 where flat) and scored (poses scored, added
  * to what is there) may be NULL; state [n] as zb_fit6_step's. work: zb_fit6_workspace(n) bytes,
- * 256-byte aligned. */
+ * 256-byte aligned; it begins with the local models [n][29] f64 of the last turn (of the start with
+ * iters 0), zeros for the items not scored in it. */
 int64_t zb_fit6_workspace(int32_t n);
 int32_t zb_fit6(const float* mgrad, int32_t side, const zb_frame* frame, const float* pats, float* poses, int32_t n, int32_t unknowns,
                 int32_t iters, double lambda0, double max_rot, double max_shift, double tol, void* work, int64_t work_bytes, double* ncc,

@@ -29,7 +29,7 @@ def _lib(calls):
             return 0
         return call
 
-    return types.SimpleNamespace(zb_fit6=whole, zb_fit6_workspace=lambda n: 8, zb_fit6_step=note("step"), zb_fit6_keep=note("keep"),
+    return types.SimpleNamespace(zb_fit6=whole, zb_fit6_workspace=lambda n: 8 * fit.LOCAL * n, zb_fit6_step=note("step"), zb_fit6_keep=note("keep"),
                                  zb_local6=note("local6"), zb_sums=note("sums"), zb_sums_active=note("sums"))
 
 

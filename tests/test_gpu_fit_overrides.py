@@ -48,3 +48,30 @@ def test_a_model_of_nothing_moves_nothing(fitcase):  # noqa: F811
     poses, ncc, state = fit.fit6(_as(fitcase["field"], Flat), fitcase["poses"], iters=3)
     assert (state == 2).all() and (ncc == 0).all()
     assert torch.equal(poses.cpu(), torch.as_tensor(np.asarray(fitcase["poses"], np.float32)))
+
+
+@pytest.mark.parametrize("n,iters", [(0, 4), (5, 0), (65, 1), (130, 6), (130, 14)])
+def test_last_local_is_the_last_turns_model(fitcase, n, iters):  # noqa: F811
+    import torch
+    from tests.test_gpu_fit_turns import _turn_by_turn
+    from zebsdsolve_amd import fit
+    print(f"fit last local n {n} iters {iters}", flush=True)
+    base = np.asarray(fitcase["poses"], np.float32)
+    rng = np.random.default_rng(n)
+    poses = base[rng.integers(0, len(base), n)].copy()
+    poses[:, :3] += rng.normal(0, 0.05, (n, 3)).astype(np.float32)
+    one, two = copy.copy(fitcase["field"]), copy.copy(fitcase["field"])
+    _, ncc, state = fit.fit6(one, poses, iters=iters, tol=1e-4)
+    a = one.last_local
+    assert a.shape == (n, fit.LOCAL) and a.dtype == torch.float64
+    if n == 0:
+        return
+    _turn_by_turn(two, poses, iters, 6, 1e-4)
+    b = two.last_local
+    # the same rows scored; their models to the trials' float32 rounding
+    assert torch.equal(a[:, 1], b[:, 1]) and (a[a[:, 1] == 0] == 0).all()
+    assert ((a - b).abs() <= 1e-4 * b.abs().amax(0)).all()
+    if iters == 0:
+        assert torch.equal(a[:, 0], ncc)
+    if iters == 14:
+        assert (a[:, 1] == 0).any()  # some had converged before

@@ -263,7 +263,8 @@ __global__ void __launch_bounds__(256) k_fit6_keep(const float* __restrict__ tri
 
 // The whole of one turn of the fit for each item, a thread an item: the sums at its trial decide
 // whether it is kept (k_local6, k_fit6_keep), then the next trial (k_fit6_step). first: the sums are
-// the start's and there is nothing to keep; last: no next trial. Blocks of one wave: the items are
+// the start's and there is nothing to keep; last: no next trial, and the models just scored go to `ended`
+// (zeros for the items that were not). Blocks of one wave: the items are
 // few and every thread's work is a chain of divisions.
 // What bounded the fit was some eighty small launches a turn around k_sums6 (the poses moved, the
 // autograd pass and its copies as tensor operations): 4 000 poses of an 80 x 80 map, 20 turns:
@@ -272,7 +273,7 @@ struct Fit6Turn {
     int first, last;
     double lambda0;
     float *poses, *trial;
-    double *local, *lambda, *cur, *ncc;
+    double *local, *ended, *lambda, *cur, *ncc;
     int* state;
     unsigned long long* scored;
 };
@@ -287,6 +288,17 @@ __global__ void __launch_bounds__(64) k_fit6_turn(const float* __restrict__ sums
     double lambda = w.first ? w.lambda0 : w.lambda[i];
     double ncc = 0.0, g[6], H[36];
     bool ok = false, fresh = false;  // fresh: ncc, g, H are the kept pose's already
+    auto put = [&](double* l) {
+        l[0] = ok ? ncc : 0.0;
+        l[1] = ok ? 1.0 : 0.0;
+        int o = 8;
+#pragma unroll
+        for (int k = 0; k < 6; ++k) l[2 + k] = ok ? g[k] : 0.0;
+#pragma unroll
+        for (int r = 0; r < 6; ++r)
+#pragma unroll
+            for (int c = r; c < 6; ++c) l[o++] = ok ? H[r * 6 + c] : 0.0;
+    };
     if (state == 0) {
         ok = local6(sums + (size_t)i * kSums, ncc, g, H);
         fresh = w.first || (ok && ncc > w.cur[2 * i]);
@@ -300,18 +312,9 @@ __global__ void __launch_bounds__(64) k_fit6_turn(const float* __restrict__ sums
             }
             state = w.cur[2 * i + 1] < a.tol ? 1 : 0;
         }
-        if (fresh) {
-            kept[0] = ok ? ncc : 0.0;
-            kept[1] = ok ? 1.0 : 0.0;
-            int o = 8;
-#pragma unroll
-            for (int k = 0; k < 6; ++k) kept[2 + k] = ok ? g[k] : 0.0;
-#pragma unroll
-            for (int r = 0; r < 6; ++r)
-#pragma unroll
-                for (int c = r; c < 6; ++c) kept[o++] = ok ? H[r * 6 + c] : 0.0;
-        }
+        if (fresh) put(kept);
     }
+    if (w.last) put(w.ended + (size_t)i * kLocal);  // (ok is false where nothing was scored)
     if (!w.last && state == 0) {
         if (!fresh) ok = unpack_local(kept, ncc, g, H);
         if (ok) {
@@ -413,9 +416,9 @@ extern "C" int32_t zb_fit6_keep(const float* trial, const double* trial_local, i
     return check_launch("zb_fit6_keep");
 }
 
-// The parts of zb_fit6's workspace, each 256-byte aligned.
+// The parts of zb_fit6's workspace, each 256-byte aligned; the models of the last turn first.
 struct Fit6Work {
-    int64_t order, sums, trial, cur, lambda, local, bytes;
+    int64_t ended, order, sums, trial, cur, lambda, local, bytes;
     explicit Fit6Work(int64_t n) {
         int64_t at = 0;
         auto take = [&](int64_t b) {
@@ -423,6 +426,7 @@ struct Fit6Work {
             at += (b + 255) / 256 * 256;
             return o;
         };
+        ended = take(n * kLocal * 8);
         order = take(n * 4);
         sums = take(n * kSums * 4);
         trial = take(n * 32);
@@ -471,6 +475,7 @@ extern "C" int32_t zb_fit6(const float* mgrad, int32_t side, const zb_frame* fra
     w.cur = (double*)(base + at.cur);
     w.lambda = (double*)(base + at.lambda);
     w.local = (double*)(base + at.local);
+    w.ended = (double*)(base + at.ended);
     w.ncc = ncc;
     w.state = (int*)state;
     w.scored = (unsigned long long*)scored;

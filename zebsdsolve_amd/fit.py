@@ -280,7 +280,8 @@ def fit6(field, poses0, iters=20, unknowns=6, lambda0=1e-3, max_rot=np.radians(2
     the rotation alone, unknowns = 3), on the device (zb_fit6): per step each item's damped Newton
     step from its local model in FP64, the model at the moved poses (of the items still moving)
     deciding which are kept; an item whose step fell below tol has converged and stays put. A field
-    whose sums or local6 are its own is fitted by those, turn by turn.
+    whose sums or local6 are its own is fitted by those, turn by turn. field.last_local is the model at
+    the last poses scored (flat rows for the items not scored in the last turn).
     Returns (poses [n, 8] float32, NCC [n] float64 (None without with_ncc), state [n]: 0 still
     moving after `iters` steps, 1 converged (the last step below tol), 2 flat), all on the device. `counts` (a dict), if
     given, receives "scored": a device tensor of the poses scored (the start and every trial of
@@ -306,6 +307,7 @@ def fit6(field, poses0, iters=20, unknowns=6, lambda0=1e-3, max_rot=np.radians(2
                           float(lambda0), float(max_rot), float(max_shift), float(tol), work.data_ptr(), work.numel(),
                           None if ncc is None else ncc.data_ptr(), None if scored is None else scored.data_ptr(), state.data_ptr(),
                           stream_ptr()), "fit6")
+    field.last_local = work[:n * LOCAL * 8].view(torch.float64).view(n, LOCAL)
     if counts is not None:
         counts["scored"] = scored
     return poses, ncc, state
