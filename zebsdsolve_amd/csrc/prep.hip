@@ -1359,14 +1359,46 @@ static long prep_slot(const PrepArg& a, long scratch) {
 // caller asked for global memory), which alone decides what is refused and which workspace it takes.
 enum PrepForm { kPrepLoops, kPrepLoopsG, kPrepTiles, kPrepTilesG, kPrepBoxes };
 
-// The fast forms wherever what they keep in LDS fits (their tables differ from k_prep's scratch,
-// so it doesn't for a few images near the limit, nor for long thin ones) and pix_rc is exact; `lds`
-// becomes the bytes of dynamic LDS, `S` the image's row stride. forced: the caller asked for global
-// memory, which k_prep_box would not go through.
-static PrepForm prep_form(const PrepArg& a, bool global, bool forced, int limit, size_t& lds, int& S) {
+// Taps of a direct blur along one axis of n pixels, summed over the pixels.
+static long line_taps(int radius, int n) {
+    const long r = std::min(radius, n - 1);
+    return (2 * r + 1) * n - r * (r + 1);
+}
+
+// Whether k_prep is the faster for n patterns (the pixels are the same bit for bit): what the fast forms
+// make once a block has to be worth it. The lines lie where the two met over 8 x 8 to 160 x 160 and 1 to
+// 16 000 patterns (us of k_prep and of the fast form, u8):
+//  - every blur of the chain of few taps, 9 216 an axis (32 x 32 of 9), 2 in 5 more beside CLAHE or where rows do
+//    not come in fours (4 000 of 16 x 16, sigma 2.4: 19 and 32; 24 x 24, 3.6: 40 and 37), or by boxes on a frame
+//    that they reach across (20 x 20, sigma 14: 52 and 70; 24 x 24: 65 and 74; 28 x 28: 86 and 80), a smaller one
+//    while each CU has a block or two;
+//  - the background alone to 48 x 48 (4 000 of 32 x 32: 16 and 22; 60 x 60: 41 and 37), and CLAHE whose tables are
+//    soon made, up to 5 x 5 tiles or 2 047 levels in all (40 x 40: 71 and 87), to 64 x 64; from there, where the
+//    fast form takes 512 threads a block, past two blocks a CU to 101 x 101 (the background alone, 75 x 83: 100 of
+//    them 15 and 14, 4 000 63 and 115).
+static bool prep_general(const PrepArg& a, int n) {
+    const long hw = (long)a.h * a.w;
+    if (a.clahe && a.tiles > 5 && a.tiles * a.tiles * a.bins >= 2048) return false;  // k_prep's lanes make these on a few banks
+    if (!a.dyn && !a.bp) {
+        if (hw > 4096) return hw <= 10240 && n > 512;
+        return a.clahe || hw <= 48 * 48 || hw % 4 != 0;
+    }
+    auto little = [&](const BlurArg& g) {
+        if (g.box) return hw <= (n > 512 ? 12 : 6) * (long)g.reach;
+        const long taps = (line_taps(g.radius, a.w) * a.h + line_taps(g.radius, a.h) * a.w) / 2;
+        return 5 * taps <= 9216 * (a.clahe || hw % 4 ? 7 : 5);
+    };
+    return (!a.dyn || little(a.dynb)) && (!a.bp || little(a.coarse)) && (!a.bp_fine || little(a.fine));
+}
+
+// The fast forms wherever they are the faster, what they keep in LDS fits (their tables differ from
+// k_prep's scratch, so it doesn't for a few images near the limit, nor for long thin ones) and pix_rc is
+// exact; `lds` becomes the bytes of dynamic LDS, `S` the image's row stride. forced: the caller asked for
+// global memory, which k_prep_box would not go through.
+static PrepForm prep_form(const PrepArg& a, int n, bool global, bool forced, int limit, size_t& lds, int& S) {
     const PrepForm loops = global ? kPrepLoopsG : kPrepLoops;
     const long hw = (long)a.h * a.w, room = (long)(limit - 1024) / 4;
-    if (hw > (1L << 22) || knob(KNOB_PREP_LOOPS) != 0) return loops;
+    if (hw > (1L << 22) || knob(KNOB_PREP_LOOPS) != 0 || (!global && prep_general(a, n))) return loops;
     if (!forced && a.dyn && a.dynb.box && !a.clahe && !a.bp && box_words(a.dynb, a.h, a.w) <= room) {
         lds = (size_t)box_words(a.dynb, a.h, a.w) * 4;
         return kPrepBoxes;
@@ -1464,7 +1496,7 @@ static int32_t prep_run(const char* who, const void* raw, int32_t pixel, int32_t
     hipStream_t s = (hipStream_t)stream;
     const float* bg = o->background;
     int S = w;
-    const PrepForm form = prep_form(a, global, forced, limit, lds, S);
+    const PrepForm form = prep_form(a, n, global, forced, limit, lds, S);
     if (pixel == 0)
         prep_launch<uint8_t>(raw, bg, a, n, form, lds, S, (float*)work, slot, grid, out, s);
     else if (pixel == 1)
