@@ -66,3 +66,36 @@ def test_the_host_refuses_records_out_of_turn(queue, one_look):
         assert np.array_equal(s._e.nmi_at(0, np.arange(256), want[0, :, :4]), nmi)
     finally:
         lib.zb_knob_set(b"refine_queue", 0)
+
+
+@pytest.mark.parametrize("h,w", [(8, 8), (14, 14), (16, 16), (24, 24), (30, 30), (32, 32)])
+def test_records_do_not_depend_on_the_waves_a_count_takes(h, w):
+    """Small frames take one wave a block for many items and one or two for few: the same records."""
+    print(f"refine waves {h}x{w}", flush=True)
+    n = 1030
+    c = _setup(h, w, n, 5)
+    many = _refine(c, n, iters=4)
+    assert np.all(many[:, 7] == 9.0)
+    for few in (1, 7, 1024):
+        assert np.array_equal(_refine(c, few, iters=4), many[:few]), few
+
+
+@pytest.mark.parametrize("n", [40, 1100])
+def test_the_persistent_grid_takes_one_wave_a_block_too(n):
+    from tests import cases
+    from tests.conftest import NI
+    from zebsdsolve_amd import Solver, _native as nat
+    print(f"refine queue of one wave, {n} cells", flush=True)
+    lib = nat.load()
+    s = Solver()
+    s.configure(bandwidth=16, refine_iters=3, static_background="none", dynamic_background="none")
+    s.set_geometry(pc=cases.PC, sample_tilt_deg=70.0)
+    s.add_phase(NI)
+    s.set_patterns(np.random.default_rng(3).integers(0, 250, (1, n, 16, 16), dtype=np.uint8))
+    want = s._e.index_cells(np.arange(n))
+    lib.zb_knob_set(b"refine_queue", 1)
+    try:
+        got = s._e.index_cells(np.arange(n))
+    finally:
+        lib.zb_knob_set(b"refine_queue", 0)
+    assert np.array_equal(got[..., :7], want[..., :7])

@@ -1,4 +1,4 @@
-// Orientation refinement on the detector, fused: one block of 2 to 16 waves (64 lanes each) per
+// Orientation refinement on the detector, fused: one block of 1 to 16 waves (64 lanes each) per
 // item runs the seed, every Gauss-Newton iteration, the normalized mutual information and the
 // record, in one launch (the reference's detector.wgsl seed, refine_init, sums_rot +
 // refine_rot_step per iteration, nmi and collect; src/detector.zig:178-212).
@@ -1034,11 +1034,13 @@ static void ref_opts(RefArg& a, const zb_refine_opts* o, int out0) {
 
 // The launch of a refinement: W waves a block, how its pixels are walked, and the LDS for the
 // joint histogram and the list. The list forms' records do not depend on W, so it follows the
-// speed (measured over frames of 40 x 40 to 180 x 180 and 3 to 16 000 items, 5 and 8 iterations):
-//  - while a block's lanes hold all their pixels, as few waves as hold them (2, 3 or 4): every
+// speed (measured over frames of 8 x 8 to 180 x 180, 5 and 8 iterations):
+//  - while a block's lanes hold all their pixels, as few waves as hold them (1 to 4): every
 //    wave adds hand-overs and barriers (40 x 40, 8 000 items: 582 us with 2 waves, 788 with 4;
 //    one wave an item, the list and the pattern read in each pass: 659), and holding beats reading
-//    the list again (60 x 60, 4 500 items: 514 us against 613);
+//    the list again (60 x 60, 4 500 items: 514 us against 613). One wave where it holds them: to 3 steps, and
+//    past 4 items a CU (20 000 items of 8 x 8: 339 us, 530 with 2 waves; of 16 x 16: 513 and 650; 3 000 of 24 x 24:
+//    162 and 175), where fewer leave the second wave room (30 items of 24 x 24: 55 us with one, 48 with 2);
 //  - above that, more waves where the items are too few to fill the chip or a frame's list leaves
 //    room for few blocks a CU: 8 up to one item a CU or past 256 steps (120 x 120, 8 items: 236 us
 //    against 256 with 4 and 417 with 2; 180 x 180, 1 000 items: 1 208, 1 337 and 2 505), else 4 past
@@ -1057,7 +1059,7 @@ static RefLaunch ref_launch(RefArg& a, int n_px, long total) {
         const int steps = (n_px + 63) / 64;
         if (steps <= 4 * kHeld) {
             l.mode = REF_HELD;
-            l.waves = std::max((steps + kHeld - 1) / kHeld, 2);
+            l.waves = steps <= 3 || (steps <= kHeld && total > 1024) ? 1 : std::max((steps + kHeld - 1) / kHeld, 2);
         } else {
             l.mode = REF_LIST;
             l.waves = total <= 256 || steps > 256 ? 8 : total <= 512 || steps > 96 ? 4 : 2;
@@ -1090,6 +1092,7 @@ static int queue_blocks(const RefLaunch& l) {
     const void* kern = nullptr;
 #define ZB_KERN(W, MODE) \
     if (l.waves == W && l.mode == MODE) kern = (const void*)k_refine_queue<W, MODE>
+    ZB_KERN(1, REF_HELD);
     ZB_KERN(3, REF_HELD);
     ZB_KERN(2, REF_HELD);
     ZB_KERN(2, REF_LIST);
@@ -1133,6 +1136,7 @@ static int32_t refine_launch(const zb_refine_phase* phases, int n_phases, const 
     if (l.waves == W && l.mode == MODE) ZB_LAUNCH("k_refine", (KERNEL<W, MODE>), dim3(GRID), dim3(64 * W), l.lds, st, a, ZB_PHASES, __VA_ARGS__)
 #define ZB_REFINE(KERNEL, GRID, ...)                         \
     do {                                                     \
+        ZB_REFINE1(KERNEL, GRID, 1, REF_HELD, __VA_ARGS__);  \
         ZB_REFINE1(KERNEL, GRID, 2, REF_HELD, __VA_ARGS__);  \
         ZB_REFINE1(KERNEL, GRID, 2, REF_LIST, __VA_ARGS__);  \
         ZB_REFINE1(KERNEL, GRID, 3, REF_HELD, __VA_ARGS__);  \
