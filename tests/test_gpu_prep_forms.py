@@ -116,7 +116,7 @@ def test_either_side_of_the_general_kernels_sizes(chain, n, monkeypatch):
     """The pixels do not depend on the kernel that the size, the taps and the count choose: sizes about each line."""
     monkeypatch.setitem(CHAINS, "none", {})
     monkeypatch.setitem(CHAINS, "one tap", dict(dynamic=1, dynamic_sigma=0.5))
-    sizes = {"none": [(48, 48), (48, 49), (49, 49), (64, 64), (64, 65), (100, 102), (101, 102)], "clahe": [(64, 64), (64, 65), (101, 101), (102, 102)],
+    sizes = {"none": [(48, 48), (48, 49), (49, 49), (64, 64), (64, 65), (100, 102), (101, 102), (230, 200)], "clahe": [(64, 64), (64, 65), (101, 101), (102, 102)],
              "one tap": [(42, 42), (43, 43), (44, 44)], "boxes": [(18, 18), (19, 19), (26, 26), (27, 27)]}[chain]
     for h, w in sizes:
         print(f"prep lines {chain} {h}x{w} n {n}", flush=True)

@@ -1375,9 +1375,12 @@ static long line_taps(int radius, int n) {
 //  - the background alone to 48 x 48 (4 000 of 32 x 32: 16 and 22; 60 x 60: 41 and 37), and CLAHE whose tables are
 //    soon made, up to 5 x 5 tiles or 2 047 levels in all (40 x 40: 71 and 87), to 64 x 64; from there, where the
 //    fast form takes 512 threads a block, past two blocks a CU to 101 x 101 (the background alone, 75 x 83: 100 of
-//    them 15 and 14, 4 000 63 and 115).
-static bool prep_general(const PrepArg& a, int n) {
+//    them 15 and 14, 4 000 63 and 115);
+//  - frames past LDS with the background alone past two blocks a CU (241 x 321: 512 of them 464 and 456, 800
+//    628 and 885).
+static bool prep_general(const PrepArg& a, int n, bool global) {
     const long hw = (long)a.h * a.w;
+    if (global) return !a.dyn && !a.bp && !a.clahe && n > 512;
     if (a.clahe && a.tiles > 5 && a.tiles * a.tiles * a.bins >= 2048) return false;  // k_prep's lanes make these on a few banks
     if (!a.dyn && !a.bp) {
         if (hw > 4096) return hw <= 10240 && n > 512;
@@ -1398,7 +1401,7 @@ static bool prep_general(const PrepArg& a, int n) {
 static PrepForm prep_form(const PrepArg& a, int n, bool global, bool forced, int limit, size_t& lds, int& S) {
     const PrepForm loops = global ? kPrepLoopsG : kPrepLoops;
     const long hw = (long)a.h * a.w, room = (long)(limit - 1024) / 4;
-    if (hw > (1L << 22) || knob(KNOB_PREP_LOOPS) != 0 || (!global && prep_general(a, n))) return loops;
+    if (hw > (1L << 22) || knob(KNOB_PREP_LOOPS) != 0 || prep_general(a, n, global)) return loops;
     if (!forced && a.dyn && a.dynb.box && !a.clahe && !a.bp && box_words(a.dynb, a.h, a.w) <= room) {
         lds = (size_t)box_words(a.dynb, a.h, a.w) * 4;
         return kPrepBoxes;
