@@ -372,7 +372,8 @@ int32_t zb_prep(const void* raw, int32_t pixel, int32_t n, int32_t h, int32_t w,
 
 /* Bytes of workspace zb_prep_work needs for n patterns h x w with these filters: 0 where one
  * block's LDS holds the image and its scratch (zb_prep's case), else a slot of image and
- * scratch for each of up to 1 024 blocks. */
+ * scratch for each of up to 1 024 blocks (asked for whichever kernel takes the call: a background by
+ * boxes alone may need none of it). */
 int64_t zb_prep_workspace(int32_t n, int32_t h, int32_t w, const zb_prep_opts* opts);
 
 /* zb_prep for patterns of any size (the reference's 240 x 320 frames with its default filters):
@@ -435,15 +436,15 @@ int32_t zb_profile_report(char* buf, int32_t cap);
  * other launches run as they do unprofiled. No counterpart in the reference. */
 int32_t zb_profile_select(const char* names);
 
-/* Launch-shape knobs, process-wide, read at each launch; none changes any result bit, only how
- * the work is cut into blocks (the choices the host's tuner makes by timing). zb_knob_set
+/* Knobs, process-wide, read at each launch; none changes any result bit (refine_polls at its default),
+ * only how the work is cut into blocks and which kernel takes it. zb_knob_set
  * returns the previous value (ZB_EINVAL for an unknown name or a value out of range),
  * zb_knob_get the current one.
  *   "refine_queue" 0..2 (0): zb_refine_phases as one block per work item (0) or as a persistent
  *                            grid draining device-side queues (1; 2: the same)
  *   "rings_group"  0..64 (0): ring pairs per block of the sphere stage's ring transforms, a power
  *                            of two (0: 16, 4 and 4 for rings of 128, 256 and 512 points, else 16 KB of
- *                            LDS worth; at most n / 2 and 64 KB)
+ *                            LDS worth; at most n / 2 and 8 192 points, up to 67 KB of LDS)
  *   "prep_global"  0..1 (0): zb_prep_work's filters through global memory even where LDS holds
  *                            the image (1)
  *   "prep_loops"   0..1 (0): zb_prep and zb_prep_work by the kernels that take every call (1), also

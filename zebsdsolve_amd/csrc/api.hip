@@ -84,7 +84,7 @@ struct Knob {
 };
 static Knob g_knobs[] = {
     {"refine_queue", 0, 2, 0, {0}},  // zb_refine_phases: 0 a block per work item, 1 the persistent queue grid (2: the same)
-    {"rings_group", 0, 64, 0, {0}},  // ring pairs per k_rings block (0: 2048 / (2n), at most n / 2)
+    {"rings_group", 0, 64, 0, {0}},  // ring pairs per k_rings block (0: 16, 4, 4 for 128, 256, 512 points, else 2048 / (2n); at most n / 2)
     {"prep_global", 0, 1, 0, {0}},   // zb_prep_work: 1 the filters through global memory even where LDS holds the image
     {"refine_polls", 1, 1 << 22, 1 << 22, {1 << 22}},  // k_refine: polls of a wave's wait for its turn before its record goes unstamped
     {"prep_loops", 0, 1, 0, {0}},    // zb_prep, zb_prep_work: 1 the kernels that take every call, also where a faster form holds

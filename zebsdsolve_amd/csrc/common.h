@@ -403,11 +403,12 @@ __device__ void fft_dif(float2* buf, int log2n, int nlines, int lstride, int pst
 // cycles of a kernel that LDS bound). So point p sits at fft_at(p) = p + p / 2^shift, a line takes
 // fft_line<LOG2N> = 2^LOG2N + F points, F = 2^(LOG2N - shift), and neighbouring threads take
 // neighbouring lines and then F butterflies of one, neighbours or (where q < F) a part of the line
-// apart: with 32 / F lines 32 threads meet every bank once. With p's digits disjoint fft_at adds
-// up, so the four points of a butterfly stay a constant apart.
+// apart: with 32 / F lines the addresses of 32 threads fall on every bank once. With p's digits disjoint
+// fft_at adds up, so the four points of a butterfly stay a constant apart.
 // (The ring transforms at L = 64, 3 001 items, 8 lines a block: conflicts 44 of 67 M LDS cycles, k_rings
-// 186 us; 18 of 41 and 145 padded by one in 64, the vector units busy for 115 of them. Then 4 lines and
-// one in 32: a batch of 4 500 at 60 x 60 1 960 -> 1 944 us.)
+// 186 us; padded by one in 64 18 of 41 and 145, the vector units busy for 115 of them; 4 lines and one in
+// 32, as here, 17 of 38 and 134: the counter still has 45 % of the LDS cycles as conflicts, of accesses that
+// this count of banks does not show. A batch of 4 500 at 60 x 60 1 960 -> 1 944 us with the last.)
 constexpr int fft_shift(int log2n) { return log2n == 8 ? 5 : 6; }
 template <int LOG2N>
 __host__ __device__ constexpr int fft_at(int p) {
@@ -415,7 +416,7 @@ __host__ __device__ constexpr int fft_at(int p) {
 }
 template <int LOG2N>
 constexpr int fft_line = fft_at<LOG2N>(1 << LOG2N);
-// the lines for which a wave meets every bank once: 16, 4 and 4 of 128, 256 and 512 points
+// the lines for which 32 threads' addresses fall on every bank once: 16, 4 and 4 of 128, 256 and 512 points
 constexpr int fft_lines(int log2n) { return 32 >> (log2n - fft_shift(log2n)); }
 
 // The butterfly (of 2^BITS of a line) that index rr takes in a stage of step 2^LQ.

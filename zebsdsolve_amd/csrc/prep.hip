@@ -538,11 +538,12 @@ __global__ void __launch_bounds__(256) k_prep_g(const T* __restrict__ raw, const
 
 // ── the same chain, every sum in the same order, for what the fast forms take ──
 //
-// What bounded k_prep and k_prep_g (which stay for what these do not take): every tap of the direct
+// What bounded k_prep and k_prep_g (which stay for what these do not take, and where they are the
+// faster, prep_general): every tap of the direct
 // blur was two LDS reads and some eight instructions, the box path computed an exponential a tap and
 // pixel, an image in global memory had one wave a SIMD, and a tile's CLAHE table was read by lanes a
 // power of two apart. A pixel's last bit moves it from one NMI or CLAHE bin to the next, and records
-// with it, so every pixel here is the old kernels' bit for bit:
+// with it, so every pixel here is those kernels' bit for bit (the knob prep_loops chooses them everywhere):
 // - the direct Gaussian is two products on the matrix cores, X Gx and Gy (X Gx), G the banded matrix
 //   of the taps. v_mfma_f32_32x32x2_f32 is fma(a1, b1, fma(a0, b0, c)) to the bit (checked against the
 //   VALU), so tap 2 s in the lower and 2 s + 1 in the upper lanes gives the serial sum's rounding; a

@@ -1038,16 +1038,16 @@ static void ref_opts(RefArg& a, const zb_refine_opts* o, int out0) {
 //  - while a block's lanes hold all their pixels, as few waves as hold them (1 to 4): every
 //    wave adds hand-overs and barriers (40 x 40, 8 000 items: 582 us with 2 waves, 788 with 4;
 //    one wave an item, the list and the pattern read in each pass: 659), and holding beats reading
-//    the list again (60 x 60, 4 500 items: 514 us against 613). One wave where it holds them: to 3 steps, and
+//    the list again (60 x 60, 4 500 items: 513 us against 613). One wave where it holds them: to 3 steps, and
 //    past 4 items a CU (20 000 items of 8 x 8: 339 us, 530 with 2 waves; of 16 x 16: 513 and 650; 3 000 of 24 x 24:
 //    162 and 175), where fewer leave the second wave room (30 items of 24 x 24: 55 us with one, 48 with 2);
 //  - above that, more waves where the items are too few to fill the chip or a frame's list leaves
-//    room for few blocks a CU: 8 up to one item a CU or past 256 steps (120 x 120, 8 items: 236 us
+//    room for few blocks a CU: 8 up to one item a CU or past 256 steps (120 x 120, 8 items: 235 us
 //    against 256 with 4 and 417 with 2; 180 x 180, 1 000 items: 1 208, 1 337 and 2 505), else 4 past
 //    96 steps or up to two items a CU (120 x 120, 1 200 items: 798 us against 848 with 2 and 813
 //    with 8; 80 x 80, 400 items: 238, 294 and 244), else 2 (80 x 80, 4 000 items: 1 233, 1 308 with
 //    4, 1 392 with 8).
-// One wave an item took 725 us for 8 items of 120 x 120, 3 681 us for 40 of 240 x 240 (tiles: 567).
+// (60 x 60 was measured at 4 500 and 16 000 items; what a few items of it gain from more waves was not.)
 struct RefLaunch {
     int mode, waves;
     size_t lds;

@@ -190,8 +190,8 @@ __global__ void __launch_bounds__(256) k_rings(SphArg a, int G, const float* __r
     const int nphi = 1 << a.log2nphi;
     const int lg = __builtin_ctz((unsigned)G);  // G is a power of two
     const int n_items = gridDim.x / groups;
-    // nothing of these rings in the window: 2 groups in 8 at L = 64, the detector tilted 70 degrees and
-    // half a frame from its centre to its edge at the distance 0.55
+    // nothing of these rings in the window: 5 groups in 16 at L = 64, 60 x 80 pixels, the detector tilted 70
+    // degrees at the distance 0.55
     const int2 on = live_range(live, b);
     if (y0 >= on.y || y0 + G <= on.x) return;
     // a line's points in LDS: padded for the lengths known here (fft_at)
@@ -593,7 +593,7 @@ static int32_t sh_run(const zb_band* band, const zb_frame* frame, const float* p
     // ring pairs a block transforms: the knob's (a power of two), else what meets every LDS bank once
     // (fft_lines; k_rings over 100 000 patterns: L = 64, 8, 4 and 2 pairs 6.3, 4.1 and 5.8 ms; L = 96, 8, 4 and 2: 25.6,
     // 16.6 and 20.4; L = 32, 16, 8 and 4: 1.39, 1.41 and 1.79), 16 KB of LDS worth past these lengths; at most
-    // n / 2 and 64 KB of LDS
+    // n / 2 and 8 192 points (with the padding and the rings' entries 68 096 bytes at the most)
     const bool padded = a.log2nphi >= 7 && a.log2nphi <= 9;
     int G = knob(KNOB_RINGS_GROUP) > 0 ? knob(KNOB_RINGS_GROUP) : padded ? fft_lines(a.log2nphi) : 2048 / nphi;
     while (G & (G - 1)) G &= G - 1;
